@@ -27,20 +27,17 @@
 // k), and a 7-slot sliding window turns plane sums into outputs.
 //
 // CG (Eigen's algorithm, identity preconditioner, recursive residual):
-//   init      r = b - M x0, p = r, b.b, r.r     (stencil launch + 1-block
-//                                                finish)
-//   iterate   SpMV(k):   rr_{k-1} -> converged? beta; p = r + beta p_old
-//                        (fused into the halo load, p double-buffered);
-//                        t = M p; partial p.t per block
-//             update(k): alpha = rr_{k-1} / p.t; x += alpha p;
-//                        r -= alpha t; partial r.r per block
-// 3D: one launch per iteration (k_cg_iter3, persistent blocks) forms the
-// sums of the previous launch's partials, applies the update and the SpMV.
+//   init      r = b - M x0, b.b, r.r       (stencil launch + 1-block finish)
+//   iterate   one launch per iteration (k_cg_iter3, 2D: k_cg_iter2), which
+//             forms the sums of the previous launch's partials, applies the
+//             update (x += alpha p, r -= alpha t), the new direction
+//             p = r + beta p over the halo and t = M p, and leaves the
+//             partials of p.t, r.t, t.t and r.r
 // Every grid-wide sum is formed by the CONSUMING kernel: its blocks re-sum
-// the producer's per-block partials in a fixed order (2D: a ring of three
-// iterations; 3D: two alternating sets).  No device-scope fence or atomic is issued inside the loop --
-// on a multi-XCD part an agent-scope release writes back the L2 -- and the
-// result is bitwise reproducible.  FP32 vectors, FP64 dots and norms.  At
+// the producer's per-block partials in a fixed order (two alternating sets).
+// No device-scope fence or atomic is issued inside the loop -- on a multi-XCD
+// part an agent-scope release writes back the L2 -- and the result is
+// bitwise reproducible.  FP32 vectors, FP64 dots and norms.  At
 // convergence the FP64 true residual ||b - M x|| is checked; if it is above
 // the tolerance CG restarts from the true residual (residual replacement).
 #include <cfloat>
@@ -62,20 +59,13 @@ struct CoefD {
 
 namespace {
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-// Streaming (nontemporal) 16-byte store.
-__device__ __forceinline__ void store_nt4(float* p, float a, float b, float c,
-                                          float d) {
-    f32x4_t v = {a, b, c, d};
-    __builtin_nontemporal_store(v, (f32x4_t*)p);
-}
 
 constexpr int kT = 14;             // halo tile side (8 + 2 * 3)
 constexpr int kT2 = kT * kT;
 constexpr int kHaloIters2 = (kT2 + 63) / 64;   // 4
-constexpr int kUpdBlocks = 256;                // grid of the CG update
+constexpr int kUpdBlocks = 256;                // grid of the vector passes
 constexpr int kUpdThreads = 1024;
-constexpr int kIterBlocks = 1024;                // persistent blocks of the 3D iteration
+constexpr int kIterBlocks = 1024;              // most blocks of an iteration launch
 
 // 2D tile element e -> (neighbour brick 0..8) << 9 | local node; elements
 // past the tile map to the zero brick slot 9.  (3D decodes arithmetically.)
@@ -101,11 +91,9 @@ __constant__ HaloTab2 kHalo2 = make_halo2();
 enum Kind {
     K_DIAG = 0,        // s = -sum cc V_J; diag = max(s, alpha0)   (double)
     K_APPLY = 1,       // out = M in                                 (float)
-    K_CG_INIT = 2,     // r = b - M x0; p = r; partial b.b, r.r     (float)
-    K_SPMV_FIRST = 3,  // t = M p; partial p.t                       (float)
-    K_SPMV_FUSED = 4,  // p = r + beta p_old; t = M p; partial p.t   (float)
-    K_TRUE_RES = 5     // rt = b - M x (double); partial rt.rt      (double)
-    // (the 3D CG iteration is k_cg_iter3)
+    K_CG_INIT = 2,     // r = b - M x0; partial b.b, r.r             (float)
+    K_TRUE_RES = 3     // rt = b - M x (double); partial rt.rt      (double)
+    // (the CG iteration is k_cg_iter3, in 2D k_cg_iter2)
 };
 
 struct StencilArgs {
@@ -119,39 +107,26 @@ struct StencilArgs {
     const float* vdiag;
     const double* vdiag64;
     const float* vb;
-    const float* in;       // p / x / x0 / in (p_old when fused)
+    const float* in;       // x / x0 / in (p_old: CG iteration)
     const double* in_base; // K_TRUE_RES: FP64 base of x (x = in_base + in)
-    const float* in2;      // r for the fused update (r_old: 3D iteration)
-    const float* in3;      // t_old (3D iteration)
+    const float* in2;      // r_old (CG iteration)
+    const float* in3;      // t_old (CG iteration)
     float* out;            // t / r / out
-    float* out2;           // p_new (fused) or p (init)
-    float* out3;           // r_new (3D iteration)
-    float* xio;            // x, updated in place (3D iteration)
+    float* out2;           // p_new (CG iteration)
+    float* out3;           // r_new (CG iteration)
+    float* xio;            // x, updated in place (CG iteration)
     double* out_d;         // diag64
     float* out_f;          // diag32
     float* out_s;          // unclamped row sum s (feature of the learned start)
     double alpha0;
     CgState* st;
-    double* part0;         // this kernel's per-block partials (sum 0)
-    double* part1;         // per-block partials (sum 1: init, FIRST, UPD)
-    double* part2;         // per-block partials (sum 2: FIRST, UPD)
-    double* part3;         // per-block partials (sum 3: FIRST, UPD)
-    const double* rr1;     // update partials of iteration kk-1
-    const double* rr2;     // update partials of iteration kk-2
+    double* part0;         // per-block partials (sum 0)
+    double* part1;         // per-block partials (sum 1: init)
     int kk;                // iteration index since the (re)start
     int iter_base;         // Eigen iteration count at the (re)start
     int64_t max_iter;
     int spec;              // K_TRUE_RES: run only if the solve has converged
 };
-
-// Sum of n per-block partials, identical in every block and lane: lane l
-// adds partials l, l + 64, ... in order, then a fixed DPP tree.
-__device__ __forceinline__ double sum_partials64(const double* p, int n) {
-    const int lane = threadIdx.x & 63;
-    double s = 0;
-    for (int i = lane; i < n; i += 64) s += p[i];
-    return wave_sum_all(s);
-}
 
 template <int BS>
 __device__ __forceinline__ double block_sum(double v, double* sbuf) {
@@ -197,6 +172,21 @@ __device__ __forceinline__ void plane4(const T* pl, const C& cc, T P[4]) {
     P[3] = c9 * U0 + c10 * U1 + c11 * U2 + c13 * U4 + c14 * U5;
 }
 
+// 2D iteration: the in-plane sum P_0 alone, points grouped as in plane4.
+template <int RS>
+__device__ __forceinline__ float plane0(const float* pl, const CoefF& cc) {
+    auto at = [&](int a, int b) { return pl[a + b * RS]; };
+    auto axis4 = [&](int a) { return (at(a, 0) + at(-a, 0)) + (at(0, a) + at(0, -a)); };
+    auto diag4 = [&](int a) { return (at(a, a) + at(-a, a)) + (at(a, -a) + at(-a, -a)); };
+    auto ring8 = [&](int a, int b) {
+        return ((at(a, b) + at(-a, b)) + (at(a, -b) + at(-a, -b))) +
+               ((at(b, a) + at(-b, a)) + (at(b, -a) + at(-b, -a)));
+    };
+    return cc.c[1] * axis4(1) + cc.c[2] * diag4(1) + cc.c[4] * axis4(2) + cc.c[5] * ring8(1, 2) +
+           cc.c[8] * diag4(2) + cc.c[9] * axis4(3) + cc.c[10] * ring8(1, 3) +
+           cc.c[13] * ring8(2, 3);
+}
+
 // 2D: in-plane sum only.
 template <typename T, typename C>
 __device__ __forceinline__ T plane1(const T* pl, const C& cc) {
@@ -219,43 +209,14 @@ __device__ __forceinline__ T plane1(const T* pl, const C& cc) {
     return P;
 }
 
-// Prologue of the CG SpMV: convergence test of iteration kk-1, beta.
-// Returns false when the solve is over (block 0 records why).
-__device__ __forceinline__ bool spmv_prologue(const StencilArgs& a,
-                                              float* beta) {
-    CgState* st = a.st;
-    if (st->done) return false;
-    *beta = 0.f;
-    if (a.kk == 0) return true;
-    const double r1 = sum_partials64(a.rr1, kUpdBlocks);
-    const double r2 = a.kk >= 2 ? sum_partials64(a.rr2, kUpdBlocks) : st->abs0;
-    const int k = a.iter_base + a.kk;
-    int done = 0;
-    if (!isfinite(r1)) done = 3;
-    else if (r1 < st->thr) done = 1;
-    else if (k >= a.max_iter) done = 2;
-    if (done) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            st->rr = r1;
-            st->iter = done == 1 ? k - 1 : k;
-            st->done = done;
-        }
-        return false;
-    }
-    *beta = (float)(r1 / r2);
-    return true;
-}
-
 template <int KIND, int OP, typename T>
 __device__ __forceinline__ T load_input(const StencilArgs& a, uint32_t g,
-                                        float beta, float* pnew_out) {
+                                        float* own_out) {
     if constexpr (KIND == K_DIAG) {
         return (T)a.vvol[g];
     } else {
-        float p;
-        if constexpr (KIND == K_SPMV_FUSED) p = a.in2[g] + beta * a.in[g];
-        else p = a.in[g];
-        *pnew_out = p;
+        const float p = a.in[g];
+        *own_out = p;
         if constexpr (OP == VPS_OP_ROW) return (T)a.vvol[g] * (T)p;
         else return (T)p;
     }
@@ -284,23 +245,20 @@ constexpr int kOwnX = 11 * 64;                  // own nodes of tile planes 3..1
 template <int KIND, int OP, typename T, typename C>
 __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
     __shared__ T tile[kT * kPS];
-    // plane sums P_k of plane zp, column l; reused for the first SpMV's
-    // block partials after the outputs (8-byte aligned for that)
-    __shared__ __align__(16) T psum[kT][4][64];
-    __shared__ float own[512];      // raw own-brick input (p / x)
+    __shared__ T psum[kT][4][64];   // plane sums P_k of plane zp, column l
+    __shared__ float own[512];      // raw own-brick input (x)
     // K_TRUE_RES: the own brick's x = base + correction in FP64
     __shared__ double own64[KIND == K_TRUE_RES ? 512 : 1];
     __shared__ uint32_t sbase[27];
-    __shared__ double sred[4][4];
+    __shared__ double sred[2][4];
     __shared__ int s_done;
     const int slot = xcd_remap(blockIdx.x, (int)a.nslots);
     const int t = threadIdx.x;
     const int l = t & 63, wv = t >> 6;
     if (t < 27) sbase[t] = (uint32_t)a.nbr_slot[(int64_t)slot * 27 + t] * 512u;
-    if constexpr (KIND == K_SPMV_FIRST || KIND == K_SPMV_FUSED || KIND == K_TRUE_RES) {
-        // a solve that has ended skips the halo loads (launches past the
-        // convergence of a batch); a speculative true-residual check runs
-        // only once the recursive residual has converged
+    // a speculative true-residual check runs only once the recursive
+    // residual has converged
+    if constexpr (KIND == K_TRUE_RES) {
         if (t == 32) s_done = a.st->done;
     }
     const int x = l & 7, y = l >> 3;
@@ -315,22 +273,18 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
         Bz[q] = (KIND == K_CG_INIT || KIND == K_TRUE_RES) ? a.vb[g] : 0.f;
     }
     __syncthreads();
-    if constexpr (KIND == K_SPMV_FIRST || KIND == K_SPMV_FUSED) {
-        if (s_done) return;   // uniform over the block
-    }
     if constexpr (KIND == K_TRUE_RES) {
         if (a.spec && s_done != 1) return;   // uniform over the block
     }
     // Halo load: unit u = (line (yt, zt), part k): k = 0 the upper half row of
     // the left brick (x = -4..-1), 1 and 2 the center row, 3 the lower half
-    // row of the right brick (x = 8..11).  The raw loads do not depend on
-    // beta, so they are issued before the prologue's reductions.
-    float4 ra[kUnitIters], rb[kUnitIters], rv[kUnitIters];
+    // row of the right brick (x = 8..11).
+    float4 ra[kUnitIters], rv[kUnitIters];
     double4 rx[KIND == K_TRUE_RES ? kUnitIters : 1];
 #pragma unroll
     for (int i = 0; i < kUnitIters; i++) {
         const int u = t + kS3Threads * i;
-        ra[i] = rb[i] = rv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        ra[i] = rv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if constexpr (KIND == K_TRUE_RES) rx[i] = make_double4(0.0, 0.0, 0.0, 0.0);
         // units of the first kUnitIters - 1 rounds always exist (t < 256)
         if (i < kUnitIters - 1 || u < kUnits) {
@@ -345,15 +299,10 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
                 rv[i] = *(const float4*)(a.vvol + g);
             } else {
                 ra[i] = *(const float4*)(a.in + g);
-                if constexpr (KIND == K_SPMV_FUSED) rb[i] = *(const float4*)(a.in2 + g);
                 if constexpr (KIND == K_TRUE_RES) rx[i] = *(const double4*)(a.in_base + g);
                 if constexpr (OP == VPS_OP_ROW) rv[i] = *(const float4*)(a.vvol + g);
             }
         }
-    }
-    float beta = 0.f;
-    if constexpr (KIND == K_SPMV_FIRST || KIND == K_SPMV_FUSED) {
-        if (!spmv_prologue(a, &beta)) return;   // uniform over the grid
     }
 #pragma unroll
     for (int i = 0; i < kUnitIters; i++) {
@@ -367,10 +316,7 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
                 v[0] = (T)rv[i].x; v[1] = (T)rv[i].y; v[2] = (T)rv[i].z; v[3] = (T)rv[i].w;
                 pn[0] = pn[1] = pn[2] = pn[3] = 0.f;
             } else {
-                float4 p = ra[i];
-                if constexpr (KIND == K_SPMV_FUSED)
-                    p = make_float4(rb[i].x + beta * ra[i].x, rb[i].y + beta * ra[i].y,
-                                    rb[i].z + beta * ra[i].z, rb[i].w + beta * ra[i].w);
+                const float4 p = ra[i];
                 pn[0] = p.x; pn[1] = p.y; pn[2] = p.z; pn[3] = p.w;
                 T xv[4] = {(T)p.x, (T)p.y, (T)p.z, (T)p.w};
                 if constexpr (KIND == K_TRUE_RES) {
@@ -398,8 +344,6 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
                     const int loc = 4 * (k - 1) + 8 * ((yt - 3) + 8 * (zt - 3));
 #pragma unroll
                     for (int c = 0; c < 4; c++) own[loc + c] = pn[c];
-                    if constexpr (KIND == K_SPMV_FUSED)
-                        store_nt4(a.out2 + base + loc, pn[0], pn[1], pn[2], pn[3]);
                 }
             }
         }
@@ -413,7 +357,7 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
         for (int q = 0; q < 4; q++) psum[zp][q][l] = P[q];
     }
     __syncthreads();
-    double red0 = 0, red1 = 0, red2 = 0, red3 = 0;
+    double red0 = 0, red1 = 0;
 #pragma unroll
     for (int q = 0; q < 2; q++) {
         const int z = 2 * wv + q;
@@ -452,61 +396,23 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
                 const float b = Bg;
                 const float r = on ? b - mp : 0.f;
                 a.out[g] = r;
-                a.out2[g] = r;
                 red0 += (double)b * (double)b;
                 red1 += (double)r * (double)r;
-            } else {
-                // t = M p is read by the next kernel only: streaming store
-                __builtin_nontemporal_store(mp, &a.out[g]);
-                red0 += (double)pi * (double)mp;
-                if constexpr (KIND == K_SPMV_FIRST) red3 += (double)pi * (double)pi;
-                if constexpr (KIND == K_SPMV_FIRST)
-                    red2 += (double)mp * (double)mp;
             }
         }
     }
-    if constexpr (KIND == K_SPMV_FIRST) {
-        // four block sums (p.t, r.t, t.t, r.r; r = p after SPMV_FIRST): the
-        // lanes' values through LDS, then wave w reduces sum w -- one DPP
-        // tree per wave instead of four
-        static_assert(sizeof(psum) >= 4 * kS3Threads * sizeof(double), "partials fit psum");
-        __syncthreads();   // every wave has read its plane sums
-        double* sp = reinterpret_cast<double*>(&psum[0][0][0]);
-        sp[t] = red0;
-        sp[kS3Threads + t] = KIND == K_SPMV_FIRST ? red0 : red1;
-        sp[2 * kS3Threads + t] = red2;
-        sp[3 * kS3Threads + t] = red3;
-        __syncthreads();
-        const double* q = sp + kS3Threads * wv;
-        double v = (q[l] + q[l + 64]) + (q[l + 128] + q[l + 192]);
-        v = wave_sum_all(v);
-        double* dst = wv == 0 ? a.part0 : (wv == 1 ? a.part1 : (wv == 2 ? a.part2 : a.part3));
-        if (l == 0 && dst) dst[blockIdx.x] = v;
-    } else if constexpr (KIND != K_DIAG && KIND != K_APPLY) {
-        constexpr bool three = false;
+    if constexpr (KIND == K_CG_INIT || KIND == K_TRUE_RES) {
         red0 = wave_sum_all(red0);
         if (KIND == K_CG_INIT) red1 = wave_sum_all(red1);
-        if (three) {
-            red2 = wave_sum_all(red2);
-            red3 = wave_sum_all(red3);
-        }
         if (l == 0) {
             sred[0][wv] = red0;
             sred[1][wv] = red1;
-            sred[2][wv] = red2;
-            sred[3][wv] = red3;
         }
         __syncthreads();
         if (t == 0) {
-            const double s0 = (sred[0][0] + sred[0][1]) + (sred[0][2] + sred[0][3]);
-            a.part0[blockIdx.x] = s0;
+            a.part0[blockIdx.x] = (sred[0][0] + sred[0][1]) + (sred[0][2] + sred[0][3]);
             if (KIND == K_CG_INIT)
                 a.part1[blockIdx.x] = (sred[1][0] + sred[1][1]) + (sred[1][2] + sred[1][3]);
-            if (three && a.part2) {
-                if (KIND == K_SPMV_FIRST) a.part1[blockIdx.x] = s0;
-                a.part2[blockIdx.x] = (sred[2][0] + sred[2][1]) + (sred[2][2] + sred[2][3]);
-                a.part3[blockIdx.x] = (sred[3][0] + sred[3][1]) + (sred[3][2] + sred[3][3]);
-            }
         }
     }
 }
@@ -528,34 +434,141 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
 // 11..13, stored by it) stay in LDS, and only planes 6..13 are loaded and
 // summed.  The launch that ends the solve
 // applies only the last x update; block 0 records the state.
-static_assert(kIterBlocks <= 4 * kS3Threads, "one round of partial loads per thread");
 struct IterArgs {
     const double* prev[4];   // the previous launch's partials (p.t, r.t, t.t, r.r)
     double* out[4];          // this launch's partials, one per block
     int nprev;               // their count
-    int resume;              // alpha, beta from the state (after a replacement)
+    int resume;              // alpha, beta from the state (a start, after a replacement)
 };
 
-// Block sums of four per-thread values v[0..3] in a fixed order: the 4 x 256
-// values go through LDS scratch (8 KB), wave w adds the four values of lane
-// l, l + 64, l + 128, l + 192 of sum w and reduces them with one DPP tree;
+// Block sums of four per-thread values v[0..3] in a fixed order: the 4 x NT
+// values go through LDS scratch (32 NT bytes), wave w < 4 adds the values of
+// lanes l, l + 64, ... of sum w pairwise and reduces them with one DPP tree;
 // out[w] (LDS) holds sum w for the whole block afterwards.
+template <int NT>
 __device__ __forceinline__ void block_sums4(const double v[4], double* scratch, double* out) {
     const int t = threadIdx.x, l = t & 63, wv = t >> 6;
 #pragma unroll
-    for (int q = 0; q < 4; q++) scratch[q * kS3Threads + t] = v[q];
+    for (int q = 0; q < 4; q++) scratch[q * NT + t] = v[q];
     __syncthreads();
-    const double* a = scratch + kS3Threads * wv;
-    double s = (a[l] + a[l + 64]) + (a[l + 128] + a[l + 192]);
-    s = wave_sum_all(s);
-    if (l == 0) out[wv] = s;
+    if (wv < 4) {
+        const double* a = scratch + NT * wv;
+        double s = 0;
+#pragma unroll
+        for (int h = 0; h < NT; h += 256)
+            s += (a[l + h] + a[l + 64 + h]) + (a[l + 128 + h] + a[l + 192 + h]);
+        s = wave_sum_all(s);
+        if (l == 0) out[wv] = s;
+    }
     __syncthreads();
 }
 
-template <int OP>
-__global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc, IterArgs it,
+// What a block of an iteration launch needs of the previous one.  Every lane
+// loads (indices past the partials read the last one): loads under a
+// condition make the compiler's waits for them cover every later load.
+template <int NT>
+struct IterHead {
+    static constexpr int U = (kIterBlocks + NT - 1) / NT;
+    double v[4][U];
+    double thr_rec;
+    float alpha, beta;
+    int stop;
+    __device__ __forceinline__ void load(const StencilArgs& a, const IterArgs& it) {
+        // the state was written by earlier launches only: plain loads
+        const CgState* st = a.st;
+        stop = st->stop;
+        thr_rec = st->thr_rec;
+        alpha = st->alpha;
+        beta = st->beta;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int i = min((int)threadIdx.x + NT * u, it.nprev - 1);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[q][u] = it.prev[q][i];
+        }
+    }
+};
+
+// alpha_(kk-1) and beta_kk of an iteration launch into s_ab, and s_mode: 0 go
+// on, 1 the solve ended (apply the last x update only), 2 non-finite alpha
+// (no update).  Block 0 records the state.  The caller synchronises.
+template <int NT>
+__device__ __forceinline__ void iter_scalars(const StencilArgs& a, const IterArgs& it,
+                                             const IterHead<NT>& hd, double* scratch,
+                                             double* sred, float* s_ab, int* s_mode) {
+    const int t = threadIdx.x, kk = a.kk;
+    if (it.resume) {
+        if (t == 0) {
+            *s_mode = 0;
+            s_ab[0] = hd.alpha;
+            s_ab[1] = hd.beta;
+        }
+        return;
+    }
+    double sv[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        sv[q] = 0;
+#pragma unroll
+        for (int u = 0; u < IterHead<NT>::U; u += 2) {
+            const double w0 = t + NT * u < it.nprev ? hd.v[q][u] : 0.0;
+            const double w1 = u + 1 < IterHead<NT>::U && t + NT * (u + 1) < it.nprev
+                                  ? hd.v[q][u + 1 < IterHead<NT>::U ? u + 1 : u] : 0.0;
+            sv[q] += w0 + w1;
+        }
+    }
+    // the four sums through LDS: wave w reduces sum w with one DPP tree
+    // instead of every wave reducing all four
+    block_sums4<NT>(sv, scratch, sred);
+    if (t == 0) {
+        CgState* st = a.st;
+        const double pt = sred[0], rt = sred[1], tt = sred[2], rr = sred[3];
+        const int k = a.iter_base + kk - 1;   // Eigen's index of the reduced SpMV
+        const double ald = rr / pt;
+        const float al = (float)ald;
+        const double a64 = (double)al;   // the alpha the vectors are updated with
+        const double rn = (rr - 2.0 * a64 * rt) + a64 * a64 * tt;
+        int done = 0, iter = 0;
+        float be = 0.f;
+        if (!isfinite(ald) || !isfinite(rn)) {
+            done = 3;
+            iter = k;
+        } else if (rn < hd.thr_rec) {
+            done = 1;
+            iter = k;
+        } else if (k + 1 >= a.max_iter) {
+            done = 2;
+            iter = k + 1;
+        } else {
+            be = (float)(rn / rr);
+        }
+        *s_mode = done == 0 ? 0 : (done == 3 ? 2 : 1);
+        s_ab[0] = al;
+        s_ab[1] = be;
+        if (blockIdx.x == 0) {
+            st->alpha = al;
+            st->pt = pt;
+            st->rr_prev = rr;
+            st->rr = rn;
+            if (done) {
+                st->iter = iter;
+                st->done = done;
+                __hip_atomic_store(&st->stop, kk + 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+                st->beta = be;
+            }
+        }
+    }
+}
+
+template <int OP, int NT>
+__global__ void __launch_bounds__(NT) k_cg_iter3(StencilArgs a, CoefF cc, IterArgs it,
                                                           const int32_t* __restrict__ order) {
-    __shared__ float tile[kT * kPS];
+    constexpr int UI = (kUnits + NT - 1) / NT;   // 16-byte loads per thread and array
+    constexpr int OUT = 512 / NT;                // outputs per thread
+    static_assert(4 * NT * sizeof(double) <= kT * kPS * sizeof(float), "sums fit the tile");
+    __shared__ __align__(16) float tile[kT * kPS];   // also the scratch of the block sums
     __shared__ __align__(16) float psum[kT][4][64];
     // p and r of the own nodes by tile plane 3..13: planes 3..10 are the
     // brick's own z = 0..7, planes 11..13 the next brick's z = 0..2 when it
@@ -566,25 +579,12 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
     __shared__ double sred[4][4];
     __shared__ float s_ab[2];
     __shared__ int s_mode;
-    CgState* st = a.st;
     const int kk = a.kk;
     const int t = threadIdx.x;
-    // Everything the prologue reads goes out at once: the stop tag and the
-    // state (written by earlier launches only, so plain loads), the previous
-    // launch's partials (at most 4 x 256 per sum) and this block's first
-    // slots.  Every lane loads (indices past the partials read the last
-    // one): loads under a condition make the compiler's waits for them
-    // cover every later load.
-    const int stop = st->stop;
-    const double thr_rec = st->thr_rec;
-    const float st_alpha = st->alpha, st_beta = st->beta;
-    double v4[4][4];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int i = min(t + kS3Threads * u, it.nprev - 1);
-#pragma unroll
-        for (int q = 0; q < 4; q++) v4[q][u] = it.prev[q][i];
-    }
+    // everything the prologue reads goes out at once, this block's first
+    // slots included
+    IterHead<NT> hd;
+    hd.load(a, it);
     const int l = t & 63, wv = t >> 6;
     const int x = l & 7, y = l >> 3;
     const int nsl = (int)a.nslots;
@@ -598,7 +598,7 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
     const int nx0 = order[min(lo + 1, nsl - 1)];
     int nxt = lo + 1 < hi ? nx0 : -1;
     // a solve ended by an earlier launch (or before any): nothing to do
-    if (stop != 0 && stop != kk + 1) return;   // uniform over the grid
+    if (hd.stop != 0 && hd.stop != kk + 1) return;   // uniform over the grid
     {
         const int nb0 = a.nbr_slot[(int64_t)cur * 27 + min(t, 26)];
         if (t < 27) sbase[0][t] = (uint32_t)nb0 * 512u;
@@ -607,20 +607,20 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
     // halo (see k_stencil3) from unit u0 on -- a chained brick loads tile
     // planes 6..13 only: planes 0..5 are the previous brick's 8..13, whose
     // plane sums it copies.
-    float4 ra[kUnitIters], rb[kUnitIters], rv[kUnitIters], rc[kUnitIters];
-    float Vz[2], Dz[2], Pz[2], Xz[2];
+    float4 ra[UI], rb[UI], rv[UI], rc[UI];
+    float Vz[OUT], Dz[OUT], Pz[OUT], Xz[OUT];
     auto issue = [&](int64_t base, const uint32_t* sbc, int u0) {
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int64_t g = base + x + 8 * y + 64 * (2 * wv + q);
+        for (int q = 0; q < OUT; q++) {
+            const int64_t g = base + x + 8 * y + 64 * (OUT * wv + q);
             Vz[q] = a.vvol[g];
             Dz[q] = a.vdiag[g];
             Pz[q] = a.in[g];
             Xz[q] = a.xio[g];
         }
 #pragma unroll
-        for (int i = 0; i < kUnitIters; i++) {
-            const int u = u0 + t + kS3Threads * i;
+        for (int i = 0; i < UI; i++) {
+            const int u = u0 + t + NT * i;
             ra[i] = rb[i] = rv[i] = rc[i] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (u < kUnits) {
                 const int k = u & 3, line = u >> 2;
@@ -641,68 +641,7 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
             }
         }
     };
-    // alpha_(kk-1), beta_kk
-    if (it.resume) {
-        if (t == 0) {
-            s_mode = 0;
-            s_ab[0] = st_alpha;
-            s_ab[1] = st_beta;
-        }
-    } else {
-        double sv[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            double w[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) w[u] = t + kS3Threads * u < it.nprev ? v4[q][u] : 0.0;
-            sv[q] = (w[0] + w[1]) + (w[2] + w[3]);
-        }
-        // the four sums through LDS (psum is free here): wave w reduces sum
-        // w with one DPP tree instead of every wave reducing all four
-        block_sums4(sv, reinterpret_cast<double*>(&psum[0][0][0]), sred[0]);
-        if (t == 0) {
-            double sum[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) sum[q] = sred[0][q];
-            const double pt = sum[0], rt = sum[1], tt = sum[2], rr = sum[3];
-            const int k = a.iter_base + kk - 1;   // Eigen's index of the reduced SpMV
-            const double ald = rr / pt;
-            const float al = (float)ald;
-            const double a64 = (double)al;   // the alpha the vectors are updated with
-            const double rn = (rr - 2.0 * a64 * rt) + a64 * a64 * tt;
-            int done = 0, iter = 0;
-            float be = 0.f;
-            if (!isfinite(ald) || !isfinite(rn)) {
-                done = 3;
-                iter = k;
-            } else if (rn < thr_rec) {
-                done = 1;
-                iter = k;
-            } else if (k + 1 >= a.max_iter) {
-                done = 2;
-                iter = k + 1;
-            } else {
-                be = (float)(rn / rr);
-            }
-            s_mode = done == 0 ? 0 : (done == 3 ? 2 : 1);
-            s_ab[0] = al;
-            s_ab[1] = be;
-            if (blockIdx.x == 0) {
-                st->alpha = al;
-                st->pt = pt;
-                st->rr_prev = rr;
-                st->rr = rn;
-                if (done) {
-                    st->iter = iter;
-                    st->done = done;
-                    __hip_atomic_store(&st->stop, kk + 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                } else {
-                    st->beta = be;
-                }
-            }
-        }
-    }
+    iter_scalars<NT>(a, it, hd, reinterpret_cast<double*>(tile), sred[0], s_ab, &s_mode);
     __syncthreads();
     const int mode = s_mode;
     const float al = s_ab[0], be = s_ab[1];
@@ -711,7 +650,7 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
         // the solve ended: the last x update only (own nodes of every brick)
         for (int v = blockIdx.x; v < nsl; v += G) {
             const int64_t b0 = (int64_t)((G & 7) == 0 ? xcd_remap(v, nsl) : v) * 512;
-            for (int e = t; e < 512; e += kS3Threads)
+            for (int e = t; e < 512; e += NT)
                 a.xio[b0 + e] += al * a.in[b0 + e];
         }
         return;
@@ -733,11 +672,11 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
         const int nbv = a.nbr_slot[(int64_t)max(nxt, 0) * 27 + min(t, 26)];
         if (chained) {
             float4* ps4 = reinterpret_cast<float4*>(&psum[0][0][0]);
-            for (int e = t; e < 6 * 64; e += kS3Threads) ps4[e] = ps4[e + 8 * 64];
+            for (int e = t; e < 6 * 64; e += NT) ps4[e] = ps4[e + 8 * 64];
         }
 #pragma unroll
-        for (int i = 0; i < kUnitIters; i++) {
-            const int u = u0 + t + kS3Threads * i;
+        for (int i = 0; i < UI; i++) {
+            const int u = u0 + t + NT * i;
             if (u < kUnits) {
                 const int k = u & 3, line = u >> 2;
                 const int yt = line % kT, zt = line / kT;
@@ -783,7 +722,7 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
         }
         if (t < 27 && nxt >= 0) sbase[sb ^ 1][t] = (uint32_t)nbv * 512u;
         __syncthreads();
-        for (int zp = (chained ? 6 : 0) + wv; zp < kT; zp += 4) {
+        for (int zp = (chained ? 6 : 0) + wv; zp < kT; zp += NT / 64) {
             float P[4];
             plane4<kRS, float>(&tile[zp * kPS + (y + 3) * kRS + (x + 8)], cc, P);
 #pragma unroll
@@ -792,8 +731,8 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
         __syncthreads();
         // t = M p, and x, p, r of the own nodes
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int z = 2 * wv + q;
+        for (int q = 0; q < OUT; q++) {
+            const int z = OUT * wv + q;
             float acc = 0.f;
             acc += psum[z][3][l];
             acc += psum[z + 1][2][l];
@@ -825,8 +764,8 @@ __global__ void __launch_bounds__(kS3Threads) k_cg_iter3(StencilArgs a, CoefF cc
     }
     // this block's partials, one DPP tree per wave (see block_sums4)
     double rsum[4] = {red0, red1, red2, red3};
-    __syncthreads();   // the last brick's plane sums have been read
-    block_sums4(rsum, reinterpret_cast<double*>(&psum[0][0][0]), sred[1]);
+    // (every wave has passed the last brick's plane sums: the tile is free)
+    block_sums4<NT>(rsum, reinterpret_cast<double*>(tile), sred[1]);
     if (t < 4) {
         double* dst = t == 0 ? it.out[0] : (t == 1 ? it.out[1] : (t == 2 ? it.out[2] : it.out[3]));
         dst[blockIdx.x] = sred[1][t];
@@ -840,10 +779,6 @@ __global__ void __launch_bounds__(64) k_stencil2(StencilArgs a, C cc) {
     __shared__ float own[64];
     __shared__ double own64[KIND == K_TRUE_RES ? 64 : 1];
     __shared__ int64_t sbase[10];
-    float beta = 0.f;
-    if constexpr (KIND == K_SPMV_FIRST || KIND == K_SPMV_FUSED) {
-        if (!spmv_prologue(a, &beta)) return;
-    }
     if constexpr (KIND == K_TRUE_RES) {
         if (a.spec && a.st->done != 1) return;   // same value in every lane
     }
@@ -876,13 +811,10 @@ __global__ void __launch_bounds__(64) k_stencil2(StencilArgs a, C cc) {
             tile[e] = OP == VPS_OP_ROW ? (double)a.vvol[g] * xs : xs;
             if ((v >> 9) == 4) own64[v & 511] = xs;
         } else {
-            tile[e] = load_input<KIND, OP, T>(a, g, beta, &pn);
+            tile[e] = load_input<KIND, OP, T>(a, g, &pn);
         }
         if constexpr (KIND != K_DIAG && KIND != K_TRUE_RES) {
-            if ((v >> 9) == 4) {
-                own[v & 511] = pn;
-                if constexpr (KIND == K_SPMV_FUSED) a.out2[g] = pn;
-            }
+            if ((v >> 9) == 4) own[v & 511] = pn;
         }
     }
     __syncthreads();
@@ -916,12 +848,8 @@ __global__ void __launch_bounds__(64) k_stencil2(StencilArgs a, C cc) {
             const float b = a.vb[g];
             const float r = on ? b - mp : 0.f;
             a.out[g] = r;
-            a.out2[g] = r;
             red0 = (double)b * (double)b;
             red1 = (double)r * (double)r;
-        } else {
-            a.out[g] = mp;
-            red0 = (double)pi * (double)mp;
         }
     }
     if constexpr (KIND != K_DIAG && KIND != K_APPLY) {
@@ -934,65 +862,98 @@ __global__ void __launch_bounds__(64) k_stencil2(StencilArgs a, C cc) {
     }
 }
 
-// x += alpha p; r -= alpha t; partial r.r.  alpha = rr_{k-1} / (p.t)_k,
-// both re-summed from the producers' partials.
-__global__ void __launch_bounds__(kUpdThreads) k_cg_update(
-    int64_t n4, float4* x, float4* r, const float4* p, const float4* tt,
-    CgState* st, const double* pt_part, int npt, const double* rr_prev,
-    int kk, double* rr_out) {
-    __shared__ double sbuf[kUpdThreads / 64];
-    __shared__ int s_done;
-    // every load that does not depend on alpha is issued first: the state
-    // flag (read once per block, so the exit below is uniform), both
-    // partial sums and this thread's vector elements
-    if (threadIdx.x == 0) s_done = st->done;
-    const double abs0 = st->abs0;
-    double pt = 0, rp = 0;
-    for (int i = threadIdx.x; i < npt; i += kUpdThreads) pt += pt_part[i];
-    if (kk != 0)
-        for (int i = threadIdx.x; i < kUpdBlocks; i += kUpdThreads) rp += rr_prev[i];
-    const int64_t i0 = (int64_t)blockIdx.x * kUpdThreads + threadIdx.x;
-    const int64_t stride = (int64_t)kUpdBlocks * kUpdThreads;
-    float4 xv0{}, rv0{}, pv0{}, tv0{};
-    if (i0 < n4) {
-        xv0 = x[i0];
-        rv0 = r[i0];
-        pv0 = p[i0];
-        tv0 = tt[i0];
-    }
+// 2D CG iteration: one launch per iteration as in 3D.  A 2D system has few
+// nodes, so an iteration is bound by launches and dependent loads, not by
+// bandwidth: an SpMV and an update launch (6.7 + 4.1 us and two gaps at
+// 10,605 nodes) became one of 5.0 us.  One wave per 8x8 brick
+// (four bricks to a block, further bricks grid-strided).  The 14x14 halo is
+// 14 rows of four 16-byte half rows, 56 units: one unit of p, r and t per
+// lane, all issued before the previous launch's sums are formed.  Each wave
+// keeps its tile to itself, so no barrier is needed between its stages.
+template <int OP>
+__global__ void __launch_bounds__(256) k_cg_iter2(StencilArgs a, CoefF cc, IterArgs it) {
+    __shared__ __align__(16) float tile[4][kT * kRS];
+    __shared__ double scratch[4 * 256];
+    __shared__ double sred[2][4];
+    __shared__ float s_ab[2];
+    __shared__ int s_mode;
+    IterHead<256> hd;
+    hd.load(a, it);
+    const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int nsl = (int)a.nslots, G = (int)gridDim.x;
+    const int rbk = (G & 7) == 0 ? xcd_remap(blockIdx.x, G) : (int)blockIdx.x;
+    const int b0 = 4 * rbk + wv;
+    // this lane's unit: line yt of the tile, part k (see k_stencil3)
+    const int k = l & 3, yt = l >> 2;
+    const bool unit = l < 4 * kT;
+    const int nb = ((yt + 5) >> 3) * 3 + (k == 0 ? 0 : (k == 3 ? 2 : 1));
+    const int uloc = (k == 0 || k == 2 ? 4 : 0) + 8 * ((yt + 5) & 7);
+    const int32_t nbs = a.nbr_slot[(int64_t)min(b0, nsl - 1) * 27 + (unit ? nb : 4)];
+    // a solve ended by an earlier launch (or before any): nothing to do
+    if (hd.stop != 0 && hd.stop != a.kk + 1) return;   // uniform over the grid
+    float4 ra, rb, rc, rv = make_float4(0.f, 0.f, 0.f, 0.f);
+    float V, D, X, P, R, Tt;
+    auto issue = [&](int b, int32_t ns) {
+        const int64_t g = (int64_t)ns * 64 + uloc;
+        ra = *(const float4*)(a.in + g);
+        rb = *(const float4*)(a.in2 + g);
+        rc = *(const float4*)(a.in3 + g);
+        if constexpr (OP == VPS_OP_ROW) rv = *(const float4*)(a.vvol + g);
+        const int64_t o = (int64_t)b * 64 + l;
+        V = a.vvol[o];
+        D = a.vdiag[o];
+        X = a.xio[o];
+        P = a.in[o];
+        R = a.in2[o];
+        Tt = a.in3[o];
+    };
+    issue(min(b0, nsl - 1), nbs);
+    iter_scalars<256>(a, it, hd, scratch, sred[0], s_ab, &s_mode);
     __syncthreads();
-    if (s_done) return;
-    pt = block_sum<kUpdThreads>(pt, sbuf);
-    rp = kk == 0 ? abs0 : block_sum<kUpdThreads>(rp, sbuf);
-    const double ald = rp / pt;
-    if (!isfinite(ald)) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) st->done = 3;
-        return;
-    }
-    const float al = (float)ald;
-    double rr = 0;
-    for (int64_t i = i0; i < n4; i += stride) {
-        float4 xv, rv, pv, tv;
-        if (i == i0) {
-            xv = xv0; rv = rv0; pv = pv0; tv = tv0;
-        } else {
-            xv = x[i]; rv = r[i]; pv = p[i]; tv = tt[i];
+    const int mode = s_mode;
+    const float al = s_ab[0], be = s_ab[1];
+    if (mode == 2) return;   // non-finite alpha: no update
+    double rsum[4] = {0, 0, 0, 0};
+    float* tl = tile[wv];
+    const int x = l & 7, y = l >> 3;
+    for (int b = b0; b < nsl; b += 4 * G) {   // uniform over the wave
+        if (b != b0) issue(b, a.nbr_slot[(int64_t)b * 27 + (unit ? nb : 4)]);
+        const int64_t o = (int64_t)b * 64 + l;
+        a.xio[o] = X + al * P;
+        if (mode == 1) continue;   // the solve ended: the last x update only
+        float4 p;
+        p.x = (rb.x - al * rc.x) + be * ra.x;
+        p.y = (rb.y - al * rc.y) + be * ra.y;
+        p.z = (rb.z - al * rc.z) + be * ra.z;
+        p.w = (rb.w - al * rc.w) + be * ra.w;
+        if constexpr (OP == VPS_OP_ROW) {
+            p.x *= rv.x;
+            p.y *= rv.y;
+            p.z *= rv.z;
+            p.w *= rv.w;
         }
-        xv.x += al * pv.x;
-        xv.y += al * pv.y;
-        xv.z += al * pv.z;
-        xv.w += al * pv.w;
-        rv.x -= al * tv.x;
-        rv.y -= al * tv.y;
-        rv.z -= al * tv.z;
-        rv.w -= al * tv.w;
-        store_nt4((float*)&x[i], xv.x, xv.y, xv.z, xv.w);
-        store_nt4((float*)&r[i], rv.x, rv.y, rv.z, rv.w);
-        rr += ((double)rv.x * rv.x + (double)rv.y * rv.y) +
-              ((double)rv.z * rv.z + (double)rv.w * rv.w);
+        if (unit) *(float4*)(tl + yt * kRS + 4 + 4 * k) = p;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        const float acc = plane0<kRS>(tl + (y + 3) * kRS + (x + 8), cc);
+        __builtin_amdgcn_wave_barrier();   // the next brick overwrites the tile
+        const float ri = R - al * Tt, pi = ri + be * P;
+        const float mp = V > 0.f ? D * pi + (OP == VPS_OP_ROW ? acc : V * acc) : 0.f;
+        a.out[o] = mp;
+        a.out2[o] = pi;
+        a.out3[o] = ri;
+        rsum[0] += (double)pi * (double)mp;
+        rsum[1] += (double)ri * (double)mp;
+        rsum[2] += (double)mp * (double)mp;
+        rsum[3] += (double)ri * (double)ri;
     }
-    rr = block_sum<kUpdThreads>(rr, sbuf);
-    if (threadIdx.x == 0) rr_out[blockIdx.x] = rr;
+    if (mode == 1) return;
+    block_sums4<256>(rsum, scratch, sred[1]);
+    if (threadIdx.x < 4) {
+        const int t = threadIdx.x;
+        double* dst = t == 0 ? it.out[0] : (t == 1 ? it.out[1] : (t == 2 ? it.out[2] : it.out[3]));
+        dst[blockIdx.x] = sred[1][t];
+    }
 }
 
 // CG start: b.b and r0.r0 from the init partials -> tolerance, flags.
@@ -1038,8 +999,8 @@ __global__ void __launch_bounds__(1024) k_cg_start(const double* pbb,
     st->stop = st->done ? kStopBefore : 0;
 }
 
-// 3D residual replacement: r (the buffer the next iteration launch reads) takes the
-// FP64-checked true residual rt; partial r.r per block.
+// Residual replacement or restart: r (the buffer the next iteration launch reads)
+// takes the FP64-checked true residual rt; partial r.r per block.
 __global__ void __launch_bounds__(kUpdThreads) k_copy_rr(int64_t n4, const float4* rt,
                                                          float4* r, double* part) {
     __shared__ double sbuf[kUpdThreads / 64];
@@ -1125,70 +1086,6 @@ __global__ void __launch_bounds__(1024) k_sum_partials(const double* p, int n,
     if (threadIdx.x == 0) *out = a;
 }
 
-// The first SpMV leaves one partial per brick; the first iteration launch
-// reads them folded to G: partial g of sum q is the sum, in index order, of
-// bricks [g n / G, (g + 1) n / G), so that no block of that launch reads all
-// n (every block of an iteration launch sums every partial it is given).
-__global__ void __launch_bounds__(256) k_fold_partials(const double* p0, const double* p1,
-                                                       const double* p2, const double* p3,
-                                                       int n, int G, double* out0,
-                                                       double* out1, double* out2,
-                                                       double* out3) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= 4 * G) return;
-    const int q = i / G, g = i - q * G;
-    const double* p = q == 0 ? p0 : (q == 1 ? p1 : (q == 2 ? p2 : p3));
-    double* out = q == 0 ? out0 : (q == 1 ? out1 : (q == 2 ? out2 : out3));
-    const int a = (int)((int64_t)g * n / G), b = (int)((int64_t)(g + 1) * n / G);
-    double s = 0.0;
-    for (int j = a; j < b; j++) s += p[j];
-    out[g] = s;
-}
-
-// Residual replacement: r = rt; p = rt (restart direction); partial r.r.
-__global__ void __launch_bounds__(kUpdThreads) k_replace(int64_t n4,
-                                                         const float4* rt,
-                                                         float4* r, float4* p0,
-                                                         double* part) {
-    __shared__ double sbuf[kUpdThreads / 64];
-    double rr = 0;
-    for (int64_t i = (int64_t)blockIdx.x * kUpdThreads + threadIdx.x; i < n4;
-         i += (int64_t)kUpdBlocks * kUpdThreads) {
-        const float4 v = rt[i];
-        r[i] = v;
-        p0[i] = v;
-        rr += ((double)v.x * v.x + (double)v.y * v.y) +
-              ((double)v.z * v.z + (double)v.w * v.w);
-    }
-    rr = block_sum<kUpdThreads>(rr, sbuf);
-    if (threadIdx.x == 0) part[blockIdx.x] = rr;
-}
-
-// Residual replacement keeping the direction: r = rt; partial r.r into the
-// ring slot that the next SpMV reads as the newest r.r; the solve is open
-// again (block 0 clears the flag: no kernel of this launch reads it).
-__global__ void __launch_bounds__(kUpdThreads) k_replace_keep(int64_t n4,
-                                                              const float4* rt, float4* r,
-                                                              double* part, CgState* st) {
-    __shared__ double sbuf[kUpdThreads / 64];
-    double rr = 0;
-    for (int64_t i = (int64_t)blockIdx.x * kUpdThreads + threadIdx.x; i < n4;
-         i += (int64_t)kUpdBlocks * kUpdThreads) {
-        const float4 v = rt[i];
-        r[i] = v;
-        rr += ((double)v.x * v.x + (double)v.y * v.y) +
-              ((double)v.z * v.z + (double)v.w * v.w);
-    }
-    rr = block_sum<kUpdThreads>(rr, sbuf);
-    if (threadIdx.x == 0) {
-        part[blockIdx.x] = rr;
-        if (blockIdx.x == 0) {
-            st->done = 0;
-            st->true_rr = -1.0;
-        }
-    }
-}
-
 // After a replacement: the restart's r.r becomes abs0.
 __global__ void __launch_bounds__(1024) k_restart(const double* part,
                                                   CgState* st) {
@@ -1199,6 +1096,8 @@ __global__ void __launch_bounds__(1024) k_restart(const double* part,
     if (threadIdx.x == 0) {
         st->abs0 = a;
         st->rr = a;
+        st->alpha = 0.f;
+        st->beta = 0.f;
         st->final_kk = -1;
         st->done = a < st->thr ? 1 : 0;
         st->stop = st->done ? kStopBefore : 0;
@@ -1257,40 +1156,23 @@ static void make_coef(const vps_context* c, CoefD* d, CoefF* f) {
     }
 }
 
-// Partials layout (doubles): [3 x nbricks] SpMV ring, [3 x 256] update
-// ring, [2 x nbricks] init, [nbricks] true residual, [256] replacement,
-// [2048] misc.
-static double* part_pt(vps_context* c, int k) {
-    return c->partials.p + (int64_t)(k % 3) * c->nbricks;
-}
-static double* part_rr(vps_context* c, int k) {
-    return c->partials.p + 3 * c->nbricks + (int64_t)(k % 3) * kUpdBlocks;
-}
+// Partials layout (doubles): [2 x nbricks] init, [nbricks] true residual,
+// [256] replacement, [2048] misc, [8 x kIterBlocks] the iteration launches'
+// two sets of four sums.
 static double* part_init(vps_context* c, int which) {
-    return c->partials.p + 3 * c->nbricks + 3 * kUpdBlocks +
-           (int64_t)which * c->nbricks;
+    return c->partials.p + (int64_t)which * c->nbricks;
 }
-static double* part_true(vps_context* c) {
-    return c->partials.p + 5 * c->nbricks + 3 * kUpdBlocks;
-}
-static double* part_repl(vps_context* c) {
-    return c->partials.p + 6 * c->nbricks + 3 * kUpdBlocks;
-}
+static double* part_true(vps_context* c) { return c->partials.p + 2 * c->nbricks; }
+static double* part_repl(vps_context* c) { return c->partials.p + 3 * c->nbricks; }
 static double* part_misc(vps_context* c) {
-    return c->partials.p + 6 * c->nbricks + 4 * kUpdBlocks;
+    return c->partials.p + 3 * c->nbricks + kUpdBlocks;
 }
-// the second set of the 3D iteration's partials (the first: the SpMV ring)
 static double* part_iter(vps_context* c, int q) {
-    return c->partials.p + 6 * c->nbricks + 4 * kUpdBlocks + 2048 + (int64_t)q * kIterBlocks;
-}
-// the first SpMV's per-brick partials folded to one per iteration block
-static double* part_fold(vps_context* c, int q) {
-    return c->partials.p + 6 * c->nbricks + 4 * kUpdBlocks + 2048 +
-           (int64_t)(4 + q) * kIterBlocks;
+    return c->partials.p + 3 * c->nbricks + kUpdBlocks + 2048 + (int64_t)q * kIterBlocks;
 }
 
 int64_t partials_size(int64_t nbricks) {
-    return 6 * nbricks + 4 * kUpdBlocks + 2048 + 8 * kIterBlocks;
+    return 3 * nbricks + kUpdBlocks + 2048 + 8 * kIterBlocks;
 }
 
 static StencilArgs base_args(vps_context* c) {
@@ -1311,35 +1193,19 @@ static StencilArgs base_args(vps_context* c) {
     return a;
 }
 
-// With a pair of events the launch goes through hipExtLaunchKernelGGL, which
-// stamps them at the start and the end of the kernel's own execution (no
-// dispatch gap in the measured time).
 template <int KIND, int OP, typename T, typename C>
-static void launch(vps_context* c, const StencilArgs& a, const C& cc,
-                   hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
+static void launch(vps_context* c, const StencilArgs& a, const C& cc) {
     const dim3 grid((unsigned)c->nslots), block(64), block3(kS3Threads);
-    if (c->dim == 3) {
-        if (e0)
-            hipExtLaunchKernelGGL((k_stencil3<KIND, OP, T, C>), grid, block3, 0,
-                                  c->stream, e0, e1, 0, a, cc);
-        else
-            hipLaunchKernelGGL((k_stencil3<KIND, OP, T, C>), grid, block3, 0,
-                               c->stream, a, cc);
-    } else {
-        if (e0)
-            hipExtLaunchKernelGGL((k_stencil2<KIND, OP, T, C>), grid, block, 0,
-                                  c->stream, e0, e1, 0, a, cc);
-        else
-            hipLaunchKernelGGL((k_stencil2<KIND, OP, T, C>), grid, block, 0,
-                               c->stream, a, cc);
-    }
+    if (c->dim == 3)
+        hipLaunchKernelGGL((k_stencil3<KIND, OP, T, C>), grid, block3, 0, c->stream, a, cc);
+    else
+        hipLaunchKernelGGL((k_stencil2<KIND, OP, T, C>), grid, block, 0, c->stream, a, cc);
 }
 
 template <int KIND, typename T, typename C>
-static void launch_op(vps_context* c, const StencilArgs& a, const C& cc,
-                      hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr) {
-    if (c->p.op_mode == VPS_OP_ROW) launch<KIND, VPS_OP_ROW, T, C>(c, a, cc, e0, e1);
-    else launch<KIND, VPS_OP_TRANSPOSE, T, C>(c, a, cc, e0, e1);
+static void launch_op(vps_context* c, const StencilArgs& a, const C& cc) {
+    if (c->p.op_mode == VPS_OP_ROW) launch<KIND, VPS_OP_ROW, T, C>(c, a, cc);
+    else launch<KIND, VPS_OP_TRANSPOSE, T, C>(c, a, cc);
 }
 
 int virtual_diag(vps_context* c, bool set_alpha0) {
@@ -1404,17 +1270,28 @@ static double ms_between(hipEvent_t a, hipEvent_t b) {
     return ms;
 }
 
-// Persistent blocks of the 3D iteration: all resident at once (blocks per CU
-// from the occupancy of k_cg_iter3, at most three, times the CUs, at most
-// kIterBlocks), so that no block waits for another to finish.
+using IterKernel3 = void (*)(StencilArgs, CoefF, IterArgs, const int32_t*);
+using IterKernel2 = void (*)(StencilArgs, CoefF, IterArgs);
+
+static IterKernel3 iter_kernel3(const vps_context* c) {
+    return c->p.op_mode == VPS_OP_ROW ? k_cg_iter3<VPS_OP_ROW, kS3Threads>
+                                      : k_cg_iter3<VPS_OP_TRANSPOSE, kS3Threads>;
+}
+static IterKernel2 iter_kernel2(const vps_context* c) {
+    return c->p.op_mode == VPS_OP_ROW ? k_cg_iter2<VPS_OP_ROW> : k_cg_iter2<VPS_OP_TRANSPOSE>;
+}
+
+// Persistent blocks of the iteration launches: all resident at once (blocks
+// per CU from the occupancy of the kernel, at most three, times the CUs, at
+// most kIterBlocks), so that no block waits for another to finish.
 static int iter_blocks(vps_context* c) {
     static int cached[64][2] = {};
     const int dev = c->device >= 0 && c->device < 64 ? c->device : 0;
-    const int op = c->p.op_mode == VPS_OP_ROW ? 1 : 0;
-    if (cached[dev][op] > 0) return cached[dev][op];
+    const int which = c->dim == 2 ? 1 : 0;
+    if (cached[dev][which] > 0) return cached[dev][which];
     int per_cu = 0, cus = 0;
-    const auto kern = c->p.op_mode == VPS_OP_ROW ? (const void*)k_cg_iter3<VPS_OP_ROW>
-                                                 : (const void*)k_cg_iter3<VPS_OP_TRANSPOSE>;
+    const void* kern = c->dim == 2 ? (const void*)iter_kernel2(c)
+                                   : (const void*)iter_kernel3(c);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kS3Threads, 0) !=
             hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) !=
@@ -1427,7 +1304,7 @@ static int iter_blocks(vps_context* c) {
     // 21.7 us per launch, 8.1M: 120 against 125 us), with longer z-runs per
     // block and less contention for LDS and the caches
     const int n = std::max(8, std::min(kIterBlocks, std::min(per_cu, 3) * cus) & ~7);
-    cached[dev][op] = n;
+    cached[dev][which] = n;
     return n;
 }
 
@@ -1453,10 +1330,6 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     const int64_t max_iter =
         c->p.max_iterations >= 0 ? c->p.max_iterations : 2 * c->nvirt;
     float* x = c->vx[w].p;
-    float* r = c->vr.p;
-    float* t = c->vt.p;
-    float* p0 = c->vp[0].p;
-    float* p1 = c->vp[1].p;
     const int nslots = (int)c->nslots;
     // x = xb (FP64) + x (FP32 correction) during the solve; every return
     // after the split leaves the pressures in x
@@ -1483,19 +1356,23 @@ int cg_solve(vps_context* c, vps_stats* stats) {
         return rc;
     };
 
+    // ping-pong vectors of the iteration launches: launch kk reads the set
+    // (kk - 1) & 1 and writes kk & 1, so the start's residual goes to set 1
+    float* pb[2] = {c->vp[0].p, c->vp[1].p};
+    float* rbuf[2] = {c->vr.p, c->vr2.p};
+    float* tbuf[2] = {c->vt.p, c->vt2.p};
     {
         StencilArgs a = base_args(c);
         a.in = x;
-        a.out = r;
-        a.out2 = p0;
+        a.out = rbuf[1];
         a.part0 = part_init(c, 0);
         a.part1 = part_init(c, 1);
         launch_op<K_CG_INIT, float, CoefF>(c, a, cf);
         fold(kFoldSplit);
-        // 3D: the recursion's threshold absorbs the FP32 drift measured at
-        // the last solve (with a 10% margin); the FP64 check keeps tol
+        // the recursion's threshold absorbs the FP32 drift measured at the
+        // last solve (with a 10% margin); the FP64 check keeps tol
         double rec_scale = 1.0;
-        if (c->dim == 3 && c->cg_drift > 0.9) rec_scale = std::max(0.25, 0.9 / c->cg_drift);
+        if (c->cg_drift > 0.9) rec_scale = std::max(0.25, 0.9 / c->cg_drift);
         hipLaunchKernelGGL(k_cg_start, dim3(1), dim3(1024), 0, c->stream,
                            part_init(c, 0), part_init(c, 1), nslots, tol_in, rec_scale,
                            c->start_guard ? 1 : 0, c->cg.p);
@@ -1528,17 +1405,13 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     // convergence returns at its prologue in a few us; a batch that stops
     // short costs a host round trip of about 30 us)
     int predicted = c->prev_iters > 0 ? c->prev_iters + 3 : 8;
-    // 3D: ping-pong vectors of the one-launch iteration; resume_pending: the
-    // next launch is an update after a replacement (no reduction before it)
+    // resume_pending: the next launch takes alpha and beta from the state (a
+    // start: zero; after a replacement: alpha zero)
+    bool resume_pending = true;
+    // persistent blocks of the iteration and its two partial sets
     const bool three = c->dim == 3;
-    float* pb[2] = {p0, p1};
-    float* rbuf[2] = {r, c->vr2.p};
-    float* tbuf[2] = {t, c->vt2.p};
-    bool resume_pending = false;
-    // 3D: persistent blocks of the iteration and its two partial sets
-    const int giter = nslots >= 8 ? (std::min(nslots, iter_blocks(c)) & ~7) : nslots;
-    double* setA[4] = {part_pt(c, 0), part_pt(c, 1), part_pt(c, 2), part_init(c, 1)};
-    double* setB[4] = {part_iter(c, 0), part_iter(c, 1), part_iter(c, 2), part_iter(c, 3)};
+    const int nblk = three ? nslots : (nslots + 3) / 4;
+    const int giter = nblk >= 8 ? (std::min(nblk, iter_blocks(c)) & ~7) : nblk;
     std::vector<int> timed_iter;
     double host_launch_us = 0;
     bool post_queued = false;   // the guarded post-solve work follows this state
@@ -1547,115 +1420,50 @@ int cg_solve(vps_context* c, vps_stats* stats) {
             int batch = iter_base + kk < predicted ? predicted - (iter_base + kk) : 4;
             if (batch > 64) batch = 64;
             const auto h0 = std::chrono::steady_clock::now();
-            for (int j = 0; j < batch && three; j++) {
-                // 3D: FIRST, then per iteration one launch of persistent
-                // blocks: the sums of the previous SpMV, the update, the SpMV
+            for (int j = 0; j < batch; j++) {
+                // one launch of persistent blocks: the sums of the previous
+                // launch, the update, the SpMV.  Launch 0 of a (re)start has
+                // no direction yet: with alpha = beta = 0 it forms p = r and
+                // t = M p, reading r in the place of p and t.
                 StencilArgs s = base_args(c);
                 s.kk = kk;
                 s.iter_base = iter_base;
                 s.max_iter = max_iter;
-                s.part0 = part_pt(c, 0);
-                s.part1 = part_pt(c, 1);
-                s.part2 = part_pt(c, 2);
-                s.part3 = part_init(c, 1);   // free once k_cg_start has run
-                if (kk == 0) {
-                    s.in = p0;
-                    s.out = t;
-                    launch_op<K_SPMV_FIRST, float, CoefF>(c, s, cf);
-                    hipLaunchKernelGGL(k_fold_partials, dim3((unsigned)((4 * giter + 255) / 256)),
-                                       dim3(256), 0, c->stream, setA[0], setA[1], setA[2],
-                                       setA[3], nslots, giter, part_fold(c, 0), part_fold(c, 1),
-                                       part_fold(c, 2), part_fold(c, 3));
-                    spmv_launches++;
-                    kk++;
-                    continue;
-                }
-                // (an update resumed after a replacement: not timed)
+                // (an update resumed from the state: not timed)
                 const bool do_time = prof && timed < max_timed && !resume_pending;
                 hipEvent_t* ev = do_time ? &c->kev[4 * timed] : nullptr;
-                const int o = (kk - 1) & 1, nw = kk & 1;
-                s.in = pb[o];
+                const int o = (kk + 1) & 1, nw = kk & 1;
+                s.in = kk == 0 ? rbuf[o] : pb[o];
                 s.in2 = rbuf[o];
-                s.in3 = tbuf[o];
+                s.in3 = kk == 0 ? rbuf[o] : tbuf[o];
                 s.out = tbuf[nw];
                 s.out2 = pb[nw];
                 s.out3 = rbuf[nw];
                 s.xio = x;
-                // partials: FIRST writes set A (one per slot), folded to one
-                // per block for launch 1; launch kk writes set B when kk is
-                // odd, A when even, and reads the other
                 IterArgs ia;
-                const int32_t* corder = c->col_order.p;
                 for (int q = 0; q < 4; q++) {
-                    ia.out[q] = nw ? setB[q] : setA[q];
-                    ia.prev[q] = kk == 1 ? part_fold(c, q) : (nw ? setA[q] : setB[q]);
+                    ia.out[q] = part_iter(c, 4 * nw + q);
+                    ia.prev[q] = part_iter(c, 4 * o + q);
                 }
                 ia.nprev = giter;
                 ia.resume = resume_pending ? 1 : 0;
                 resume_pending = false;
                 const dim3 gi((unsigned)giter), bi(kS3Threads);
-                if (c->p.op_mode == VPS_OP_ROW) {
-                    if (ev)
-                        hipExtLaunchKernelGGL(k_cg_iter3<VPS_OP_ROW>, gi, bi, 0, c->stream, ev[0],
-                                              ev[1], 0, s, cf, ia, corder);
-                    else
-                        hipLaunchKernelGGL(k_cg_iter3<VPS_OP_ROW>, gi, bi, 0, c->stream, s, cf, ia,
-                                           corder);
-                } else {
-                    if (ev)
-                        hipExtLaunchKernelGGL(k_cg_iter3<VPS_OP_TRANSPOSE>, gi, bi, 0, c->stream,
-                                              ev[0], ev[1], 0, s, cf, ia, corder);
-                    else
-                        hipLaunchKernelGGL(k_cg_iter3<VPS_OP_TRANSPOSE>, gi, bi, 0, c->stream, s,
-                                           cf, ia, corder);
-                }
+                const int32_t* corder = c->col_order.p;
+                if (three && ev)
+                    hipExtLaunchKernelGGL(iter_kernel3(c), gi, bi, 0, c->stream, ev[0],
+                                          ev[1], 0, s, cf, ia, corder);
+                else if (three)
+                    hipLaunchKernelGGL(iter_kernel3(c), gi, bi, 0, c->stream, s, cf, ia,
+                                       corder);
+                else if (ev)
+                    hipExtLaunchKernelGGL(iter_kernel2(c), gi, bi, 0, c->stream, ev[0], ev[1], 0,
+                                          s, cf, ia);
+                else
+                    hipLaunchKernelGGL(iter_kernel2(c), gi, bi, 0, c->stream, s, cf, ia);
                 if (do_time) {
                     // an iteration of index kk - 1 (its reduction and update)
                     timed_iter.push_back(iter_base + kk - 1);
-                    timed++;
-                }
-                spmv_launches++;
-                kk++;
-            }
-            for (int j = 0; j < batch && !three; j++) {
-                StencilArgs s = base_args(c);
-                s.kk = kk;
-                s.iter_base = iter_base;
-                s.max_iter = max_iter;
-                s.rr1 = part_rr(c, kk + 2);   // (kk - 1) mod 3
-                s.rr2 = part_rr(c, kk + 1);   // (kk - 2) mod 3
-                s.part0 = part_pt(c, kk);
-                s.out = t;
-                float* dir = (kk == 0) ? p0 : ((kk & 1) ? p1 : p0);
-                // the first SpMV of a (re)start is not fused: only fused
-                // launches are timed
-                const bool do_time = prof && timed < max_timed && kk > 0;
-                hipEvent_t* ev = do_time ? &c->kev[4 * timed] : nullptr;
-                if (kk == 0) {
-                    s.in = p0;
-                    launch_op<K_SPMV_FIRST, float, CoefF>(c, s, cf);
-                } else {
-                    s.in = (kk & 1) ? p0 : p1;   // previous direction
-                    s.in2 = r;
-                    s.out2 = dir;
-                    launch_op<K_SPMV_FUSED, float, CoefF>(c, s, cf,
-                                                          ev ? ev[0] : nullptr,
-                                                          ev ? ev[1] : nullptr);
-                }
-                if (ev)
-                    hipExtLaunchKernelGGL(k_cg_update, dim3(kUpdBlocks), dim3(kUpdThreads),
-                                          0, c->stream, ev[2], ev[3], 0, n4, (float4*)x,
-                                          (float4*)r, (const float4*)dir,
-                                          (const float4*)t, c->cg.p, part_pt(c, kk),
-                                          nslots, part_rr(c, kk + 2), kk, part_rr(c, kk));
-                else
-                    hipLaunchKernelGGL(k_cg_update, dim3(kUpdBlocks), dim3(kUpdThreads),
-                                       0, c->stream, n4, (float4*)x, (float4*)r,
-                                       (const float4*)dir, (const float4*)t, c->cg.p,
-                                       part_pt(c, kk), nslots, part_rr(c, kk + 2), kk,
-                                       part_rr(c, kk));
-                if (do_time) {
-                    timed_iter.push_back(iter_base + kk);
                     timed++;
                 }
                 spmv_launches++;
@@ -1667,7 +1475,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
                 StencilArgs tr = base_args(c);
                 tr.in = x;
                 tr.in_base = xb;
-                tr.out = three ? c->vrt.p : t;   // r_true
+                tr.out = c->vrt.p;   // r_true
                 tr.part0 = part_true(c);
                 tr.spec = 1;
                 launch_op<K_TRUE_RES, double, CoefD>(c, tr, cd);
@@ -1736,7 +1544,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
             c->spec_done = post_queued;
             break;
         }
-        if (three && replacements == 0 && hs.rr > 0 && hs.true_rr >= 0 &&
+        if (replacements == 0 && hs.rr > 0 && hs.true_rr >= 0 &&
             std::isfinite(hs.true_rr / hs.rr))
             c->cg_drift = hs.true_rr / hs.rr;
         if (hs.true_rr < hs.thr) {
@@ -1752,7 +1560,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
         // the correction so far goes into the FP64 base; the iteration goes
         // on with a fresh FP32 correction from the true residual
         fold(kFoldMerge);
-        if (three && hs.iter > iter_base) {
+        if (hs.iter > iter_base) {
             // residual replacement (van der Vorst and Ye): r takes the true
             // residual, the direction is kept and the iteration continues
             // from the same x.  The launch that applied the last update
@@ -1769,28 +1577,13 @@ int cg_solve(vps_context* c, vps_stats* stats) {
             predicted = iter_base + kk + 2;
             continue;
         }
-        if (!three && hs.iter > iter_base) {
-            // residual replacement (van der Vorst and Ye): r takes the true
-            // residual, the direction is kept and the iteration continues
-            // where convergence was declared.  The SpMV that declared it is
-            // launched again: its prologue forms beta from the new r.r,
-            // written into the ring slot of the previous update.
-            kk = hs.iter - iter_base + 1;
-            hipLaunchKernelGGL(k_replace_keep, dim3(kUpdBlocks), dim3(kUpdThreads), 0,
-                               c->stream, n4, (const float4*)t, (float4*)r,
-                               part_rr(c, kk + 2), c->cg.p);
-            VPS_HIP(c, hipGetLastError());
-            hs.done = 0;   // k_replace_keep reopened the solve on the device
-            predicted = iter_base + kk + 2;
-            continue;
-        }
         // converged before any iteration of this (re)start: restart from the
         // true residual
         iter_base = hs.iter;
         kk = 0;
-        hipLaunchKernelGGL(k_replace, dim3(kUpdBlocks), dim3(kUpdThreads), 0,
-                           c->stream, n4, (const float4*)(three ? c->vrt.p : t), (float4*)r,
-                           (float4*)p0, part_repl(c));
+        resume_pending = true;
+        hipLaunchKernelGGL(k_copy_rr, dim3(kUpdBlocks), dim3(kUpdThreads), 0, c->stream, n4,
+                           (const float4*)c->vrt.p, (float4*)rbuf[1], part_repl(c));
         hipLaunchKernelGGL(k_restart, dim3(1), dim3(1024), 0, c->stream,
                            part_repl(c), c->cg.p);
         VPS_HIP(c, hipGetLastError());
@@ -1801,13 +1594,11 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     if (!c->spec_done) fold(kFoldFinal);
     VPS_HIP(c, hipGetLastError());
     c->prev_iters = hs.iter;
-    double spmv_ms = 0, upd_ms = 0;
+    double spmv_ms = 0;
     int64_t counted = 0;
     for (int64_t j = 0; j < timed; j++) {
         if (timed_iter[(size_t)j] > hs.iter) break;   // no-op launches
         spmv_ms += ms_between(c->kev[4 * j], c->kev[4 * j + 1]);
-        // 3D: the update is part of the iteration launch
-        if (!three) upd_ms += ms_between(c->kev[4 * j + 2], c->kev[4 * j + 3]);
         counted++;
     }
     if (stats) {
@@ -1819,7 +1610,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
         stats->rhs_norm = std::sqrt(hs.bb);
         stats->spmv_launches = spmv_launches;
         stats->ms_spmv_avg = counted ? spmv_ms / counted : 0;
-        stats->ms_update_avg = counted ? upd_ms / counted : 0;
+        stats->ms_update_avg = 0;   // the update is part of the iteration launch
         stats->reserved[0] = replacements;
         stats->reserved[1] = (int64_t)host_launch_us;   // host time spent launching
     }
