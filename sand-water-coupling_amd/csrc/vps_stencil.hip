@@ -1270,42 +1270,57 @@ static double ms_between(hipEvent_t a, hipEvent_t b) {
     return ms;
 }
 
-using IterKernel3 = void (*)(StencilArgs, CoefF, IterArgs, const int32_t*);
-using IterKernel2 = void (*)(StencilArgs, CoefF, IterArgs);
+// An iteration launch: the kernel, its threads and its blocks, all resident at
+// once (the rules below stay within the occupancy of the kernels), so that no
+// block waits for another to finish.
+struct IterLaunch {
+    void (*kern3)(StencilArgs, CoefF, IterArgs, const int32_t*) = nullptr;
+    void (*kern2)(StencilArgs, CoefF, IterArgs) = nullptr;
+    int threads = 256, blocks = 0;
+};
 
-static IterKernel3 iter_kernel3(const vps_context* c) {
-    return c->p.op_mode == VPS_OP_ROW ? k_cg_iter3<VPS_OP_ROW, kS3Threads>
-                                      : k_cg_iter3<VPS_OP_TRANSPOSE, kS3Threads>;
-}
-static IterKernel2 iter_kernel2(const vps_context* c) {
-    return c->p.op_mode == VPS_OP_ROW ? k_cg_iter2<VPS_OP_ROW> : k_cg_iter2<VPS_OP_TRANSPOSE>;
-}
-
-// Persistent blocks of the iteration launches: all resident at once (blocks
-// per CU from the occupancy of the kernel, at most three, times the CUs, at
-// most kIterBlocks), so that no block waits for another to finish.
-static int iter_blocks(vps_context* c) {
-    static int cached[64][2] = {};
+// The 3D rule, from launches timed at 12, 270, 600, 2,411 and 18,720 bricks
+// (us per launch, 256 threads and three blocks per CU against 512 threads):
+//   8.96 / 7.8   9.5 / 7.75   10.2 / 9.9   20.7 / 20.2   118 / 137
+// Up to a few bricks per block the launch is one chain of loads, sums and
+// barriers, which 512 threads per brick shorten (two rounds of loads and
+// plane sums instead of four); with a dozen bricks per CU and more the
+// launch streams from HBM, where smaller blocks overlap better.  Of the
+// wide blocks one per CU is best while nearly all of them hold one brick
+// (270 bricks: 7.75 with 256 blocks, 8.5 with 264), two beyond (600 bricks:
+// 9.8 against 10.1).
+static IterLaunch iter_launch(const vps_context* c, int nslots) {
+    static int cus_of[64] = {};
     const int dev = c->device >= 0 && c->device < 64 ? c->device : 0;
-    const int which = c->dim == 2 ? 1 : 0;
-    if (cached[dev][which] > 0) return cached[dev][which];
-    int per_cu = 0, cus = 0;
-    const void* kern = c->dim == 2 ? (const void*)iter_kernel2(c)
-                                   : (const void*)iter_kernel3(c);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kS3Threads, 0) !=
-            hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) !=
-            hipSuccess ||
-        per_cu <= 0 || cus <= 0) {
-        (void)hipGetLastError();
-        return kIterBlocks;
+    if (cus_of[dev] == 0) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, c->device) !=
+                hipSuccess ||
+            n <= 0) {
+            (void)hipGetLastError();
+            n = 256;
+        }
+        cus_of[dev] = n;
     }
-    // three blocks per CU: measured faster than four (1M: 21.2 against
-    // 21.7 us per launch, 8.1M: 120 against 125 us), with longer z-runs per
-    // block and less contention for LDS and the caches
-    const int n = std::max(8, std::min(kIterBlocks, std::min(per_cu, 3) * cus) & ~7);
-    cached[dev][which] = n;
-    return n;
+    const int cus = cus_of[dev];
+    const bool row = c->p.op_mode == VPS_OP_ROW;
+    IterLaunch L;
+    int work, per_cu;
+    if (c->dim == 2) {
+        L.kern2 = row ? k_cg_iter2<VPS_OP_ROW> : k_cg_iter2<VPS_OP_TRANSPOSE>;
+        work = (nslots + 3) / 4;
+        per_cu = 3;
+    } else {
+        const bool wide = nslots <= 12 * cus;
+        if (wide) L.kern3 = row ? k_cg_iter3<VPS_OP_ROW, 512> : k_cg_iter3<VPS_OP_TRANSPOSE, 512>;
+        else L.kern3 = row ? k_cg_iter3<VPS_OP_ROW, 256> : k_cg_iter3<VPS_OP_TRANSPOSE, 256>;
+        L.threads = wide ? 512 : 256;
+        work = nslots;
+        per_cu = !wide ? 3 : (4 * nslots <= 5 * cus ? 1 : 2);
+    }
+    const int most = std::min(kIterBlocks, per_cu * cus);
+    L.blocks = work >= 8 ? std::max(8, std::min(work, most) & ~7) : work;
+    return L;
 }
 
 // residual replacements of one solve before it fails (the FP64 base of x
@@ -1410,8 +1425,8 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     bool resume_pending = true;
     // persistent blocks of the iteration and its two partial sets
     const bool three = c->dim == 3;
-    const int nblk = three ? nslots : (nslots + 3) / 4;
-    const int giter = nblk >= 8 ? (std::min(nblk, iter_blocks(c)) & ~7) : nblk;
+    const IterLaunch il = iter_launch(c, nslots);
+    const int giter = il.blocks;
     std::vector<int> timed_iter;
     double host_launch_us = 0;
     bool post_queued = false;   // the guarded post-solve work follows this state
@@ -1448,19 +1463,18 @@ int cg_solve(vps_context* c, vps_stats* stats) {
                 ia.nprev = giter;
                 ia.resume = resume_pending ? 1 : 0;
                 resume_pending = false;
-                const dim3 gi((unsigned)giter), bi(kS3Threads);
+                const dim3 gi((unsigned)giter), bi((unsigned)il.threads);
                 const int32_t* corder = c->col_order.p;
                 if (three && ev)
-                    hipExtLaunchKernelGGL(iter_kernel3(c), gi, bi, 0, c->stream, ev[0],
-                                          ev[1], 0, s, cf, ia, corder);
+                    hipExtLaunchKernelGGL(il.kern3, gi, bi, 0, c->stream, ev[0], ev[1], 0, s, cf,
+                                          ia, corder);
                 else if (three)
-                    hipLaunchKernelGGL(iter_kernel3(c), gi, bi, 0, c->stream, s, cf, ia,
-                                       corder);
+                    hipLaunchKernelGGL(il.kern3, gi, bi, 0, c->stream, s, cf, ia, corder);
                 else if (ev)
-                    hipExtLaunchKernelGGL(iter_kernel2(c), gi, bi, 0, c->stream, ev[0], ev[1], 0,
-                                          s, cf, ia);
+                    hipExtLaunchKernelGGL(il.kern2, gi, bi, 0, c->stream, ev[0], ev[1], 0, s, cf,
+                                          ia);
                 else
-                    hipLaunchKernelGGL(iter_kernel2(c), gi, bi, 0, c->stream, s, cf, ia);
+                    hipLaunchKernelGGL(il.kern2, gi, bi, 0, c->stream, s, cf, ia);
                 if (do_time) {
                     // an iteration of index kk - 1 (its reduction and update)
                     timed_iter.push_back(iter_base + kk - 1);
