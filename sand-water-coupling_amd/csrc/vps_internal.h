@@ -431,6 +431,9 @@ struct vps_context {
     vps::DBuf<float4> vel_next;         // velocities after a Jacobi pass (DEM, viscosity)
     vps::DBuf<double> couple_stage;     // grain coupling: boundary x, n, v
     int64_t couple_walls = -1;          // walls already staged there (-1: none)
+    vps::DBuf<double> io_stage;         // host state in and out, caller layout
+    char* io_host = nullptr;            // two pinned pieces of io_host_piece bytes
+    size_t io_host_piece = 0;
     vps::DBuf<int32_t> cell_of, slot_of, perm;
     int64_t ncells = 0;
     vps::DBuf<int32_t> cell_count, cell_start;
