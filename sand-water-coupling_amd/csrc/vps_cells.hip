@@ -223,29 +223,13 @@ __global__ void __launch_bounds__(256) k_density3f(const double4* pos, const flo
     }
 }
 
-// FP32 offset of every (sorted) particle from its cell corner; w = its cell
-// x + 1, negated when the particle is clamped into a border cell (|offset|
-// > 2 cells).  The walks read the sign; the density also the cell.
+// FP32 offset of every (sorted) particle (see cell_offset3).  The walks read
+// the sign of w; the density also the cell.
 __global__ void __launch_bounds__(256) k_cell_offsets3(const double4* pos,
                                                        int64_t n, KConst k,
                                                        float4* ofs) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const double4 p = pos[i];
-    const double pc[3] = {p.x, p.y, p.z};
-    const float far = 2.f * (float)k.cell_size;
-    float of[3];
-    bool is_far = false;
-    int cx = 0;
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        const int c = cell_coord(pc[a], k.cell_lo[a], k.cell_inv, k.cdims[a]);
-        if (a == 0) cx = c;
-        of[a] = (float)(pc[a] - cell_corner(k, a, c));
-        is_far |= !(fabsf(of[a]) <= far);
-    }
-    const float w = (float)(cx + 1);
-    ofs[i] = make_float4(of[0], of[1], of[2], is_far ? -w : w);
+    if (i < n) ofs[i] = cell_offset3(k, pos[i]);
 }
 
 // Boundary density from boundary-only neighbours (the boundary set has its

@@ -224,6 +224,26 @@ __device__ __forceinline__ double cell_corner(const KConst& k, int a, int c) {
     return k.cell_lo[a] + (double)c * k.cell_size;
 }
 
+// FP32 offset of a 3D particle from its cell corner; w = its cell x + 1,
+// negated when the particle is clamped into a border cell (|offset| > 2
+// cells).
+__device__ __forceinline__ float4 cell_offset3(const KConst& k, const double4& p) {
+    const double pc[3] = {p.x, p.y, p.z};
+    const float far = 2.f * (float)k.cell_size;
+    float of[3];
+    bool is_far = false;
+    int cx = 0;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const int c = cell_coord(pc[a], k.cell_lo[a], k.cell_inv, k.cdims[a]);
+        if (a == 0) cx = c;
+        of[a] = (float)(pc[a] - cell_corner(k, a, c));
+        is_far |= !(fabsf(of[a]) <= far);
+    }
+    const float w = (float)(cx + 1);
+    return make_float4(of[0], of[1], of[2], is_far ? -w : w);
+}
+
 // Walks the candidates of a radius-h query: the 3^(D-1) x-rows of 3 cells
 // around the query cell, each one contiguous range of the cell-sorted set.
 // Positions are loaded 4 at a time so their latencies overlap; f(j, x_j)

@@ -273,8 +273,7 @@ int apply_viscosity(vps_context* c, double dt, double nu) {
                            c->rpos[s].p, c->cell_start.p, c->rvel[s].p, c->rrho.p, n, c->k,
                            scale, c->vel_next.p);
     VPS_HIP(c, hipGetLastError());
-    VPS_HIP(c, hipMemcpyAsync(c->rvel[s].p, c->vel_next.p, (size_t)n * sizeof(float4),
-                              hipMemcpyDeviceToDevice, c->stream));
+    std::swap(c->rvel[s], c->vel_next);   // every particle's velocity was written
     return VPS_OK;
 }
 
