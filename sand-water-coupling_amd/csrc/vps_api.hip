@@ -204,7 +204,7 @@ void free_all(vps_context* c) {
         dfree(c->brick_slot[b]);
         dfree(c->slot_brick[b]);
         dfree(c->nbr_slot);
-        dfree(c->col_run);
+        dfree(c->col_off);
         dfree(c->col_order);
         dfree(c->vx[b]);
         dfree(c->vp[b]);
@@ -467,7 +467,7 @@ int vps_create(const vps_params* params, vps_context** out) {
     ALLOC(c->vq, cap);
     ALLOC(c->vrank, cap);
     ALLOC(c->nbr_slot, (size_t)(c->nbricks + 1) * 27);
-    ALLOC(c->col_run, c->nbricks + 1);
+    ALLOC(c->col_off, (int64_t)k.bdims[0] * k.bdims[1]);
     ALLOC(c->col_order, c->nbricks + 1);
     ALLOC(c->bits, c->nwords + 1);
     ALLOC(c->word_prefix, c->nwords + 1);
@@ -728,15 +728,13 @@ static int project_impl(vps_context* c, vps_stats* st, int e0) {
     VPS_HIP(c, hipEventRecord(c->ev[e0], c->stream));
     VPS_TRY(virtual_diag(c, false));
     VPS_HIP(c, hipEventRecord(c->ev[e0 + 1], c->stream));
-    const int w = c->which;
-    float* x0 = c->vx[w].p;
     const int mode = c->p.warm_start;
     // the history of pressures (and the learned start) is kept only when
     // the network is used or trained
     if (mlp_active(c)) {
-        VPS_TRY(mlp_warm_start(c, mode, x0));
+        VPS_TRY(mlp_warm_start(c, mode));
     } else {
-        VPS_TRY(warm_start(c, mode, x0));
+        VPS_TRY(warm_start(c, mode));
     }
     vps_stats local{};
     vps_stats* s = st ? st : &local;
@@ -751,7 +749,7 @@ static int project_impl(vps_context* c, vps_stats* st, int e0) {
     int rc = cg_solve(c, s);
     if (rc == kStartRejected) {
         // the plain start: the reference's index-carried pressures
-        VPS_TRY(warm_start(c, VPS_WARM_INDEX_CARRY, x0));
+        VPS_TRY(warm_start(c, VPS_WARM_INDEX_CARRY));
         c->start_fallbacks++;
         c->start_guard = false;
         rc = cg_solve(c, s);
@@ -846,9 +844,9 @@ int vps_advance(vps_context* c, const vps_step_params* sp, vps_stats* st) {
     if (st) std::memset(st, 0, sizeof(*st));
     VPS_HIP(c, hipEventRecord(c->ev[0], c->stream));
     VPS_TRY(move_collide(c, sp->dt, sp->colliders, sp->n_colliders));
-    VPS_TRY(cells_sort_real(c));
+    // gravity rides on the sort (the densities do not read the velocities)
+    VPS_TRY(cells_sort_real(c, sp->enable_gravity ? (float)(sp->gravity * sp->dt) : 0.f));
     VPS_TRY(real_density(c, false));
-    if (sp->enable_gravity) VPS_TRY(apply_gravity(c, sp->dt, sp->gravity));
     VPS_TRY(apply_viscosity(c, sp->dt, sp->viscosity));
     VPS_HIP(c, hipEventRecord(c->ev[1], c->stream));
     VPS_TRY(virtual_generate(c));

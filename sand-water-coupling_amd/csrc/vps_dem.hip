@@ -85,20 +85,16 @@ __device__ __forceinline__ bool near_walls(const KConst& k, const int32_t* bcsta
     return found != 0;
 }
 
-// What the forces need of every (sorted) grain: its FP32 offset from its cell
-// corner (3D, as the density's offsets), and the grains next to a wall, listed
-// and flagged.  The list's order is arbitrary; a grain's sums are its own.
+// The (sorted) grains next to a wall, listed and flagged.  The list's order is
+// arbitrary; a grain's sums are its own.
 template <int D>
 __global__ void __launch_bounds__(256) k_dem_prepare(KConst k, int64_t n, const double4* pos,
-                                                     const int32_t* bcstart, float4* ofs,
-                                                     int32_t* near, int32_t* near_list,
+                                                     const int32_t* bcstart, int32_t* near, int32_t* near_list,
                                                      int32_t* near_count) {
     const int64_t i = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
     bool is_near = false;
     if (i < n) {
-        const double4 p = pos[i];
-        if constexpr (D == 3) ofs[i] = cell_offset3(k, p);
-        is_near = near_walls<D>(k, bcstart, p);
+        is_near = near_walls<D>(k, bcstart, pos[i]);
         near[i] = is_near ? 1 : 0;
     }
     // one atomic per block with any (one per wave, all on one address, bound
@@ -466,7 +462,7 @@ int dem_step(vps_context* c, double dt, double g, const vps_dem_params* dp) {
     const unsigned nlist = c->nb > 0 ? std::min(512u, (nb + 7) & ~7u) : 0;
     auto forces = [&](auto prepare, auto kern) {
         hipLaunchKernelGGL(prepare, dim3(nb), dim3(256), 0, c->stream, c->k, n, c->rpos[s].p, bcs,
-                           c->rofs.p, near, near_list, near_count);
+                           near, near_list, near_count);
         hipLaunchKernelGGL(kern, dim3(nlist + nb), dim3(256), 0, c->stream, c->k, dk, n,
                            (int)nlist, c->rpos[s].p, c->rofs.p, c->rvel[s].p, c->cell_start.p, bp,
                            c->bofs.p, c->bvel.p, c->bnrm.p, bcs, near, near_list, near_count,

@@ -189,21 +189,6 @@ constexpr int kGradThreads = 256;
 constexpr int kGradCap = 7168;   // staged nodes (28 KB: five blocks per CU)
 constexpr int kGradBoxBricks = 128;   // bricks a staged box may touch
 
-__global__ void __launch_bounds__(256) k_spans(KConst k, int span_cells, int nspan,
-                                               const int32_t* cstart, int4* chunks,
-                                               int32_t* count) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t nrows = (int64_t)k.cdims[1] * k.cdims[2];
-    if (i >= nrows * nspan) return;
-    const int64_t row = i / nspan;
-    const int sp = (int)(i - row * nspan);
-    const int64_t c0 = row * k.cdims[0] + (int64_t)sp * span_cells;
-    const int e = (sp + 1) * span_cells < k.cdims[0] ? (sp + 1) * span_cells : k.cdims[0];
-    const int64_t c1 = row * k.cdims[0] + e;
-    const int a = cstart[c0], b = cstart[c1];
-    if (b > a) chunks[atomicAdd(count, 1)] = make_int4(a, b, (int)c0, (int)c1);
-}
-
 __device__ __forceinline__ int node_floor(double x, double o, double inv) {
     double f = floor((x - o) * inv);
     f = f < -1.0e9 ? -1.0e9 : (f > 1.0e9 ? 1.0e9 : f);
@@ -554,14 +539,16 @@ int gradient_setup(vps_context* c) {
     return VPS_OK;
 }
 
-int gradient_spans(vps_context* c) {
-    if (c->grad_span_cells <= 0) return VPS_OK;
-    const int64_t total = (int64_t)c->k.cdims[1] * c->k.cdims[2] * c->grad_nspan;
-    hipLaunchKernelGGL(k_spans, dim3(blocks(total, 256)), dim3(256), 0, c->stream, c->k,
-                       c->grad_span_cells, c->grad_nspan, c->cell_start.p,
-                       c->grad_chunks.p, (int32_t*)(c->counters.p + 2));
-    VPS_HIP(c, hipGetLastError());
-    return VPS_OK;
+SpanArgs gradient_span_args(vps_context* c, bool append) {
+    SpanArgs a{};
+    if (!append || c->grad_span_cells <= 0) return a;
+    a.total = (int64_t)c->k.cdims[1] * c->k.cdims[2] * c->grad_nspan;
+    a.span_cells = c->grad_span_cells;
+    a.nspan = c->grad_nspan;
+    a.cstart = c->cell_start.p;
+    a.chunks = c->grad_chunks.p;
+    a.count = (int32_t*)(c->counters.p + 2);
+    return a;
 }
 
 // Terms of the staged gradient's virtual walk per real particle (test

@@ -280,6 +280,26 @@ __device__ __forceinline__ void for_each_candidate(const KConst& k,
         }
 }
 
+// Work units of the 3D gradient: spans of up to span_cells consecutive cells
+// of one cell row.  Thread i appends span i when it holds particles.
+struct SpanArgs {
+    int64_t total = 0;
+    int span_cells = 0, nspan = 0;
+    const int32_t* cstart = nullptr;
+    int4* chunks = nullptr;   // particle range, cell range
+    int32_t* count = nullptr;
+};
+__device__ __forceinline__ void span_append(const KConst& k, const SpanArgs& a, int64_t i) {
+    if (i >= a.total) return;
+    const int64_t row = i / a.nspan;
+    const int sp = (int)(i - row * a.nspan);
+    const int64_t c0 = row * k.cdims[0] + (int64_t)sp * a.span_cells;
+    const int e = (sp + 1) * a.span_cells < k.cdims[0] ? (sp + 1) * a.span_cells : k.cdims[0];
+    const int64_t c1 = row * k.cdims[0] + e;
+    const int b = a.cstart[c0], f = a.cstart[c1];
+    if (f > b) a.chunks[atomicAdd(a.count, 1)] = make_int4(b, f, (int)c0, (int)c1);
+}
+
 // ---- reductions ----------------------------------------------------------
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
@@ -482,10 +502,10 @@ struct vps_context {
     // slots of the 27 neighbour bricks of every slot of the current layout
     // (the zero brick nbricks where absent), built after each generation
     vps::DBuf<int32_t> nbr_slot;
-    // 3D slots in column order (every z-run of bricks bottom to top, runs in
-    // the order of their first slots) and the run lengths / offsets it is
-    // built from, after each generation
-    vps::DBuf<int32_t> col_run, col_order;
+    // 3D slots in column order (the active bricks of every (x, y) column bottom
+    // to top, column after column) and the columns' offsets it is built from,
+    // after each generation
+    vps::DBuf<int32_t> col_off, col_order;
     // per-node fields, slot-major
     vps::DBuf<float> vrho, vvol, vb, vdiag, vx[2], vr, vp[2], vt, vq, vrowsum;
     // 3D CG iteration: second r and t (ping-pong with vr, vt) and the
@@ -520,7 +540,8 @@ struct vps_context {
     // scratch
     vps::DBuf<double> partials;
     vps::DBuf<vps::CgState> cg;
-    vps::DBuf<uint32_t> scan_tmp;
+    vps::DBuf<uint64_t> scan_tmp;       // scan status words and ticket
+    uint32_t scan_epoch = 0;
     vps::DBuf<int64_t> counters;        // small device counters
     vps::CgState* host_cg = nullptr;    // pinned
     int64_t* host_counters = nullptr;   // pinned
@@ -576,13 +597,15 @@ void dfree(DBuf<T>& b) {
 // launchers (defined in the .hip files)
 // 3D gradient set-up at creation: span length and the span list buffer
 int gradient_setup(vps_context* c);
-// appends the non-empty cell spans of the current sort (count in counters[2])
-int gradient_spans(vps_context* c);
+// the spans of the current sort for span_append (total 0: none to append)
+SpanArgs gradient_span_args(vps_context* c, bool append);
 // exclusive scan of in into out (out may alias in); clear_in (== in, not
 // aliased with out) zeroes the input once read
 int scan_exclusive_i32(vps_context* c, const int32_t* in, int32_t* out,
                        int64_t n, int32_t* total_dev, int32_t* clear_in = nullptr);
-int cells_sort_real(vps_context* c);
+// sorts the real particles by cell (3D: with their cell offsets) and takes
+// v.y -= gdt on the way
+int cells_sort_real(vps_context* c, float gdt = 0.f);
 int cells_sort_boundary(vps_context* c);
 int upload_boundary_device(vps_context* c, int64_t n, const double* dx,
                            const double* dn, const double* dv);
@@ -607,16 +630,32 @@ int query_neighbors(vps_context* c, int which, int64_t nq, const double* q,
 int reduce_max_f32(vps_context* c, const float* in, int64_t n, double* out);
 int gather_virtual(vps_context* c, int64_t* node, double* rho, double* vol,
                    double* div, double* diag, double* pressure);
-int warm_start(vps_context* c, int mode, float* x0);
-// after_solve: the kernel (guarded) and, with an unguarded call, the host
-// bookkeeping; after_solve_commit: the bookkeeping alone
-int after_solve(vps_context* c, SolveGuard g = SolveGuard{});
+// where a warm start goes: x0 (read by the CG's first residual, in the scratch
+// vector vt) and the solution's two parts
+struct StartOut {
+    float* x0;
+    double* xb;
+    float* x;
+    __device__ __forceinline__ void put(int64_t g, float v) const {
+        x0[g] = v;
+        xb[g] = v;
+        x[g] = 0.f;
+    }
+};
+inline StartOut start_out(vps_context* c) {
+    return StartOut{c->vt.p, c->vxb.p, c->vx[c->which].p};
+}
+int warm_start(vps_context* c, int mode);
+// after_solve: the kernel (guarded; fold: the solution's parts first) and,
+// with an unguarded call, the host bookkeeping; after_solve_commit: the
+// bookkeeping alone
+int after_solve(vps_context* c, SolveGuard g = SolveGuard{}, bool fold = false);
 void after_solve_commit(vps_context* c);
 
 // learned warm start
 int mlp_create(vps_context* c);
 void mlp_destroy(vps_context* c);
-int mlp_warm_start(vps_context* c, int mode, float* x0);
+int mlp_warm_start(vps_context* c, int mode);
 int mlp_after_solve(vps_context* c, const vps_stats* st);
 bool mlp_active(const vps_context* c);
 // the rest of the SPH step (vps_sph.hip)

@@ -200,7 +200,7 @@ struct FeatSrc {
     const float* vvol;
     const float* scale;   // device scales (SC_*)
     float inv_a0, inv_vs;
-    float* corr;          // the network's correction c per node, or null
+    float* corr;          // output of the inference: the correction c per node
 };
 
 // Polynomial extrapolation of the node history (the prior of the network).
@@ -322,7 +322,7 @@ __device__ __forceinline__ void load_raw(const FeatSrc& s, int64_t tile, int64_t
 // Inference over the slot nodes with the next tile's loads in flight while
 // the current one runs through the network.
 __global__ void __launch_bounds__(256) k_mlp_infer_pipe(const float* P, FeatSrc fs,
-                                                        int64_t nn, float* out) {
+                                                        int64_t nn) {
     // the block reads the parameters once (coalesced) into LDS; each wave
     // builds its register tiles from there
     __shared__ float sP[kNParams];
@@ -360,15 +360,9 @@ __global__ void __launch_bounds__(256) k_mlp_infer_pipe(const float* P, FeatSrc 
                                     ok ? f[3] : 0.f);
             Fwd F;
             forward<false>(W, nullptr, xb, F);
-            // lanes 0..15 hold node r's output and (q = 0) its raw history
-            if (lane < 16 && cur.g < nn) {
-                out[cur.g] = ok ? cur.v[0] + prior(cur.h, cur.v[1], cur.v[2]) + tau * F.out
-                                : 0.f;
-                if (fs.corr) fs.corr[cur.g] = ok ? tau * F.out : 0.f;
-            }
+            if (lane < 16 && cur.g < nn) fs.corr[cur.g] = ok ? tau * F.out : 0.f;
         } else if (lane < 16 && cur.g < nn) {
-            out[cur.g] = 0.f;
-            if (fs.corr) fs.corr[cur.g] = 0.f;
+            fs.corr[cur.g] = 0.f;
         }
         cur = nxt;
     }
@@ -514,21 +508,21 @@ __global__ void __launch_bounds__(1024) k_galerkin_solve(const double* part, int
 
 __global__ void __launch_bounds__(256) k_galerkin_combine(int64_t nn, const float* P,
                                                           const float* E, const float* Cc,
-                                                          const double* y, float* x0) {
+                                                          const double* y, StartOut so) {
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (g >= nn) return;
     const float y0 = (float)y[0], y1 = (float)y[1], y2 = (float)y[2];
-    x0[g] = fmaf(y2, Cc[g], fmaf(y1, E[g], y0 * P[g]));
+    so.put(g, fmaf(y2, Cc[g], fmaf(y1, E[g], y0 * P[g])));
 }
 
 // x0 = p1 + e (the untrained network's answer, without the MLP).
 __global__ void __launch_bounds__(256) k_extrapolate(FeatSrc fs, int64_t nn,
-                                                     float* out) {
+                                                     StartOut so) {
     const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (g >= nn) return;
     const int h = fs.hh[g];
-    out[g] = fs.vvol[g] > 0.f && h >= 1 ? fs.p1[g] + prior(h, fs.dp1[g], fs.dp2[g])
-                                        : 0.f;
+    so.put(g, fs.vvol[g] > 0.f && h >= 1 ? fs.p1[g] + prior(h, fs.dp1[g], fs.dp2[g])
+                                         : 0.f);
 }
 
 __device__ __forceinline__ uint64_t mix64(uint64_t x) {
@@ -1106,7 +1100,7 @@ static FeatSrc feat_src(vps_context* c, int scale_buf) {
 
 // Gathers the node history into the current slot layout, then the warm
 // start of the chosen mode.
-int mlp_warm_start(vps_context* c, int mode, float* x0) {
+int mlp_warm_start(vps_context* c, int mode) {
     MlpState* m = S(c);
     VPS_TRY(ensure_history(c));
     const int w = c->which;
@@ -1115,7 +1109,7 @@ int mlp_warm_start(vps_context* c, int mode, float* x0) {
     const bool hist = m->have_history && lb >= 0;
     if (!hist) m->hist_solves = 0;
     m->step_scale = m->cur_scale;
-    if (nn == 0) return warm_start(c, mode, x0);
+    if (nn == 0) return warm_start(c, mode);
     hipLaunchKernelGGL(k_history_gather, dim3(blocks(nn, 256)), dim3(256), 0,
                        c->stream, nn, c->brick_nodes, c->slot_brick[w].p,
                        c->vvol.p, hist ? c->brick_slot[lb].p : nullptr,
@@ -1126,7 +1120,8 @@ int mlp_warm_start(vps_context* c, int mode, float* x0) {
     if (mode == VPS_WARM_LEARNED) {
         // The Galerkin start over [p1 e c], with the CG's scratch vectors:
         // inputs of M in vp[0], vp[1] and vr2 (their zero brick stays zero),
-        // products in vt, vt2 and vr.  The CG overwrites all of them.
+        // products in vt, vt2 and vr.  The start itself then goes to vt (see
+        // start_out); the CG overwrites the others.
         float* P = c->vp[0].p;
         float* E = c->vp[1].p;
         float* Cc = c->vr2.p;
@@ -1135,7 +1130,7 @@ int mlp_warm_start(vps_context* c, int mode, float* x0) {
         // about 8 tiles of 16 nodes per wave
         const int64_t nblk = std::min<int64_t>(std::max<int64_t>((nn + 511) / 512, 1), 8192);
         hipLaunchKernelGGL(k_mlp_infer_pipe, dim3((unsigned)nblk), dim3(256), 0,
-                           c->stream, m->P.p, fs, nn, x0);
+                           c->stream, m->P.p, fs, nn);
         hipLaunchKernelGGL(k_galerkin_fields, dim3(blocks(nn, 256)), dim3(256), 0, c->stream,
                            fs, nn, P, E);
         VPS_TRY(apply_operator_f32(c, P, c->vt.p, c->p.op_mode));
@@ -1148,12 +1143,12 @@ int mlp_warm_start(vps_context* c, int mode, float* x0) {
         hipLaunchKernelGGL(k_galerkin_solve, dim3(1), dim3(1024), 0, c->stream, m->gpart.p,
                            ng, m->gy.p);
         hipLaunchKernelGGL(k_galerkin_combine, dim3(nb), dim3(256), 0, c->stream, nn, P, E,
-                           Cc, m->gy.p, x0);
+                           Cc, m->gy.p, start_out(c));
     } else if (mode == VPS_WARM_EXTRAPOLATE) {
         hipLaunchKernelGGL(k_extrapolate, dim3(blocks(nn, 256)), dim3(256), 0,
-                           c->stream, feat_src(c, m->step_scale), nn, x0);
+                           c->stream, feat_src(c, m->step_scale), nn, start_out(c));
     } else {
-        return warm_start(c, mode, x0);
+        return warm_start(c, mode);
     }
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;

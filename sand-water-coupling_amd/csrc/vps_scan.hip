@@ -1,128 +1,29 @@
-// vps_scan.hip -- device-wide exclusive scan and max reduction.
-//
-// Used for the cell counting sort (cell_start), brick compaction (slots) and
-// the lattice-bitmask ranks.  Three passes: per-block totals, one-block scan
-// of the totals, per-block scan plus offset.  All integer, so the result is
-// exact and independent of scheduling.
-#include "vps_internal.h"
+// vps_scan.hip -- the int32 array scan, its workspace, and the max reduction.
+#include "vps_scan.h"
 
 namespace vps {
 namespace {
 
-constexpr int kScanBS = 256;
-constexpr int kScanIPT = 4;
-constexpr int kScanTile = kScanBS * kScanIPT;
-
-__device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
-    __shared__ int swave[kScanBS / 64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // inclusive wave scan
-    int x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) swave[wv] = x;
-    __syncthreads();
-    int off = 0, tot = 0;
-#pragma unroll
-    for (int i = 0; i < kScanBS / 64; i++) {
-        if (i < wv) off += swave[i];
-        tot += swave[i];
-    }
-    __syncthreads();
-    *total = tot;
-    return off + x - v;
-}
-
-__global__ void __launch_bounds__(kScanBS) k_tile_sums(const int32_t* in,
-                                                       int64_t n,
-                                                       int32_t* sums) {
-    const int64_t base = (int64_t)blockIdx.x * kScanTile;
-    int s = 0;
-#pragma unroll
-    for (int k = 0; k < kScanIPT; k++) {
-        const int64_t i = base + (int64_t)k * kScanBS + threadIdx.x;
-        if (i < n) s += in[i];
-    }
-    s = wave_sum(s);
-    __shared__ int sw[kScanBS / 64];
-    if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int i = 0; i < kScanBS / 64; i++) t += sw[i];
-        sums[blockIdx.x] = t;
-    }
-}
-
-// One block scans the tile totals in place; writes the grand total.
-__global__ void __launch_bounds__(1024) k_scan_sums(int32_t* sums, int nt,
-                                                     int32_t* total) {
-    __shared__ int sw[16];
-    const int per = (nt + 1023) / 1024;
-    const int b0 = threadIdx.x * per;
-    int local = 0;
-    for (int i = 0; i < per; i++)
-        if (b0 + i < nt) local += sums[b0 + i];
-    // block exclusive scan of 'local' over 1024 threads
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    int x = local;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) sw[wv] = x;
-    __syncthreads();
-    int off = 0, tot = 0;
-    for (int i = 0; i < 16; i++) {
-        if (i < wv) off += sw[i];
-        tot += sw[i];
-    }
-    int run = off + x - local;
-    for (int i = 0; i < per; i++)
-        if (b0 + i < nt) {
-            const int v = sums[b0 + i];
-            sums[b0 + i] = run;
-            run += v;
-        }
-    if (threadIdx.x == 0 && total) *total = tot;
-}
-
+struct LoadI32 {
+    static constexpr bool kWide = true;
+    const int32_t* in;
+    __device__ __forceinline__ int operator()(int64_t i) const { return in[i]; }
+    __device__ __forceinline__ int4 four(int64_t i) const { return *(const int4*)(in + i); }
+};
 // clear != nullptr (the input itself, not aliased with out): the input is
 // zeroed once read, ready for the next counting pass.
-__global__ void __launch_bounds__(kScanBS) k_tile_scan(const int32_t* in,
-                                                       int64_t n,
-                                                       const int32_t* sums,
-                                                       int32_t* out, int32_t* clear) {
-    const int64_t base = (int64_t)blockIdx.x * kScanTile;
-    // each thread owns kScanIPT consecutive elements
-    int v[kScanIPT];
-    int s = 0;
-#pragma unroll
-    for (int k = 0; k < kScanIPT; k++) {
-        const int64_t i = base + (int64_t)threadIdx.x * kScanIPT + k;
-        v[k] = i < n ? in[i] : 0;
-        s += v[k];
+struct StoreI32 {
+    static constexpr bool kWide = true;
+    int32_t *out, *clear;
+    __device__ __forceinline__ void four(int64_t i, int4 pre) const {
+        *(int4*)(out + i) = pre;
+        if (clear) *(int4*)(clear + i) = make_int4(0, 0, 0, 0);
     }
-    if (clear) {
-#pragma unroll
-        for (int k = 0; k < kScanIPT; k++) {
-            const int64_t i = base + (int64_t)threadIdx.x * kScanIPT + k;
-            if (i < n) clear[i] = 0;
-        }
+    __device__ __forceinline__ void operator()(int64_t i, int, int pre) const {
+        out[i] = pre;
+        if (clear) clear[i] = 0;
     }
-    int tot;
-    int run = block_exclusive_scan(s, &tot) + sums[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < kScanIPT; k++) {
-        const int64_t i = base + (int64_t)threadIdx.x * kScanIPT + k;
-        if (i < n) out[i] = run;
-        run += v[k];
-    }
-}
+};
 
 __global__ void __launch_bounds__(256) k_max_f32(const float* in, int64_t n,
                                                  double* partials,
@@ -160,23 +61,27 @@ __global__ void __launch_bounds__(256) k_max_f32(const float* in, int64_t n,
 
 }  // namespace
 
+int scan_workspace(vps_context* c, int64_t tiles, uint64_t** status, uint32_t** ticket,
+                   uint32_t* epoch) {
+    // the status words, then the ticket; zero words belong to no epoch
+    if (c->scan_tmp.n < (size_t)tiles + 1 || c->scan_epoch >= (1u << 30) - 1) {
+        VPS_TRY(dalloc(c, c->scan_tmp, (size_t)tiles + 1));
+        VPS_HIP(c, hipMemsetAsync(c->scan_tmp.p, 0, c->scan_tmp.n * sizeof(uint64_t), c->stream));
+        c->scan_epoch = 0;
+    }
+    *status = c->scan_tmp.p;
+    *ticket = (uint32_t*)(c->scan_tmp.p + c->scan_tmp.n - 1);
+    *epoch = ++c->scan_epoch;
+    return VPS_OK;
+}
+
 int scan_exclusive_i32(vps_context* c, const int32_t* in, int32_t* out,
                        int64_t n, int32_t* total_dev, int32_t* clear_in) {
     if (n <= 0) {
         if (total_dev) VPS_HIP(c, hipMemsetAsync(total_dev, 0, 4, c->stream));
         return VPS_OK;
     }
-    const int64_t nt = (n + kScanTile - 1) / kScanTile;
-    VPS_TRY(dalloc(c, c->scan_tmp, (size_t)nt));
-    int32_t* sums = (int32_t*)c->scan_tmp.p;
-    hipLaunchKernelGGL(k_tile_sums, dim3((unsigned)nt), dim3(kScanBS), 0,
-                       c->stream, in, n, sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, c->stream, sums,
-                       (int)nt, total_dev);
-    hipLaunchKernelGGL(k_tile_scan, dim3((unsigned)nt), dim3(kScanBS), 0,
-                       c->stream, in, n, sums, out, clear_in);
-    VPS_HIP(c, hipGetLastError());
-    return VPS_OK;
+    return scan_launch(c, LoadI32{in}, StoreI32{out, clear_in}, n, total_dev);
 }
 
 int reduce_max_f32(vps_context* c, const float* in, int64_t n, double* out) {

@@ -1020,21 +1020,17 @@ __global__ void __launch_bounds__(kUpdThreads) k_copy_rr(int64_t n4, const float
 // correction x that the iterations update.  A correction is small next to
 // the solution once the start is close, so its FP32 rounding stays far
 // below the tolerance even where ||b|| is small next to ||M|| ||x||.
-//   kFoldSplit  xb = x0, x = 0             (start of the solve)
+// (the start of a solve, xb = x0 and x = 0, is written by the warm start)
 //   kFoldMerge  xb += x, x = 0             (each residual replacement)
 //   kFoldFinal  x = (float)(xb + x)        (end of the solve: the pressures)
 //   kFoldZero   x = 0, xb = 0              (b = 0: Eigen's x = 0)
-enum FoldMode { kFoldSplit = 0, kFoldMerge = 1, kFoldFinal = 2, kFoldZero = 3 };
+enum FoldMode { kFoldMerge, kFoldFinal, kFoldZero };
 __global__ void __launch_bounds__(kUpdThreads) k_fold_x(int64_t n4, float4* x, double4* xb,
-                                                        int mode, SolveGuard guard) {
-    if (!solve_accepted(guard)) return;
+                                                        int mode) {
     for (int64_t i = (int64_t)blockIdx.x * kUpdThreads + threadIdx.x; i < n4;
          i += (int64_t)kUpdBlocks * kUpdThreads) {
         const float4 d = x[i];
-        if (mode == kFoldSplit) {
-            xb[i] = make_double4(d.x, d.y, d.z, d.w);
-            x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        } else if (mode == kFoldMerge) {
+        if (mode == kFoldMerge) {
             const double4 b = xb[i];
             xb[i] = make_double4(b.x + d.x, b.y + d.y, b.z + d.z, b.w + d.w);
             x[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1349,9 +1345,9 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     // x = xb (FP64) + x (FP32 correction) during the solve; every return
     // after the split leaves the pressures in x
     double* xb = c->vxb.p;
-    auto fold = [&](int mode, SolveGuard g = SolveGuard{}) {
+    auto fold = [&](int mode) {
         hipLaunchKernelGGL(k_fold_x, dim3(kUpdBlocks), dim3(kUpdThreads), 0, c->stream, n4,
-                           (float4*)x, (double4*)xb, mode, g);
+                           (float4*)x, (double4*)xb, mode);
     };
     // the post-solve work behind a batch, run only if the batch ends the
     // solve accepted (the state is read back before it, so the host learns
@@ -1360,8 +1356,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     c->spec_done = false;
     auto queue_post = [&]() -> int {
         const SolveGuard g{c->cg.p, c->check_true ? 2 : 1};
-        fold(kFoldFinal, g);
-        VPS_TRY(after_solve(c, g));
+        VPS_TRY(after_solve(c, g, true));
         VPS_HIP(c, hipEventRecord(c->ev[6], c->stream));
         VPS_TRY(pressure_gradient(c, g));
         return VPS_OK;
@@ -1378,12 +1373,11 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     float* tbuf[2] = {c->vt.p, c->vt2.p};
     {
         StencilArgs a = base_args(c);
-        a.in = x;
+        a.in = c->vt.p;   // x0 (start_out); tbuf[0] is free until launch 0
         a.out = rbuf[1];
         a.part0 = part_init(c, 0);
         a.part1 = part_init(c, 1);
         launch_op<K_CG_INIT, float, CoefF>(c, a, cf);
-        fold(kFoldSplit);
         // the recursion's threshold absorbs the FP32 drift measured at the
         // last solve (with a 10% margin); the FP64 check keeps tol
         double rec_scale = 1.0;

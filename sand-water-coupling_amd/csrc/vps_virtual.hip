@@ -21,7 +21,9 @@
 //   4. the reference order (x-fastest node rank) comes from a lattice bitmask
 //      and a popcount scan, so every node knows its index in the reference's
 //      virtual list without the list ever being materialised.
-#include "vps_internal.h"
+#include <algorithm>
+
+#include "vps_scan.h"
 
 namespace vps {
 namespace {
@@ -62,22 +64,25 @@ __global__ void __launch_bounds__(256) k_mark_bricks(const double4* pos,
                 flag[((int64_t)bz * k.bdims[1] + by) * k.bdims[0] + bx] = 1u;
 }
 
-__global__ void __launch_bounds__(256) k_assign_slots(uint32_t* flag,
-                                                      int64_t nbricks,
-                                                      int32_t* slot_of_brick,
-                                                      int32_t* brick_of_slot) {
-    const int64_t b = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (b >= nbricks) return;
-    // slot_of_brick holds the exclusive prefix of flag on entry; the flag is
-    // cleared for the next generation
-    const int s = slot_of_brick[b];
-    if (flag[b]) {
-        brick_of_slot[s] = (int32_t)b;
-        flag[b] = 0u;
-    } else {
-        slot_of_brick[b] = -1;
+// Brick compaction: the scan of the flags gives every flagged brick its slot
+// (ordered by brick id); the flags are cleared for the next generation.
+struct LoadFlag {
+    static constexpr bool kWide = false;
+    const uint32_t* flag;
+    __device__ __forceinline__ int operator()(int64_t b) const { return (int)flag[b]; }
+};
+struct AssignSlot {
+    static constexpr bool kWide = false;
+    uint32_t* flag;
+    int32_t *slot_of_brick, *brick_of_slot;
+    __device__ __forceinline__ void operator()(int64_t b, int flagged, int slot) const {
+        slot_of_brick[b] = flagged ? slot : -1;
+        if (flagged) {
+            brick_of_slot[slot] = (int32_t)b;
+            flag[b] = 0u;
+        }
     }
-}
+};
 
 // Real-neighbour sums of one node: w, sum W_H, sum V^2 W, sum V W (the v
 // denominator), sum v W / rho and the divergence terms.  dx = q - x_j.
@@ -612,16 +617,44 @@ __global__ void __launch_bounds__(512) k_virtual_sums3s(
                    vvol, vb, bits);
 }
 
-// Slots of the 3^D neighbour bricks of every slot (zero brick if absent).
+// Column order of the 3D slots, for the CG iteration's walk up z-runs of
+// bricks: the active bricks of every (x, y) column bottom to top, column after
+// column.  The scan of the columns' counts gives every column its place.
+struct LoadColumn {
+    static constexpr bool kWide = false;
+    int32_t plane, nz;   // columns, bricks of a column
+    const int32_t* slot_of_brick;
+    __device__ __forceinline__ int operator()(int64_t col) const {
+        int len = 0;
+#pragma unroll 8
+        for (int z = 0; z < nz; z++) len += slot_of_brick[col + (int64_t)z * plane] >= 0;
+        return len;
+    }
+};
+struct StoreColumn {
+    static constexpr bool kWide = false;
+    int32_t* off;
+    __device__ __forceinline__ void operator()(int64_t col, int, int pre) const {
+        off[col] = pre;
+    }
+};
+
+// Tables over the slots of one generation, in one launch: the slots of the
+// 3^D neighbour bricks of every slot (zero brick if absent), and in 3D the
+// column order, order[off[column] + active bricks below] = slot (by the thread
+// of the middle neighbour), and the gradient's spans (by the first threads;
+// see span_append).
 template <int D>
-__global__ void __launch_bounds__(256) k_nbr_slots(KConst k,
-                                                   const int32_t* brick_of_slot,
-                                                   const int32_t* slot_of_brick,
-                                                   const int32_t* nslots_p, int32_t zero,
-                                                   int32_t* nbr) {
+__global__ void __launch_bounds__(256) k_slot_tables(
+    KConst k, const int32_t* brick_of_slot, const int32_t* slot_of_brick, const int32_t* nslots_p,
+    int64_t grid, int32_t zero, int32_t* nbr, const int32_t* off, int32_t* order, SpanArgs sp) {
     constexpr int NN = D == 3 ? 27 : 9;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (int64_t)*nslots_p * NN) return;
+    if constexpr (D == 3) span_append(k, sp, i);
+    const int32_t nsl = *nslots_p;
+    // the grid may exceed the slot count; a count beyond the grid leaves the
+    // tables to the rerun on the exact grid
+    if (i >= (int64_t)nsl * NN || nsl > grid) return;
     const int64_t slot = i / NN;
     const int t = (int)(i - slot * NN);
     const int brick = brick_of_slot[slot];
@@ -637,53 +670,32 @@ __global__ void __launch_bounds__(256) k_nbr_slots(KConst k,
         if (sl >= 0) s = sl;
     }
     nbr[slot * 27 + t] = s;
+    if (D == 3 && t == 13) {
+        const int32_t plane = k.bdims[0] * k.bdims[1];
+        const int32_t col = brick - bz * plane;
+        int d = 0;
+#pragma unroll 8
+        for (int z = 0; z < bz; z++) d += slot_of_brick[col + (int64_t)z * plane] >= 0;
+        order[off[col] + d] = (int32_t)slot;
+    }
 }
 
-// Column order of the 3D slots, for the CG iteration's walk up z-runs of
-// bricks.  A run starts at a slot whose dz = -1 neighbour (index 4 of the
-// 27) is the zero brick and continues through the dz = +1 neighbours (index
-// 22); run[s] is the run's length at its first slot and 0 elsewhere.
-__global__ void __launch_bounds__(256) k_col_runs(const int32_t* nbr, const int32_t* nslots_p,
-                                                  int64_t grid, int32_t zero, int32_t* run) {
-    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (s >= grid) return;
-    // the grid may exceed the slot count; a count beyond the grid (the
-    // neighbour table is then incomplete) leaves the order to the rerun on
-    // the exact grid
-    const int32_t nsl = *nslots_p;
-    if (s >= nsl || nsl > grid) {
-        run[s] = 0;
-        return;
+// Words of the lattice bitmask before each word, for the node ranks.
+struct LoadPopc {
+    static constexpr bool kWide = true;
+    __device__ __forceinline__ int4 four(int64_t i) const {
+        const uint4 w = *(const uint4*)(bits + i);
+        return make_int4(__popc(w.x), __popc(w.y), __popc(w.z), __popc(w.w));
     }
-    int32_t len = 0;
-    if (nbr[s * 27 + 4] == zero) {
-        int32_t b = (int32_t)s;
-        len = 1;
-        while ((b = nbr[(int64_t)b * 27 + 22]) != zero) len++;
-    }
-    run[s] = len;
-}
-
-// order[off[first slot of the run] + height in the run] = slot
-__global__ void __launch_bounds__(256) k_col_place(const int32_t* nbr, const int32_t* nslots_p,
-                                                   int64_t grid, int32_t zero,
-                                                   const int32_t* off, int32_t* order) {
-    const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int32_t nsl = *nslots_p;
-    if (s >= nsl || nsl > grid) return;
-    int32_t b = (int32_t)s, d = 0, n;
-    while ((n = nbr[(int64_t)b * 27 + 4]) != zero) {
-        b = n;
-        d++;
-    }
-    order[off[b] + d] = (int32_t)s;
-}
-
-__global__ void __launch_bounds__(256) k_popc(const uint32_t* bits,
-                                              int64_t nwords, int32_t* cnt) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < nwords) cnt[i] = __popc(bits[i]);
-}
+    const uint32_t* bits;
+    __device__ __forceinline__ int operator()(int64_t i) const { return __popc(bits[i]); }
+};
+struct StorePrefix {
+    static constexpr bool kWide = true;
+    __device__ __forceinline__ void four(int64_t i, int4 pre) const { *(int4*)(prefix + i) = pre; }
+    int32_t* prefix;
+    __device__ __forceinline__ void operator()(int64_t i, int, int pre) const { prefix[i] = pre; }
+};
 
 template <int D, int NB>
 __global__ void __launch_bounds__(NB) k_node_rank(KConst k,
@@ -713,12 +725,14 @@ __global__ void __launch_bounds__(NB) k_node_rank(KConst k,
     rank[out] = prefix[lin >> 5] + __popc(below);
 }
 
-// CG initial guess for every node of the active bricks (0 off the set).
+// CG initial guess for every node of the active bricks (0 off the set): x0
+// for the residual, and the solution in its two parts (base x0, correction
+// 0; see k_fold_x in vps_stencil.hip).
 template <int D, int NB>
 __global__ void __launch_bounds__(NB) k_warm_start(
     int mode, KConst k, const int32_t* brick_of_slot, const float* vvol,
     const int32_t* rank, const float* p_rank_prev, int64_t nprev,
-    const int32_t* prev_slot_of_brick, const float* x_prev, float* x0) {
+    const int32_t* prev_slot_of_brick, const float* x_prev, StartOut so) {
     const int slot = blockIdx.x;
     const int64_t out = (int64_t)slot * NB + threadIdx.x;
     float v = 0.f;
@@ -733,21 +747,26 @@ __global__ void __launch_bounds__(NB) k_warm_start(
             }
         }
     }
-    x0[out] = v;
+    so.put(out, v);
 }
 
 // After the solve: pressures by reference rank (index-carry warm start of
-// the next step) and q = V p for the pressure gradient.
+// the next step) and q = V p for the pressure gradient.  With xb, the
+// solution's two parts are folded into the pressures on the way.
 __global__ void __launch_bounds__(256) k_after_solve(int64_t nnode,
                                                      const float* vvol,
-                                                     const float* x,
+                                                     float* x, const double* xb,
                                                      const int32_t* rank,
                                                      float* p_rank, float* q,
                                                      SolveGuard guard) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= nnode || !solve_accepted(guard)) return;
     const float V = vvol[i];
-    const float p = x[i];
+    float p = x[i];
+    if (xb) {
+        p = (float)(xb[i] + p);
+        x[i] = p;
+    }
     q[i] = V * p;
     if (V > 0.f) p_rank[rank[i]] = p;
 }
@@ -755,8 +774,9 @@ __global__ void __launch_bounds__(256) k_after_solve(int64_t nnode,
 }  // namespace
 
 // Slot-indexed passes of one generation on a grid of `grid` blocks (slots);
-// blocks at or beyond the device-side slot count return at once.
-static int generate_slots(vps_context* c, int w, int64_t grid) {
+// blocks at or beyond the device-side slot count return at once.  first: not a
+// rerun on the exact grid (the gradient's spans are appended once).
+static int generate_slots(vps_context* c, int w, int64_t grid, bool first) {
     const int D = c->dim;
     const int rs = c->cur;
     const int32_t* nsl = (const int32_t*)c->counters.p;   // slot count
@@ -775,28 +795,25 @@ static int generate_slots(vps_context* c, int w, int64_t grid) {
                            c->cell_start.p, c->bpos.p, c->bvel.p, c->bnrm.p,
                            c->bcell_start.p, c->vrho.p, c->vvol.p, c->vb.p,
                            c->bits.p);
+    // the column order and the tables, on the grid (before the read-back
+    // below, so that they run while the host waits)
+    const int32_t* bos = c->slot_brick[w].p;
+    const int32_t* sob = c->brick_slot[w].p;
     if (D == 3) {
-        hipLaunchKernelGGL(k_nbr_slots<3>, dim3(blocks(grid * 27, 256)), dim3(256),
-                           0, c->stream, c->k, c->slot_brick[w].p, c->brick_slot[w].p,
-                           nsl, (int32_t)c->nbricks, c->nbr_slot.p);
-        // the column order, on the grid (before the read-back below, so
-        // that it runs while the host waits)
-        hipLaunchKernelGGL(k_col_runs, dim3(blocks(grid, 256)), dim3(256), 0, c->stream,
-                           c->nbr_slot.p, nsl, grid, (int32_t)c->nbricks, c->col_run.p);
-        VPS_TRY(scan_exclusive_i32(c, c->col_run.p, c->col_run.p, grid, nullptr));
-        hipLaunchKernelGGL(k_col_place, dim3(blocks(grid, 256)), dim3(256), 0, c->stream,
-                           c->nbr_slot.p, nsl, grid, (int32_t)c->nbricks, c->col_run.p,
-                           c->col_order.p);
+        const int32_t plane = c->k.bdims[0] * c->k.bdims[1];
+        // (one column per thread: each is a loop of its own)
+        VPS_TRY(scan_launch_as<1>(c, LoadColumn{plane, c->k.bdims[2], sob},
+                                  StoreColumn{c->col_off.p}, plane, nullptr));
+        const SpanArgs sp = gradient_span_args(c, first);
+        hipLaunchKernelGGL(k_slot_tables<3>, dim3(blocks(std::max(grid * 27, sp.total), 256)),
+                           dim3(256), 0, c->stream, c->k, bos, sob, nsl, grid,
+                           (int32_t)c->nbricks, c->nbr_slot.p, c->col_off.p, c->col_order.p, sp);
     } else
-        hipLaunchKernelGGL(k_nbr_slots<2>, dim3(blocks(grid * 9, 256)), dim3(256),
-                           0, c->stream, c->k, c->slot_brick[w].p, c->brick_slot[w].p,
-                           nsl, (int32_t)c->nbricks, c->nbr_slot.p);
-    hipLaunchKernelGGL(k_popc, dim3(blocks(c->nwords, 256)), dim3(256), 0,
-                       c->stream, c->bits.p, c->nwords,
-                       (int32_t*)c->word_prefix.p);
-    VPS_TRY(scan_exclusive_i32(c, (const int32_t*)c->word_prefix.p,
-                               (int32_t*)c->word_prefix.p, c->nwords,
-                               (int32_t*)(dcnt + 1)));
+        hipLaunchKernelGGL(k_slot_tables<2>, dim3(blocks(grid * 9, 256)), dim3(256), 0, c->stream,
+                           c->k, bos, sob, nsl, grid, (int32_t)c->nbricks, c->nbr_slot.p,
+                           (const int32_t*)nullptr, (int32_t*)nullptr, SpanArgs{});
+    VPS_TRY(scan_launch(c, LoadPopc{c->bits.p}, StorePrefix{(int32_t*)c->word_prefix.p}, c->nwords,
+                        (int32_t*)(dcnt + 1)));
     if (D == 3)
         hipLaunchKernelGGL((k_node_rank<3, 512>), dim3((unsigned)grid),
                            dim3(512), 0, c->stream, c->k, c->slot_brick[w].p,
@@ -838,14 +855,10 @@ int virtual_generate(vps_context* c) {
                            0, c->stream, c->rpos[s].p, c->n, c->k,
                            c->brick_flag.p, c->bits.p, c->nwords,
                            (int32_t*)(c->counters.p + 2));
-    VPS_TRY(gradient_spans(c));
     int64_t* dcnt = c->counters.p;
-    VPS_TRY(scan_exclusive_i32(c, (const int32_t*)c->brick_flag.p,
-                               c->brick_slot[w].p, c->nbricks,
-                               (int32_t*)dcnt));
-    hipLaunchKernelGGL(k_assign_slots, dim3(blocks(c->nbricks, 256)), dim3(256),
-                       0, c->stream, c->brick_flag.p, c->nbricks,
-                       c->brick_slot[w].p, c->slot_brick[w].p);
+    VPS_TRY(scan_launch(c, LoadFlag{c->brick_flag.p},
+                        AssignSlot{c->brick_flag.p, c->brick_slot[w].p, c->slot_brick[w].p},
+                        c->nbricks, (int32_t*)dcnt));
     // The slot count stays on the device: the slot passes run on a grid
     // sized from the last generation's count (all bricks the first time),
     // and again on the exact grid in the rare step where it grew past that.
@@ -854,12 +867,12 @@ int virtual_generate(vps_context* c) {
         grid = c->nslots + c->nslots / 8 + 64;
         if (grid > c->nbricks) grid = c->nbricks;
     }
-    VPS_TRY(generate_slots(c, w, grid));
+    VPS_TRY(generate_slots(c, w, grid, true));
     int64_t nslots = *(int32_t*)c->host_counters;
     if (nslots > grid) {
         hipLaunchKernelGGL(k_fill_u32, dim3(blocks(c->nwords, 256)), dim3(256), 0,
                            c->stream, c->bits.p, c->nwords, 0u);
-        VPS_TRY(generate_slots(c, w, nslots));
+        VPS_TRY(generate_slots(c, w, nslots, false));
         nslots = *(int32_t*)c->host_counters;
     }
     c->nslots = nslots;
@@ -869,7 +882,7 @@ int virtual_generate(vps_context* c) {
     return VPS_OK;
 }
 
-int warm_start(vps_context* c, int mode, float* x0) {
+int warm_start(vps_context* c, int mode) {
     const int w = c->which;
     const int lb = c->last_solve_buf;
     const int32_t* prev_map = lb >= 0 ? c->brick_slot[lb].p : nullptr;
@@ -880,22 +893,22 @@ int warm_start(vps_context* c, int mode, float* x0) {
         hipLaunchKernelGGL((k_warm_start<3, 512>), dim3((unsigned)c->nslots),
                            dim3(512), 0, c->stream, mode, c->k,
                            c->slot_brick[w].p, c->vvol.p, c->vrank.p, p_prev,
-                           nprev, prev_map, x_prev, x0);
+                           nprev, prev_map, x_prev, start_out(c));
     else
         hipLaunchKernelGGL((k_warm_start<2, 64>), dim3((unsigned)c->nslots),
                            dim3(64), 0, c->stream, mode, c->k,
                            c->slot_brick[w].p, c->vvol.p, c->vrank.p, p_prev,
-                           nprev, prev_map, x_prev, x0);
+                           nprev, prev_map, x_prev, start_out(c));
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;
 }
 
-int after_solve(vps_context* c, SolveGuard g) {
+int after_solve(vps_context* c, SolveGuard g, bool fold) {
     const int w = c->which;
     const int64_t nn = c->nslots * c->brick_nodes;
     if (nn == 0) return VPS_OK;
     hipLaunchKernelGGL(k_after_solve, dim3(blocks(nn, 256)), dim3(256), 0,
-                       c->stream, nn, c->vvol.p, c->vx[w].p, c->vrank.p,
+                       c->stream, nn, c->vvol.p, c->vx[w].p, fold ? c->vxb.p : nullptr, c->vrank.p,
                        c->p_by_rank[w].p, c->vq.p, g);
     VPS_HIP(c, hipGetLastError());
     if (g.mode == 0) after_solve_commit(c);
