@@ -11,7 +11,7 @@ from vps import Projection, VpsError, scenes, _abi
 
 pytestmark = pytest.mark.gpu
 
-PIECE = 2 << 20   # bytes
+PIECE = 512 << 10   # bytes
 
 
 def grains(dim, n, seed=3):
