@@ -139,23 +139,26 @@ __global__ void __launch_bounds__(256) k_density(const double4* pos,
 // offsets fit, so the loads take a scalar base and a 32-bit lane offset).
 // CNT (test support): only the number of terms that enter the sum (a > 0: r < h,
 // where the spline is nonzero) into members[i].
-template <bool BND, typename Off, bool CNT = false>
+// L: lanes of a wave that share a particle, each taking every L-th candidate
+// of a row; their sums meet in a butterfly.  One lane per particle is the
+// least work; with few particles the machine is not full, and the time is that
+// of one particle's chain of about 216 candidates (see walk_lanes).
+template <bool BND, typename Off, int L, bool CNT = false>
 __global__ void __launch_bounds__(256) k_density3f(const double4* pos, const float4* ofs,
                                                    const int32_t* cstart, int64_t n,
                                                    KConst k, float* rho, float* rinv,
                                                    float4* nrm, float4* vel, int set_volume,
                                                    int32_t* members = nullptr) {
-    const int nb = (int)((n + 255) / 256);
-    const int64_t i = (int64_t)xcd_remap(blockIdx.x, nb) * 256 + threadIdx.x;
-    if (i >= n) return;
+    const int64_t tid = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    const int64_t i = tid / L;
+    const int sub = L > 1 ? (int)(tid % L) : 0;
+    if (i >= n) return;   // uniform over the lanes of a particle
     const double4 q = pos[i];
     const int cc0 = cell_coord(q.x, k.cell_lo[0], k.cell_inv, k.cdims[0]);
     const int cc1 = cell_coord(q.y, k.cell_lo[1], k.cell_inv, k.cdims[1]);
     const int cc2 = cell_coord(q.z, k.cell_lo[2], k.cell_inv, k.cdims[2]);
     const int x0 = cc0 > 0 ? cc0 - 1 : 0;
     const int x1 = cc0 + 1 < k.cdims[0] ? cc0 + 1 : k.cdims[0] - 1;
-    const int zlo = cc2 > 0 ? cc2 - 1 : 0, zhi = cc2 + 1 < k.cdims[2] ? cc2 + 1 : k.cdims[2] - 1;
-    const int ylo = cc1 > 0 ? cc1 - 1 : 0, yhi = cc1 + 1 < k.cdims[1] ? cc1 + 1 : k.cdims[1] - 1;
     // q - C_x0, rounded once from FP64 (the staged x_j - C_j complete
     // q - x_j).  A candidate in cell x0 + d (d = 0, 1, 2; the offset's w is
     // its cell x + 1) takes q - C_x0 - d cells, formed by one fma: exact
@@ -179,19 +182,14 @@ __global__ void __launch_bounds__(256) k_density3f(const double4* pos, const flo
     const float ih = k.inv_h, ih2 = 2.f * k.inv_h;
     float suma = 0.f, sumc = 0.f;
     int32_t nterms = 0;
-    for (int z = zlo; z <= zhi; z++) {
-        const float tz = (float)(q.z - cell_corner(k, 2, z));
-        for (int y = ylo; y <= yhi; y++) {
-            const float ty = (float)(q.y - cell_corner(k, 1, y));
-            const int64_t row = ((int64_t)z * k.cdims[1] + y) * k.cdims[0];
-            const int b = cstart[row + x0], e = cstart[row + x1 + 1];
-            for (int j = b; j < e; j++) {
+    for_each_row<L>(k, cstart, q, cc1, cc2, x0, x1, [&](float ty, float tz, int b, int e) {
+            for (int j = b + sub; j < e; j += L) {
                 const Off o = (Off)j * 16u;
                 const float4 p = *(const float4*)((const char*)ofs + o);
                 const float tx = fmaf(x0w - p.w, csf, tx0);
                 const float dx = tx - p.x, dy = ty - p.y, dz = tz - p.z;
                 float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                if (p.w < 0.f || qfar) {   // rare: FP64 distance
+                if ((p.w < 0.f) | qfar) {   // rare: FP64 distance
                     const double4 pj = *(const double4*)((const char*)pos + (uint64_t)o * 2u);
                     d2 = (float)sq_dist3(pj.x, pj.y, pj.z, q.x, q.y, q.z);
                 }
@@ -205,12 +203,17 @@ __global__ void __launch_bounds__(256) k_density3f(const double4* pos, const flo
                 sumc = fmaf(c * c, c, sumc);
                 if constexpr (CNT) nterms += a > 0.f;
             }
-        }
-    }
+    });
     if constexpr (CNT) {
         members[i] = nterms;
         return;
     }
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) {
+        suma += __shfl_xor(suma, o, 64);
+        sumc += __shfl_xor(sumc, o, 64);
+    }
+    if (sub != 0) return;
     const float r = k.mass * k.c0h * fmaf(2.f, suma, -sumc);
     if constexpr (BND) {
         nrm[i].w = r;
@@ -350,16 +353,18 @@ int real_density(vps_context* c, bool set_volume) {
     const int64_t n = c->n;
     const int s = c->cur;
     if (c->dim == 3) {
-        if (n * 16 <= (int64_t)UINT32_MAX)
-            hipLaunchKernelGGL((k_density3f<false, uint32_t>), dim3(blocks(n, 256)), dim3(256),
-                               0, c->stream, c->rpos[s].p, c->rofs.p, c->cell_start.p, n,
-                               c->k, c->rrho.p, c->rrinv.p, (float4*)nullptr, c->rvel[s].p,
-                               set_volume ? 1 : 0);
-        else
-            hipLaunchKernelGGL((k_density3f<false, uint64_t>), dim3(blocks(n, 256)), dim3(256),
-                               0, c->stream, c->rpos[s].p, c->rofs.p, c->cell_start.p, n,
-                               c->k, c->rrho.p, c->rrinv.p, (float4*)nullptr, c->rvel[s].p,
-                               set_volume ? 1 : 0);
+        auto run = [&](auto kern, int lanes) {
+            hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
+                               c->rpos[s].p, c->rofs.p, c->cell_start.p, n, c->k, c->rrho.p,
+                               c->rrinv.p, (float4*)nullptr, c->rvel[s].p, set_volume ? 1 : 0,
+                               (int32_t*)nullptr);
+        };
+        const int lanes = walk_lanes(n);
+        if (lanes == 8) run(k_density3f<false, uint32_t, 8>, 8);
+        else if (lanes == 4) run(k_density3f<false, uint32_t, 4>, 4);
+        else if (lanes == 2) run(k_density3f<false, uint32_t, 2>, 2);
+        else if (n * 16 <= (int64_t)UINT32_MAX) run(k_density3f<false, uint32_t, 1>, 1);
+        else run(k_density3f<false, uint64_t, 1>, 1);
     } else
         hipLaunchKernelGGL(k_density<2>, dim3(blocks(n, 256)), dim3(256), 0,
                            c->stream, c->rpos[s].p, c->cell_start.p, n, c->k,
@@ -388,7 +393,7 @@ int density_member_counts(vps_context* c, int which, int32_t* members) {
         const int s = c->cur;
         hipLaunchKernelGGL(k_cell_offsets3, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
                            c->rpos[s].p, n, c->k, c->rofs.p);
-        hipLaunchKernelGGL((k_density3f<false, uint64_t, true>), dim3(blocks(n, 256)),
+        hipLaunchKernelGGL((k_density3f<false, uint64_t, 1, true>), dim3(blocks(n, 256)),
                            dim3(256), 0, c->stream, c->rpos[s].p, c->rofs.p, c->cell_start.p,
                            n, c->k, (float*)nullptr, (float*)nullptr, (float4*)nullptr,
                            (float4*)nullptr, 0, members);
@@ -397,7 +402,7 @@ int density_member_counts(vps_context* c, int which, int32_t* members) {
         VPS_TRY(dalloc(c, ofs, (size_t)n));
         hipLaunchKernelGGL(k_cell_offsets3, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
                            c->bpos.p, n, c->k, ofs.p);
-        hipLaunchKernelGGL((k_density3f<true, uint64_t, true>), dim3(blocks(n, 256)),
+        hipLaunchKernelGGL((k_density3f<true, uint64_t, 1, true>), dim3(blocks(n, 256)),
                            dim3(256), 0, c->stream, c->bpos.p, ofs.p, c->bcell_start.p, n,
                            c->k, (float*)nullptr, (float*)nullptr, (float4*)nullptr,
                            (float4*)nullptr, 0, members);
@@ -416,11 +421,11 @@ int boundary_density(vps_context* c) {
         // the density walk as for the real particles, on the sort's offsets,
         // then the offsets with w = +-1 / rho_b for the virtual sums
         if (nb * 16 <= (int64_t)UINT32_MAX)
-            hipLaunchKernelGGL((k_density3f<true, uint32_t>), dim3(blocks(nb, 256)), dim3(256),
+            hipLaunchKernelGGL((k_density3f<true, uint32_t, 1>), dim3(blocks(nb, 256)), dim3(256),
                                0, c->stream, c->bpos.p, c->bofs.p, c->bcell_start.p, nb, c->k,
                                (float*)nullptr, (float*)nullptr, c->bnrm.p, c->bvel.p, 0);
         else
-            hipLaunchKernelGGL((k_density3f<true, uint64_t>), dim3(blocks(nb, 256)), dim3(256),
+            hipLaunchKernelGGL((k_density3f<true, uint64_t, 1>), dim3(blocks(nb, 256)), dim3(256),
                                0, c->stream, c->bpos.p, c->bofs.p, c->bcell_start.p, nb, c->k,
                                (float*)nullptr, (float*)nullptr, c->bnrm.p, c->bvel.p, 0);
         hipLaunchKernelGGL(k_boundary_offsets3, dim3(blocks(nb, 256)), dim3(256), 0,

@@ -280,6 +280,56 @@ __device__ __forceinline__ void for_each_candidate(const KConst& k,
         }
 }
 
+// The 3 x 3 x-rows of cells around cell (., cy, cz), each one candidate range
+// of the cells x0 .. x1: f(ty, tz, begin, end) with ty, tz = q - C of the row's
+// cells, rounded once from FP64.  With several lanes per particle
+// (L > 1: one particle's chain is what counts) the bounds of all nine are
+// loaded at once; with one lane each row loads its own when its turn comes
+// (fewer registers, and the other waves cover the wait).
+template <int L, typename F>
+__device__ __forceinline__ void for_each_row(const KConst& k, const int32_t* cstart,
+                                             const double4& q, int cy, int cz, int x0, int x1,
+                                             F&& f) {
+    if constexpr (L == 1) {
+        const int zlo = cz > 0 ? cz - 1 : 0, zhi = cz + 1 < k.cdims[2] ? cz + 1 : k.cdims[2] - 1;
+        const int ylo = cy > 0 ? cy - 1 : 0, yhi = cy + 1 < k.cdims[1] ? cy + 1 : k.cdims[1] - 1;
+        for (int z = zlo; z <= zhi; z++) {
+            const float tz = (float)(q.z - cell_corner(k, 2, z));
+            for (int y = ylo; y <= yhi; y++) {
+                const float ty = (float)(q.y - cell_corner(k, 1, y));
+                const int64_t row = ((int64_t)z * k.cdims[1] + y) * k.cdims[0];
+                f(ty, tz, cstart[row + x0], cstart[row + x1 + 1]);
+            }
+        }
+    } else {
+        int b[9], e[9];
+#pragma unroll
+        for (int r = 0; r < 9; r++) {
+            const int y = min(max(cy + r % 3 - 1, 0), k.cdims[1] - 1);
+            const int z = min(max(cz + r / 3 - 1, 0), k.cdims[2] - 1);
+            const int64_t row = ((int64_t)z * k.cdims[1] + y) * k.cdims[0];
+            b[r] = cstart[row + x0];
+            e[r] = cstart[row + x1 + 1];
+        }
+#pragma unroll
+        for (int r = 0; r < 9; r++) {
+            const int y = cy + r % 3 - 1, z = cz + r / 3 - 1;
+            if (y < 0 || z < 0 || y >= k.cdims[1] || z >= k.cdims[2]) continue;
+            f((float)(q.y - cell_corner(k, 1, y)), (float)(q.z - cell_corner(k, 2, z)), b[r], e[r]);
+        }
+    }
+}
+
+// Lanes per particle of the 3D candidate walks (density, viscosity): the
+// fewest that fill the machine.  us of the density with 1, 2, 4, 8 lanes:
+//   576 particles 35, 21, 16, 10     64,800 (the viscosity)  42, 25, 18, 17
+//   212,503       45, 35, 35, 41                            (77, 46, 33, 38)
+//   300,000       53, 53, 52, 59     600,000  96, 84, 90, 107
+//   1,012,500    131, 131, 142, 172
+inline int walk_lanes(int64_t n) {
+    return n <= 32000 ? 8 : (n <= 400000 ? 4 : (n <= 900000 ? 2 : 1));
+}
+
 // Work units of the 3D gradient: spans of up to span_cells consecutive cells
 // of one cell row.  Thread i appends span i when it holds particles.
 struct SpanArgs {

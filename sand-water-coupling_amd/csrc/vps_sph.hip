@@ -102,16 +102,18 @@ struct ViscAcc {
 
 // 3D from the FP32 cell-corner offsets (as the density): W' is zero at h,
 // so the FP32 distance decides which terms enter.  CNT (test support): only
-// the number of terms into members[i].
-template <bool CNT = false>
+// the number of terms into members[i].  L: lanes that share a particle (see
+// k_density3f).
+template <int L, bool CNT = false>
 __global__ void __launch_bounds__(256) k_viscosity3f(const double4* pos, const float4* ofs,
                                                      const int32_t* cstart, const float4* vel,
                                                      const float* rho, int64_t n, KConst k,
                                                      float scale, float4* vout,
                                                      int32_t* members = nullptr) {
-    const int nb = (int)((n + 255) / 256);
-    const int64_t i = (int64_t)xcd_remap(blockIdx.x, nb) * 256 + threadIdx.x;
-    if (i >= n) return;
+    const int64_t tid = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    const int64_t i = tid / L;
+    const int sub = L > 1 ? (int)(tid % L) : 0;
+    if (i >= n) return;   // uniform over the lanes of a particle
     const double4 q = pos[i];
     const float4 vi = vel[i];
     const int cc0 = cell_coord(q.x, k.cell_lo[0], k.cell_inv, k.cdims[0]);
@@ -119,12 +121,13 @@ __global__ void __launch_bounds__(256) k_viscosity3f(const double4* pos, const f
     const int cc2 = cell_coord(q.z, k.cell_lo[2], k.cell_inv, k.cdims[2]);
     const int x0 = cc0 > 0 ? cc0 - 1 : 0;
     const int x1 = cc0 + 1 < k.cdims[0] ? cc0 + 1 : k.cdims[0] - 1;
-    const int zlo = cc2 > 0 ? cc2 - 1 : 0, zhi = cc2 + 1 < k.cdims[2] ? cc2 + 1 : k.cdims[2] - 1;
-    const int ylo = cc1 > 0 ? cc1 - 1 : 0, yhi = cc1 + 1 < k.cdims[1] ? cc1 + 1 : k.cdims[1] - 1;
-    // q - C_c per candidate cell, rounded once from FP64
+    // q - C_c per candidate cell, each rounded once from FP64 (a coincident
+    // particle's difference is exactly zero); the cell of a candidate is in
+    // its offset's w (cell x + 1)
     const float tx0 = (float)(q.x - cell_corner(k, 0, x0));
     const float tx1 = (float)(q.x - cell_corner(k, 0, x0 + 1));
     const float tx2 = (float)(q.x - cell_corner(k, 0, x0 + 2));
+    const float w0 = (float)(x0 + 1), w1 = (float)(x0 + 2);
     const float far = 2.f * (float)k.cell_size;
     const float qo0 = (float)(q.x - cell_corner(k, 0, cc0));
     const float qo1 = (float)(q.y - cell_corner(k, 1, cc1));
@@ -133,42 +136,40 @@ __global__ void __launch_bounds__(256) k_viscosity3f(const double4* pos, const f
     const float h2 = (float)k.h2;
     ViscAcc acc;
     int32_t nterms = 0;
-    for (int z = zlo; z <= zhi; z++) {
-        const float tz = (float)(q.z - cell_corner(k, 2, z));
-        for (int y = ylo; y <= yhi; y++) {
-            const float ty = (float)(q.y - cell_corner(k, 1, y));
-            const int64_t row = ((int64_t)z * k.cdims[1] + y) * k.cdims[0];
-            const int b = cstart[row + x0], e = cstart[row + x1 + 1];
-            const int b1 = x0 + 1 <= x1 ? cstart[row + x0 + 1] : e;
-            const int b2 = x0 + 2 <= x1 ? cstart[row + x0 + 2] : e;
-            for (int j = b; j < e; j++) {
-                const float4 p = ofs[j];
-                const float tx = j < b1 ? tx0 : (j < b2 ? tx1 : tx2);
-                float dx, dy, dz;   // x_j - x_i
-                if (p.w >= 0.f && !qfar) {
-                    dx = p.x - tx;
-                    dy = p.y - ty;
-                    dz = p.z - tz;
-                } else {
-                    const double4 pj = pos[j];
-                    dx = (float)(pj.x - q.x);
-                    dy = (float)(pj.y - q.y);
-                    dz = (float)(pj.z - q.z);
-                }
-                const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                if (!(d2 > 0.f) || !(d2 < h2)) continue;   // d = 0 is skipped
-                if constexpr (CNT) {
-                    nterms++;
-                    continue;
-                }
-                acc.add(k, d2, dx, dy, dz, vi, vel[j], rho[j]);
+    for_each_row<L>(k, cstart, q, cc1, cc2, x0, x1, [&](float ty, float tz, int b, int e) {
+        for (int j = b + sub; j < e; j += L) {
+            const float4 p = ofs[j];
+            float dx, dy, dz;   // x_j - x_i
+            if ((p.w >= 0.f) & !qfar) {
+                dx = p.x - (p.w == w0 ? tx0 : (p.w == w1 ? tx1 : tx2));
+                dy = p.y - ty;
+                dz = p.z - tz;
+            } else {
+                const double4 pj = pos[j];
+                dx = (float)(pj.x - q.x);
+                dy = (float)(pj.y - q.y);
+                dz = (float)(pj.z - q.z);
             }
+            const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+            if (!(d2 > 0.f) || !(d2 < h2)) continue;   // d = 0 is skipped
+            if constexpr (CNT) {
+                nterms++;
+                continue;
+            }
+            acc.add(k, d2, dx, dy, dz, vi, vel[j], rho[j]);
         }
-    }
+    });
     if constexpr (CNT) {
         members[i] = nterms;
         return;
     }
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) {
+        acc.lx += __shfl_xor(acc.lx, o, 64);
+        acc.ly += __shfl_xor(acc.ly, o, 64);
+        acc.lz += __shfl_xor(acc.lz, o, 64);
+    }
+    if (sub != 0) return;
     float4 v = vi;
     v.x += scale * acc.lx;
     v.y += scale * acc.ly;
@@ -247,7 +248,7 @@ int viscosity_member_counts(vps_context* c, int32_t* members) {
     if (n == 0) return VPS_OK;
     VPS_TRY(real_offsets(c));
     const int s = c->cur;
-    hipLaunchKernelGGL(k_viscosity3f<true>, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((k_viscosity3f<1, true>), dim3(blocks(n, 256)), dim3(256), 0, c->stream,
                        c->rpos[s].p, c->rofs.p, c->cell_start.p, c->rvel[s].p, c->rrho.p, n,
                        c->k, 0.f, (float4*)nullptr, members);
     VPS_HIP(c, hipGetLastError());
@@ -264,11 +265,18 @@ int apply_viscosity(vps_context* c, double dt, double nu) {
     const int s = c->cur;
     // v += nu lapl dt with lapl = 2 (Dim + 2) m sum(...)
     const float scale = (float)(nu * (2.0 * (c->dim + 2.0) * c->p.mass) * dt);
-    if (c->dim == 3)
-        hipLaunchKernelGGL(k_viscosity3f<false>, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
-                           c->rpos[s].p, c->rofs.p, c->cell_start.p, c->rvel[s].p, c->rrho.p,
-                           n, c->k, scale, c->vel_next.p);
-    else
+    if (c->dim == 3) {
+        auto run = [&](auto kern, int lanes) {
+            hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
+                               c->rpos[s].p, c->rofs.p, c->cell_start.p, c->rvel[s].p, c->rrho.p,
+                               n, c->k, scale, c->vel_next.p, (int32_t*)nullptr);
+        };
+        const int lanes = walk_lanes(n);
+        if (lanes == 8) run(k_viscosity3f<8>, 8);
+        else if (lanes == 4) run(k_viscosity3f<4>, 4);
+        else if (lanes == 2) run(k_viscosity3f<2>, 2);
+        else run(k_viscosity3f<1>, 1);
+    } else
         hipLaunchKernelGGL(k_viscosity2, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
                            c->rpos[s].p, c->cell_start.p, c->rvel[s].p, c->rrho.p, n, c->k,
                            scale, c->vel_next.p);
