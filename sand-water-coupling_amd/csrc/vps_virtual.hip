@@ -94,6 +94,11 @@ struct RealAcc {
     float nvx = 0.f, nvy = 0.f, nvz = 0.f;   // sum v_j W / rho_j
     float gx = 0.f, gy = 0.f, gz = 0.f;      // sum V_j gradK
     float dr = 0.f;                           // sum V_j v_j . gradK
+    // the sums of this lane and of the one `o` away (lanes that share a node)
+    __device__ __forceinline__ void add_lanes(int o) {
+        for (float* f : {&w, &sH, &sV, &den, &nvx, &nvy, &nvz, &gx, &gy, &gz, &dr})
+            *f += __shfl_xor(*f, o, 64);
+    }
     template <int D>
     __device__ __forceinline__ void add(const KConst& k, double d2, float dx,
                                         float dy, float dz, float4 vj,
@@ -134,16 +139,17 @@ struct RealAcc {
         const float wr = wh * inv_rhoj;
         w += wh;
         sH += spline_w_ab(spline_ab(r, k.inv_H), 1.f);
-        sV += Vj * Vj * wh;
-        den += Vj * wh;
+        const float vw = Vj * wh;
+        sV += Vj * vw;
+        den += vw;
         nvx += vj.x * wr;
         nvy += vj.y * wr;
         nvz += vj.z * wr;
-        const float ex = dx * sh, ey = dy * sh, ez = D == 3 ? dz * sh : 0.f;
-        gx += Vj * ex;
-        gy += Vj * ey;
-        gz += Vj * ez;
-        dr += Vj * (vj.x * ex + vj.y * ey + vj.z * ez);
+        const float vs = Vj * sh;
+        gx += dx * vs;
+        gy += dy * vs;
+        gz += D == 3 ? dz * vs : 0.f;
+        dr += vs * (vj.x * dx + vj.y * dy + (D == 3 ? vj.z * dz : 0.f));
     }
 };
 
@@ -152,6 +158,9 @@ struct RealAcc {
 struct BAcc {
     float den = 0.f, bnx = 0.f, bny = 0.f, bnz = 0.f;
     float hx = 0.f, hy = 0.f, hz = 0.f, db = 0.f;
+    __device__ __forceinline__ void add_lanes(int o) {
+        for (float* f : {&den, &bnx, &bny, &bnz, &hx, &hy, &hz, &db}) *f += __shfl_xor(*f, o, 64);
+    }
     // boundary particle at pj within h (FP64 test passed): accurate spline
     template <int D>
     __device__ __forceinline__ void add_exact(const KConst& k, double qx, double qy,
@@ -215,7 +224,9 @@ struct BoundaryWalkGlobal {
     }
 };
 
-template <int D, typename BW>
+// S lanes share a node: the real sums are the node's, the boundary walk is one
+// lane's part, and lane 0 writes.
+template <int D, int S = 1, typename BW>
 __device__ __forceinline__ void finish_node(
     const KConst& k, const RealAcc& a, double qx, double qy, double qz,
     int cx, int cy, int cz, int64_t out, const double4* rpos,
@@ -234,16 +245,20 @@ __device__ __forceinline__ void finish_node(
         });
         virt = w64 > 1e-6;
     }
+    const bool writes = S == 1 || threadIdx.x % S == 0;
     if (!virt) {
-        vrho[out] = 0.f;
-        vvol[out] = 0.f;
-        vb[out] = 0.f;
+        if (writes) vrho[out] = vvol[out] = vb[out] = 0.f;
         return;
     }
     // boundary neighbours within h
     BAcc b;
-    b.den = a.den;
+    if (writes) b.den = a.den;
     bwalk(k, qx, qy, qz, bvel, bnrm, b);
+    if constexpr (S > 1) {
+#pragma unroll
+        for (int o = 1; o < S; o <<= 1) b.add_lanes(o);
+    }
+    if (!writes) return;
     // v_I = (m sum v_j W/rho_j + m_b sum v_b W/rho_b) / (sum V W + sum V_b W + 1e-6)
     const float inv_den = 1.f / fmaf(b.den, k.c0h, 1e-6f);
     const float mc = k.mass * k.c0h;
@@ -317,304 +332,362 @@ __global__ void __launch_bounds__(NB) k_virtual_sums(
                    vb, bits);
 }
 
-// 3D with the brick's real neighbourhood staged in LDS (one workgroup of
-// 512 threads per brick, thread = node).  The cells within one cell of the
-// brick's nodes form <= kStageRows x-rows of <= kStageCx cells; their
-// particles (contiguous per row in the cell-sorted order) are copied once,
-// each as its FP32 offset from its own cell corner with 1/rho_j, and every
-// node walks its 3 x 3 x 3 cells from LDS in the order of the global walk.
+// 3D with the brick's neighbourhood staged in LDS: one workgroup of 512
+// threads per brick, thread = node, or S workgroups of 8 / S z-planes each
+// with S lanes per node.  The cells within one cell of the nodes form
+// <= kStageRows x-rows of <= kStageCx cells; their particles (contiguous per
+// row in the cell-sorted order) are copied once, each as its FP32 offset from
+// its own cell corner with 1/rho_j, first the real and behind them the
+// boundary ones, and every node walks its 3 x 3 x 3 cells from LDS in the
+// order of the global walk.
 // q - x_j = (q - C_q) - (x_j - C_j) + (C_q - C_j) with C the FP64 cell
 // corners, so the FP32 difference is accurate to a few ulp of h.
 // Membership is pre-tested in FP32 with a band around h^2 in which the
 // exact FP64 test on the original positions decides (also at r = 0 and for
 // particles clamped into a border cell), so the neighbour sets stay exact.
-// The boundary cell table of the same rows is staged too, so nodes away
-// from the walls skip the boundary walk without touching global memory.
 constexpr int kStageCap = 4096;
 constexpr int kStageRows = 64;
 constexpr int kStageCx = 8;
 
-// Boundary walk of one node over the staged rows' boundary cell table, with
-// the FP32 pre-test on the boundary's cell offsets (bofs) and the FP64 test
-// in the band around h (the boundary set stays exact).
-struct BoundaryWalkStaged {
-    const int (*bcs)[kStageCx + 1];   // global starts of the staged rows
-    const int* meta;                  // clo x,y,z; ncx, ncy
-    const double4* bpos;
-    const float4* bofs;
-    __device__ __forceinline__ void operator()(const KConst& k, double qx, double qy,
-                                               double qz, const float4* bvel,
-                                               const float4* bnrm, BAcc& b) const {
+// The staged neighbourhood.  px is taken from the corner of the row's first
+// cell (NaN: exact test only), py and pz from the particle's own cell; pw is
+// 1 / rho of a real particle, x from its own cell of a boundary particle.
+// Separate arrays: the membership test reads 12 bytes per candidate as three
+// 4-byte loads.  Two workgroups per CU, which is also what their registers
+// allow.
+template <int S>
+struct Stage {
+    // the scan reads up to 4 S - 1 entries beyond a row
+    float px[kStageCap + 4 * S], py[kStageCap + 4 * S], pz[kStageCap + 4 * S],
+        pw[kStageCap + 4 * S];
+    int cs[kStageRows][kStageCx + 1];    // cell starts of the rows, global
+    int bcs[kStageRows][kStageCx + 1];   // the boundary's
+    int rg[kStageRows], brg[kStageRows]; // global - staged index of a row
+};
+
+// One lane's part (candidates c0, c0 + S, ...) of a staged row's range
+// [c0, je): in chunks of 32, the cheap FP32 test near(j) sets a bit per
+// candidate not surely outside, then the lane visits only its own bits: fast(j)
+// says whether the FP32 test is certain (and then adds the pair), and the
+// others go to exact(j) afterwards, the lanes' together.  (A lane has ~15% of
+// its candidates within h, so the wave does not run the accumulation for every
+// candidate.)  The test appends its bit at the low end, so the highest set bit
+// is the next in order; it runs four candidates at a time past the end of the
+// range, whose bits are cleared.
+template <int S, typename Near, typename Fast, typename Exact>
+__device__ __forceinline__ void staged_range(int c0, int je, Near&& near, Fast&& fast,
+                                             Exact&& exact) {
+    for (; c0 < je; c0 += 32 * S) {
+        const int nc = min((je - c0 + S - 1) / S, 32);
+        uint32_t m = 0u, mexact = 0u;
+        int i = 0;
+        for (; i < nc; i += 4) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) m = m + m + near(c0 + (i + u) * S);
+        }
+        // candidate 0 to bit 31, candidates nc and on cleared
+        m = (m << (32 - i)) & (uint32_t)((int32_t)0x80000000 >> (nc - 1));
+        while (m) {
+            const int b = __builtin_clz(m);
+            const uint32_t bit = 0x80000000u >> b;
+            m &= ~bit;
+            if (!fast(c0 + b * S)) mexact |= bit;
+        }
+        while (mexact) {
+            const int b = __builtin_clz(mexact);
+            mexact &= ~(0x80000000u >> b);
+            exact(c0 + b * S);
+        }
+    }
+}
+
+// The staged rows around one node: f(jb, je, rg, ty, tz) per row with
+// candidates, jb .. je its staged range and q - C its y and z.
+// Cells whose nearest point lies beyond h (1 - 2e-6) are skipped: a whole row
+// by its y and z distance, the end cells of a row by their x distance.  Only
+// interior cells are culled (a border cell may hold particles clamped into it
+// from outside its extent).  The margin is twenty times the FP32 error of
+// these distances; a member it drops lies within 2.1e-6 h of the cutoff,
+// where W and W' are below 1e-17 and 5e-12 of their peaks, far below FP32
+// resolution of the sums.  On a lattice aligned with the cell grid (a node
+// every half cell) it skips the cells behind a node on a cell face; the nodes
+// of a wave share their z, so the rows behind them in z are skipped by the
+// whole wave.
+struct StagedRows {
+    int clo0, clo1, clo2, ncy;
+    template <typename F>
+    __device__ __forceinline__ void walk(const KConst& k, double qx, double qy, double qz,
+                                         const int (*cs)[kStageCx + 1], const int* rgs,
+                                         F&& f) const {
         const int cx = cell_coord(qx, k.cell_lo[0], k.cell_inv, k.cdims[0]);
         const int cy = cell_coord(qy, k.cell_lo[1], k.cell_inv, k.cdims[1]);
         const int cz = cell_coord(qz, k.cell_lo[2], k.cell_inv, k.cdims[2]);
         const int xlo = max(cx - 1, 0), xhi = min(cx + 1, k.cdims[0] - 1);
-        const int i0 = xlo - meta[0], i1 = xhi - meta[0] + 1;
-        float tx0 = (float)(qx - cell_corner(k, 0, xlo));
-        float tx1 = (float)(qx - cell_corner(k, 0, xlo + 1));
-        float tx2 = (float)(qx - cell_corner(k, 0, xlo + 2));
-        asm volatile("" : "+v"(tx0), "+v"(tx1), "+v"(tx2));
-        for (int z = max(cz - 1, 0); z <= min(cz + 1, k.cdims[2] - 1); z++) {
+        const int ylo = max(cy - 1, 0), yhi = min(cy + 1, k.cdims[1] - 1);
+        const int zlo = max(cz - 1, 0), zhi = min(cz + 1, k.cdims[2] - 1);
+        const int i0 = xlo - clo0, i1 = xhi - clo0;
+        const float csf = (float)k.cell_size;
+        const float h2c = (float)k.h2 * (1.f - 4e-6f);
+        auto gap = [csf](float t) { return fmaxf(fmaxf(-t, t - csf), 0.f); };   // q - C -> distance
+        const bool cut_l = xlo < xhi && xlo > 0, cut_r = xhi > xlo && xhi < k.cdims[0] - 1;
+        const float gl = gap((float)(qx - cell_corner(k, 0, xlo)));
+        const float gr = gap((float)(qx - cell_corner(k, 0, xhi)));
+        const float dl2 = cut_l ? gl * gl : 1e30f, dr2 = cut_r ? gr * gr : 1e30f;
+        for (int z = zlo; z <= zhi; z++) {
             const float tz = (float)(qz - cell_corner(k, 2, z));
-            for (int y = max(cy - 1, 0); y <= min(cy + 1, k.cdims[1] - 1); y++) {
-                const int r = (z - meta[2]) * meta[4] + (y - meta[1]);
-                const int jb = bcs[r][i0], je = bcs[r][i1];
-                if (jb >= je) continue;
+            const float gz = z > 0 && z < k.cdims[2] - 1 ? gap(tz) : 0.f;
+            for (int y = ylo; y <= yhi; y++) {
                 const float ty = (float)(qy - cell_corner(k, 1, y));
-                const int b1 = bcs[r][min(i0 + 1, i1)], b2 = bcs[r][min(i0 + 2, i1)];
-                for (int j0 = jb; j0 < je; j0 += 4) {
-                  float4 bov[4];
-#pragma unroll
-                  for (int u = 0; u < 4; u++)
-                      bov[u] = j0 + u < je ? bofs[j0 + u] : make_float4(1e30f, 0.f, 0.f, 1.f);
-#pragma unroll
-                  for (int u = 0; u < 4; u++) {
-                    const int j = j0 + u;
-                    const float4 bo = bov[u];
-                    const float tx = j < b1 ? tx0 : (j < b2 ? tx1 : tx2);
-                    const float dx = tx - bo.x, dy = ty - bo.y, dz = tz - bo.z;
-                    const float d2f = dx * dx + dy * dy + dz * dz;
-                    const Pretest t = pretest(k, d2f, bo.w);
-                    if (t.fast) b.add_fast(k, d2f, dx, dy, dz, bvel[j], bo.w);
-                    if (t.exact) {
-                        const double4 pj = bpos[j];
-                        const double d2 = sq_dist3(pj.x, pj.y, pj.z, qx, qy, qz);
-                        if (d2 < k.h2) b.add_exact<3>(k, qx, qy, qz, pj, d2, bvel[j], bnrm[j].w);
-                    }
-                  }
-                }
+                const float gy = y > 0 && y < k.cdims[1] - 1 ? gap(ty) : 0.f;
+                const float rem = h2c - gy * gy - gz * gz;
+                if (!(rem > 0.f)) continue;
+                const int r = (z - clo2) * ncy + (y - clo1);
+                const int rg = rgs[r];
+                const int jb = cs[r][i0 + (dl2 >= rem)] - rg;
+                const int je = cs[r][i1 + 1 - (dr2 >= rem)] - rg;
+                if (jb < je) f(jb, je, rg, ty, tz);
             }
         }
     }
 };
 
-__global__ void __launch_bounds__(512) k_virtual_sums3s(
+// Lanes per node: the fewest that fill the machine (a brick by itself takes
+// 52 us with one lane per node).  By the particles, not the bricks of the last
+// generation, so that a state gives the same bits however it was reached.  us
+// with 1, 2, 4, 8 lanes:
+//   576 particles 51, 31, 26, 21     16,000  53, 34, 28, 27
+//   32,000        54, 35, 33, 47     64,800  59, 45, 55, 71
+//   212,503       94, 90, 112, 153   300,000 112, 116, 147, 219
+//   1,012,500    264, 274, 382, 558
+inline int sums_lanes(int64_t n) {
+    return n <= 16000 ? 8 : (n <= 32000 ? 4 : (n <= 250000 ? 2 : 1));
+}
+
+// Bound by instructions and the latency of the walk (of 280 us at 1M: staging
+// 45, candidate tests 105, sums 85, boundary 45).  Before (one lane per node
+// for all sizes, the boundary walked in global memory, two masks per test,
+// rows staged through a binary search): 70 us at 576 particles, 77 at 64,800,
+// 120 at 212,503, 297 at 1,012,500.
+template <int S>
+__global__ void __launch_bounds__(512, 4) k_virtual_sums3s(
     KConst k, const int32_t* brick_of_slot, const int32_t* nslots_p,
     const double4* rpos, const float4* rvel, const float* rrho, const float* rrinv,
     const float4* rofs, const int32_t* rcstart, const double4* bpos,
     const float4* bofs, const float4* bvel, const float4* bnrm, const int32_t* bcstart,
     float* vrho, float* vvol, float* vb, uint32_t* bits) {
-    // x_j - C_clo (NaN: exact test only), y_j - C_j, z_j - C_j as separate
-    // arrays (the membership test and the sums read 12 bytes per candidate
-    // as three 4-byte loads); x from the row's first cell, y and z from the
-    // particle's own cell
-    __shared__ float s_px[kStageCap], s_py[kStageCap], s_pz[kStageCap];
-    __shared__ int s_cs[kStageRows][kStageCx + 1];  // real cell starts (staged)
-    __shared__ int s_bcs[kStageRows][kStageCx + 1]; // boundary cell starts
-    __shared__ int s_rg[kStageRows];    // global - staged index
-    __shared__ int s_off[kStageRows + 1];
-    __shared__ int s_meta[8];   // clo x,y,z; ncx, ncy, ncz; total; ok
+    constexpr int kPlanes = kBrick / S;
+    constexpr int kRowsAtOnce = 5;   // rows a wave loads at once (36 rows of a brick in one go)
+    __shared__ Stage<S> st;
     const int nslots = *nslots_p;   // the grid may exceed the slot count
-    if ((int)blockIdx.x >= nslots) return;
-    const int slot = xcd_remap(blockIdx.x, nslots);
+    if ((int)blockIdx.x >= nslots * S) return;
+    const int part = xcd_remap(blockIdx.x, nslots * S);
+    const int slot = part / S;
     const int brick = brick_of_slot[slot];
-    const int t = threadIdx.x;
-    // a wave: the 8 x 8 nodes of one z-plane of the brick
-    const int lx = t & 7, ly = (t >> 3) & 7, lz = t >> 6;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // a wave: the 8 x 8 nodes of one z-plane of the brick, or 8 x 8 / S of them
+    const int sub = S > 1 ? t % S : 0;
+    const int node = (part % S) * (512 / S) + t / S;
     const int bx = brick % k.bdims[0];
     const int by = (brick / k.bdims[0]) % k.bdims[1];
     const int bz = brick / k.bdims[0] / k.bdims[1];
-    const int n0[3] = {bx * kBrick, by * kBrick, bz * kBrick};
-    if (t == 0) {
-        int ok = 1, nrows = 1;
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            const int last = min(n0[a] + kBrick - 1, k.ndims[a] - 1);
-            const int clo = max(cell_coord(node_coord(k.origin[a], n0[a], k.spacing),
-                                           k.cell_lo[a], k.cell_inv, k.cdims[a]) - 1, 0);
-            const int chi = min(cell_coord(node_coord(k.origin[a], last, k.spacing),
-                                           k.cell_lo[a], k.cell_inv, k.cdims[a]) + 1,
-                                k.cdims[a] - 1);
-            s_meta[a] = clo;
-            s_meta[3 + a] = chi - clo + 1;
-            if (a > 0) nrows *= chi - clo + 1;
-        }
-        if (s_meta[3] > kStageCx || nrows > kStageRows) ok = 0;
-        s_meta[7] = ok;
-    }
-    __syncthreads();
-    const int ncx = s_meta[3], ncy = s_meta[4], ncz = s_meta[5];
-    const int nrows = ncy * ncz;
-    if (s_meta[7] && t < nrows) {
-        const int y = s_meta[1] + t % ncy, z = s_meta[2] + t / ncy;
-        const int64_t grow = ((int64_t)z * k.cdims[1] + y) * k.cdims[0] + s_meta[0];
-        for (int i = 0; i <= ncx; i++) {
-            s_cs[t][i] = rcstart[grow + i];
-            s_bcs[t][i] = bcstart[grow + i];
-        }
-    }
-    __syncthreads();
-    if (t == 0 && s_meta[7]) {
-        int acc = 0;
-        for (int r = 0; r < nrows; r++) {
-            s_off[r] = acc;
-            acc += s_cs[r][ncx] - s_cs[r][0];
-        }
-        s_off[nrows] = acc;
-        s_meta[6] = acc;
-        if (acc > kStageCap) s_meta[7] = 0;
-    }
-    __syncthreads();
-    const bool staged = s_meta[7] != 0;
-    if (staged) {
-        if (t < nrows) {
-            const int g0 = s_cs[t][0];
-            s_rg[t] = g0 - s_off[t];
-            for (int i = 0; i <= ncx; i++) s_cs[t][i] += s_off[t] - g0;
-        }
-        __syncthreads();
-        const int total = s_meta[6];
-        for (int e0 = 0; e0 < total; e0 += 4 * 512) {
-            float4 pj[4];
-            int ci[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int e = e0 + u * 512 + t;
-                ci[u] = 0;
-                if (e < total) {
-                    // row of staged element e: last r with s_off[r] <= e
-                    int lo = 0, hi = nrows - 1;
-                    while (lo < hi) {
-                        const int mid = (lo + hi + 1) >> 1;
-                        if (s_off[mid] <= e) lo = mid;
-                        else hi = mid - 1;
-                    }
-                    pj[u] = rofs[e + s_rg[lo]];
-                    // its cell within the row (x = clo + ci)
-                    for (int i = 1; i < ncx; i++) ci[u] += s_cs[lo][i] <= e;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int e = e0 + u * 512 + t;
-                if (e < total) {
-                    // x relative to the corner of the row's first cell
-                    // (C_(clo+ci) - C_clo = ci cells), rounded once from
-                    // FP64; a particle marked for the exact test only gets
-                    // x = NaN, which no FP32 test passes
-                    const float xr = pj[u].w < 0.f
-                                         ? __builtin_nanf("")
-                                         : (float)((double)pj[u].x + (double)ci[u] * k.cell_size);
-                    s_px[e] = xr;
-                    s_py[e] = pj[u].y;
-                    s_pz[e] = pj[u].z;
-                }
-            }
-        }
-        __syncthreads();
-    }
-    const int cx = n0[0] + lx, cy = n0[1] + ly, cz = n0[2] + lz;
-    const int64_t out = (int64_t)slot * 512 + t;
-    if (cx >= k.ndims[0] || cy >= k.ndims[1] || cz >= k.ndims[2]) {
-        vrho[out] = 0.f;
-        vvol[out] = 0.f;
-        vb[out] = 0.f;
+    const int n0[3] = {bx * kBrick, by * kBrick, bz * kBrick + (part % S) * kPlanes};
+    const int cx = n0[0] + (node & 7), cy = n0[1] + ((node >> 3) & 7),
+              cz = bz * kBrick + (node >> 6);
+    const int64_t out = (int64_t)slot * 512 + node;
+    if (S > 1 && n0[2] >= k.ndims[2]) {   // no plane of this block is on the lattice
+        if (sub == 0) vrho[out] = vvol[out] = vb[out] = 0.f;
         return;
+    }
+    int clo[3], nc[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const int last = min(n0[a] + (a == 2 ? kPlanes : kBrick) - 1, k.ndims[a] - 1);
+        clo[a] = max(cell_coord(node_coord(k.origin[a], n0[a], k.spacing), k.cell_lo[a],
+                                k.cell_inv, k.cdims[a]) - 1, 0);
+        nc[a] = min(cell_coord(node_coord(k.origin[a], last, k.spacing), k.cell_lo[a],
+                               k.cell_inv, k.cdims[a]) + 1, k.cdims[a] - 1) - clo[a] + 1;
+    }
+    const int ncx = nc[0], ncy = nc[1], nrows = nc[1] * nc[2];
+    bool staged = ncx <= kStageCx && nrows <= kStageRows, pooled = false;
+    int nboundary = 0;
+    if (staged) {
+        for (int e = t; e < nrows * (kStageCx + 1); e += 512) {
+            const int r = e / (kStageCx + 1), i = e % (kStageCx + 1);
+            if (i > ncx) continue;
+            const int64_t g = ((int64_t)(clo[2] + r / ncy) * k.cdims[1] + clo[1] + r % ncy) *
+                                  k.cdims[0] + clo[0] + i;
+            st.cs[r][i] = rcstart[g];
+            st.bcs[r][i] = bcstart[g];
+        }
+        __syncthreads();
+        // Every wave scans the rows' lengths for itself (lane = row).
+        const int row = min(lane, nrows - 1);
+        const int rlen = lane < nrows ? st.cs[row][ncx] - st.cs[row][0] : 0;
+        const int blen = lane < nrows ? st.bcs[row][ncx] - st.bcs[row][0] : 0;
+        int rend = rlen, bend = blen;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int a = __shfl_up(rend, o, 64), b = __shfl_up(bend, o, 64);
+            if (lane >= o) {
+                rend += a;
+                bend += b;
+            }
+        }
+        const int total = __shfl(rend, 63, 64);
+        staged = total <= kStageCap;
+        nboundary = __shfl(bend, 63, 64);
+        pooled = staged && total + nboundary <= kStageCap;
+        if (wave == 0 && lane < nrows) {
+            st.rg[lane] = st.cs[lane][0] - (rend - rlen);
+            st.brg[lane] = st.bcs[lane][0] - (total + bend - blen);
+        }
+        // The waves take the rows in turn, kRowsAtOnce of them loading together.
+        auto put = [&](int e, const float4& p, int cell, float pw) {
+            // x relative to the corner of the row's first cell (C_c - C_clo =
+            // c - clo cells), rounded once from FP64; a particle marked for
+            // the exact test only gets x = NaN, which no FP32 test passes
+            st.px[e] = p.w < 0.f ? __builtin_nanf("")
+                                 : (float)((double)p.x + (double)cell * k.cell_size);
+            st.py[e] = p.y;
+            st.pz[e] = p.z;
+            st.pw[e] = pw;
+        };
+        auto put_real = [&](int e, const float4& p, float rinv) {
+            put(e, p, (int)p.w - 1 - clo[0], rinv);
+        };
+        auto put_boundary = [&](int r, int e, int at, const float4& p) {
+            int cell = 0;
+            for (int i = 1; i < ncx; i++) cell += st.bcs[r][i] <= st.bcs[r][0] + e;
+            put(at + e, p, cell, p.x);
+        };
+        for (int r0 = wave; staged && r0 < nrows; r0 += 8 * kRowsAtOnce) {
+            float4 p[kRowsAtOnce], pb[kRowsAtOnce];
+            float ri[kRowsAtOnce];
+            int at[kRowsAtOnce], bat[kRowsAtOnce], len[kRowsAtOnce], bl[kRowsAtOnce];
+#pragma unroll
+            for (int u = 0; u < kRowsAtOnce; u++) {
+                const int r = min(r0 + 8 * u, nrows - 1);
+                len[u] = r0 + 8 * u < nrows ? __shfl(rlen, r, 64) : 0;
+                bl[u] = r0 + 8 * u < nrows && pooled ? __shfl(blen, r, 64) : 0;
+                at[u] = __shfl(rend, r, 64) - len[u];
+                bat[u] = total + __shfl(bend, r, 64) - bl[u];
+                if (lane < len[u]) {
+                    p[u] = rofs[st.cs[r][0] + lane];
+                    ri[u] = rrinv[st.cs[r][0] + lane];
+                }
+                if (lane < bl[u]) pb[u] = bofs[st.bcs[r][0] + lane];
+            }
+#pragma unroll
+            for (int u = 0; u < kRowsAtOnce; u++) {
+                if (lane < len[u]) put_real(at[u] + lane, p[u], ri[u]);
+                const int r = min(r0 + 8 * u, nrows - 1);
+                if (lane < bl[u]) put_boundary(r, lane, bat[u], pb[u]);
+                for (int e = 64 + lane; e < len[u]; e += 64)
+                    put_real(at[u] + e, rofs[st.cs[r][0] + e], rrinv[st.cs[r][0] + e]);
+                for (int e = 64 + lane; e < bl[u]; e += 64)
+                    put_boundary(r, e, bat[u], bofs[st.bcs[r][0] + e]);
+            }
+        }
+        __syncthreads();
+    }
+    if (cx >= k.ndims[0] || cy >= k.ndims[1] || cz >= k.ndims[2]) {
+        if (sub == 0) vrho[out] = vvol[out] = vb[out] = 0.f;
+        return;   // uniform over the lanes of a node
     }
     const double qx = node_coord(k.origin[0], cx, k.spacing);
     const double qy = node_coord(k.origin[1], cy, k.spacing);
     const double qz = node_coord(k.origin[2], cz, k.spacing);
     RealAcc a;
     if (!staged) {
+        if (sub != 0) return;
         real_walk_global<3>(k, rcstart, rpos, rvel, rrho, qx, qy, qz, a);
         finish_node<3>(k, a, qx, qy, qz, cx, cy, cz, out, rpos, rcstart,
                        BoundaryWalkGlobal<3>{bcstart, bpos}, bvel, bnrm, vrho,
                        vvol, vb, bits);
         return;
     }
-    // q - C_c per axis for the candidate cell c, rounded once from FP64
-    // (the staged x_j - C_j complete the difference q - x_j)
-    const int cc0 = cell_coord(qx, k.cell_lo[0], k.cell_inv, k.cdims[0]);
-    const int cc1 = cell_coord(qy, k.cell_lo[1], k.cell_inv, k.cdims[1]);
-    const int cc2 = cell_coord(qz, k.cell_lo[2], k.cell_inv, k.cdims[2]);
-    const int xlo = max(cc0 - 1, 0), xhi = min(cc0 + 1, k.cdims[0] - 1);
-    const int zlo = max(cc2 - 1, 0), zhi = min(cc2 + 1, k.cdims[2] - 1);
-    const int ylo = max(cc1 - 1, 0), yhi = min(cc1 + 1, k.cdims[1] - 1);
-    // The (up to) three cells xlo .. xhi of a row are one contiguous staged
-    // range.  The membership test and a member's sums take x relative to the
-    // same corner C_clo for all of them (one offset per node, rounded once
+    // The membership test and a real member's sums take x relative to the same
+    // corner C_clo for all cells of a row (one offset per node, rounded once
     // from FP64: within 2e-7 h for offsets of up to three cells, inside the
     // FP64 band for the test and far below the tolerance of the sums).
-    const float tx = (float)(qx - cell_corner(k, 0, s_meta[0]));
-    float tx0 = (float)(qx - cell_corner(k, 0, xlo));
-    float tx1 = (float)(qx - cell_corner(k, 0, xlo + 1));
-    float tx2 = (float)(qx - cell_corner(k, 0, xlo + 2));
-    asm volatile("" : "+v"(tx0), "+v"(tx1), "+v"(tx2));
-    const int i0 = xlo - s_meta[0], i1 = xhi - s_meta[0];
+    const float tx = (float)(qx - cell_corner(k, 0, clo[0]));
     // h2_min < d2f < h2f_lo as one unsigned test on the bits (NaN fails).
     // Below h2_min (the band's width, far above the error of d2f near 0)
     // the exact test decides, so a fast member's accurate d2f is > 0.
     const uint32_t lo_min = __float_as_uint(k.h2f_hi - k.h2f_lo);
     const uint32_t lo_span = __float_as_uint(k.h2f_lo) - lo_min - 1u;
-    // Cells whose nearest point lies beyond h (1 - 2e-6) are skipped: a
-    // whole row by its y and z distance, the end cells of a row by their x
-    // distance.  Only interior cells are culled (a border cell may hold
-    // particles clamped into it from outside its extent).  The margin is
-    // twenty times the FP32 error of these distances; a member it drops lies
-    // within 2.1e-6 h of the cutoff, where W and W' are below 1e-17 and
-    // 5e-12 of their peaks, far below FP32 resolution of the sums.  On a
-    // lattice aligned with the cell grid (a node every half cell) it skips
-    // the cells behind a node on a cell face; the nodes of a wave share
-    // their z, so the rows behind them in z are skipped by the whole wave.
-    const float csf = (float)k.cell_size;
-    const float h2c = (float)k.h2 * (1.f - 4e-6f);
-    auto gap = [csf](float t) { return fmaxf(fmaxf(-t, t - csf), 0.f); };   // q - C -> distance
-    const float txh = xhi - xlo == 2 ? tx2 : (xhi - xlo == 1 ? tx1 : tx0);
-    const bool cut_l = xlo < xhi && xlo > 0, cut_r = xhi > xlo && xhi < k.cdims[0] - 1;
-    const float gl = gap(tx0), gr = gap(txh);
-    const float dl2 = cut_l ? gl * gl : 1e30f, dr2 = cut_r ? gr * gr : 1e30f;
-    for (int z = zlo; z <= zhi; z++) {
-        const float tz = (float)(qz - cell_corner(k, 2, z));
-        const float gz = z > 0 && z < k.cdims[2] - 1 ? gap(tz) : 0.f;
-        for (int y = ylo; y <= yhi; y++) {
-            const float ty = (float)(qy - cell_corner(k, 1, y));
-            const float gy = y > 0 && y < k.cdims[1] - 1 ? gap(ty) : 0.f;
-            const float rem = h2c - gy * gy - gz * gz;
-            if (!(rem > 0.f)) continue;
-            const int r = (z - s_meta[2]) * ncy + (y - s_meta[1]);
-            const int rg = s_rg[r];
-            const int jb = s_cs[r][i0 + (dl2 >= rem)], je = s_cs[r][i1 + 1 - (dr2 >= rem)];
-            // Two passes per chunk of 32 candidates: the cheap FP32 test
-            // sets one bit per member, then each lane visits only its own
-            // members (a lane has ~15% of its candidates within h, so the
-            // wave no longer runs the accumulation for every candidate).
-            // Candidate c0 + i sits at bit i, so the lowest set bit is the
-            // next in order.
-            for (int c0 = jb; c0 < je; c0 += 32) {
-                const int c1 = min(c0 + 32, je);
-                uint32_t mfast = 0u, mexact = 0u;
-                for (int j = c0; j < c1; j++) {
-                    const float dx = tx - s_px[j], dy = ty - s_py[j], dz = tz - s_pz[j];
-                    const float d2f = dx * dx + dy * dy + dz * dz;
-                    const bool fast = __float_as_uint(d2f) - lo_min - 1u < lo_span;
-                    const bool exact = !(d2f >= k.h2f_hi) & !fast;   // NaN: exact
-                    mfast |= (uint32_t)fast << (j - c0);
-                    mexact |= (uint32_t)exact << (j - c0);
-                }
-                while (mfast) {
-                    const int j = c0 + __builtin_ctz(mfast);
-                    mfast &= mfast - 1u;
-                    const float dx = tx - s_px[j], dy = ty - s_py[j], dz = tz - s_pz[j];
-                    const float d2f = dx * dx + dy * dy + dz * dz;
-                    a.add_fast<3>(k, d2f, dx, dy, dz, rvel[j + rg], rrinv[j + rg]);
-                }
-                while (mexact) {
-                    // the reference's FP64 test and the accurate spline
-                    const int j = c0 + __builtin_ctz(mexact);
-                    mexact &= mexact - 1u;
+    auto sq = [](const float3& d) { return d.x * d.x + d.y * d.y + d.z * d.z; };
+    auto sure = [&](float d2f) { return __float_as_uint(d2f) - lo_min - 1u < lo_span; };
+    const StagedRows rows{clo[0], clo[1], clo[2], ncy};
+    rows.walk(k, qx, qy, qz, st.cs, st.rg, [&](int jb, int je, int rg, float ty, float tz) {
+        auto offset = [&](int j) {
+            return make_float3(tx - st.px[j], ty - st.py[j], tz - st.pz[j]);
+        };
+        staged_range<S>(
+            jb + sub, je, [&](int j) { return !(sq(offset(j)) >= k.h2f_hi); },
+            [&](int j) {
+                const float3 d = offset(j);
+                const float d2f = sq(d);
+                const bool in = sure(d2f);
+                if (in) a.add_fast<3>(k, d2f, d.x, d.y, d.z, rvel[j + rg], st.pw[j]);
+                return in;
+            },
+            [&](int j) {
+                // the reference's FP64 test and the accurate spline
+                const int g = j + rg;
+                const double4 pj = rpos[g];
+                const double d2 = sq_dist3(pj.x, pj.y, pj.z, qx, qy, qz);
+                if (d2 < k.h2)
+                    a.add<3>(k, d2, (float)(qx - pj.x), (float)(qy - pj.y), (float)(qz - pj.z),
+                             rvel[g], st.pw[j]);
+            });
+    });
+    if constexpr (S > 1) {
+#pragma unroll
+        for (int o = 1; o < S; o <<= 1) a.add_lanes(o);
+    }
+    // One lane's part of the boundary walk, over the staged rows as well; from
+    // global memory where the boundary did not fit the stage.  The sums take x
+    // from the particle's own cell.
+    auto boundary = [&](const KConst& k, double qx, double qy, double qz, const float4* bvel,
+                        const float4* bnrm, BAcc& b) {
+        if (!pooled) {
+            if (sub == 0) BoundaryWalkGlobal<3>{bcstart, bpos}(k, qx, qy, qz, bvel, bnrm, b);
+            return;
+        }
+        if (nboundary == 0) return;
+        const int xlo = max(cell_coord(qx, k.cell_lo[0], k.cell_inv, k.cdims[0]) - 1, 0);
+        float tx0 = (float)(qx - cell_corner(k, 0, xlo));
+        float tx1 = (float)(qx - cell_corner(k, 0, xlo + 1));
+        float tx2 = (float)(qx - cell_corner(k, 0, xlo + 2));
+        const float s1 = (float)((double)(xlo - clo[0]) + 0.5) * (float)k.cell_size;
+        rows.walk(k, qx, qy, qz, st.bcs, st.brg, [&](int jb, int je, int rg, float ty, float tz) {
+            auto offset = [&](int j) {
+                return make_float3(tx - st.px[j], ty - st.py[j], tz - st.pz[j]);
+            };
+            staged_range<S>(
+                jb + sub, je, [&](int j) { return !(sq(offset(j)) >= k.h2f_hi); },
+                [&](int j) {
+                    float3 d = offset(j);
+                    const bool in = sure(sq(d));
+                    if (in) {
+                        const float own = st.pw[j], c = st.px[j] - own - s1;
+                        d.x = (c < 0.f ? tx0 : (c < (float)k.cell_size ? tx1 : tx2)) - own;
+                        b.add_fast(k, sq(d), d.x, d.y, d.z, bvel[j + rg], bofs[j + rg].w);
+                    }
+                    return in;
+                },
+                [&](int j) {
                     const int g = j + rg;
-                    const double4 pj = rpos[g];
+                    const double4 pj = bpos[g];
                     const double d2 = sq_dist3(pj.x, pj.y, pj.z, qx, qy, qz);
                     if (d2 < k.h2)
-                        a.add<3>(k, d2, (float)(qx - pj.x), (float)(qy - pj.y),
-                                 (float)(qz - pj.z), rvel[g], rrinv[g]);
-                }
-            }
-        }
-    }
-    finish_node<3>(k, a, qx, qy, qz, cx, cy, cz, out, rpos, rcstart,
-                   BoundaryWalkStaged{s_bcs, s_meta, bpos, bofs}, bvel, bnrm, vrho,
-                   vvol, vb, bits);
+                        b.add_exact<3>(k, qx, qy, qz, pj, d2, bvel[g], bnrm[g].w);
+                });
+        });
+    };
+    finish_node<3, S>(k, a, qx, qy, qz, cx, cy, cz, out, rpos, rcstart, boundary, bvel, bnrm, vrho,
+                      vvol, vb, bits);
 }
 
 // Column order of the 3D slots, for the CG iteration's walk up z-runs of
@@ -781,14 +854,20 @@ static int generate_slots(vps_context* c, int w, int64_t grid, bool first) {
     const int rs = c->cur;
     const int32_t* nsl = (const int32_t*)c->counters.p;   // slot count
     int64_t* dcnt = c->counters.p;
-    if (D == 3)
-        hipLaunchKernelGGL(k_virtual_sums3s, dim3((unsigned)grid),
-                           dim3(512), 0, c->stream, c->k, c->slot_brick[w].p,
-                           nsl, c->rpos[rs].p, c->rvel[rs].p, c->rrho.p, c->rrinv.p, c->rofs.p,
-                           c->cell_start.p, c->bpos.p, c->bofs.p, c->bvel.p, c->bnrm.p,
-                           c->bcell_start.p, c->vrho.p, c->vvol.p, c->vb.p,
-                           c->bits.p);
-    else
+    if (D == 3) {
+        auto run = [&](auto kern, int s) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)(grid * s)), dim3(512), 0, c->stream, c->k,
+                               c->slot_brick[w].p, nsl, c->rpos[rs].p, c->rvel[rs].p, c->rrho.p,
+                               c->rrinv.p, c->rofs.p, c->cell_start.p, c->bpos.p, c->bofs.p,
+                               c->bvel.p, c->bnrm.p, c->bcell_start.p, c->vrho.p, c->vvol.p,
+                               c->vb.p, c->bits.p);
+        };
+        const int lanes = sums_lanes(c->n);
+        if (lanes == 8) run(k_virtual_sums3s<8>, 8);
+        else if (lanes == 4) run(k_virtual_sums3s<4>, 4);
+        else if (lanes == 2) run(k_virtual_sums3s<2>, 2);
+        else run(k_virtual_sums3s<1>, 1);
+    } else
         hipLaunchKernelGGL((k_virtual_sums<2, 64>), dim3((unsigned)grid),
                            dim3(64), 0, c->stream, c->k, c->slot_brick[w].p,
                            nsl, c->rpos[rs].p, c->rvel[rs].p, c->rrho.p,
