@@ -215,7 +215,7 @@ void free_all(vps_context* c) {
     dfree(c->rofs);
     dfree(c->bofs);
     dfree(c->vel_next);
-    dfree(c->grad_chunks);
+    dfree(c->grad_units);
     dfree(c->grad_over);
     dfree(c->couple_stage);
     dfree(c->io_stage);
@@ -1058,7 +1058,7 @@ int vps_debug_apply_operator(vps_context* c, const double* p, double* out) {
 int vps_debug_member_counts(vps_context* c, int32_t which, int32_t* counts) {
     if (!c || !counts || which < 0 || which > 3) return VPS_ERR_INVALID_ARG;
     if (c->dim != 3) return fail(c, VPS_ERR_INVALID_ARG, "member counts are 3D only");
-    if (which == 2 && (c->nslots == 0 || c->grad_span_cells <= 0))
+    if (which == 2 && (c->nslots == 0 || !c->grad_staged))
         return fail(c, VPS_ERR_STATE, "no virtual set or no staged gradient");
     const int64_t n = which == 1 ? c->nb : c->n;
     if (n == 0) return VPS_OK;

@@ -12,6 +12,7 @@
 // Grid::dataPosition rounds them) and the exact FP64 test
 // ((dx^2 + dy^2) + dz^2) < H^2 decides membership.  The brick map gives
 // q_J = V_J p_J (zero on non-virtual nodes).
+#include <algorithm>
 #include <cmath>
 
 #include "vps_internal.h"
@@ -24,13 +25,14 @@ inline unsigned blocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs)
 constexpr int kBox = 10;   // max node candidates per axis (2H/s + 2)
 
 // Boundary part of the update: -sum_b V_b min(n_b.(v_i - v_b), 0) n_b W_h.
-template <int D>
+// L lanes share a particle, each taking every L-th candidate of a row.
+template <int D, int L = 1>
 __device__ __forceinline__ void boundary_term(const KConst& k, const double4& q,
                                               const float4& vi, const double4* bpos,
                                               const float4* bvel, const float4* bnrm,
                                               const int32_t* bcstart, float& fx,
-                                              float& fy, float& fz) {
-    for_each_candidate<D>(k, bcstart, bpos, q.x, q.y, q.z, [&](int j, const double4& pj) {
+                                              float& fy, float& fz, int sub = 0) {
+    auto visit = [&](int j, const double4& pj) {
         const double d2 = D == 3 ? sq_dist3(pj.x, pj.y, pj.z, q.x, q.y, q.z)
                                  : sq_dist2(pj.x, pj.y, q.x, q.y);
         if (d2 < k.h2) {
@@ -55,9 +57,23 @@ __device__ __forceinline__ void boundary_term(const KConst& k, const double4& q,
             fy -= sc * nb.y;
             if (D == 3) fz -= sc * nb.z;
         }
-    });
+    };
+    if constexpr (L == 1) {
+        for_each_candidate<D>(k, bcstart, bpos, q.x, q.y, q.z, visit);
+    } else {
+        const int cx = cell_coord(q.x, k.cell_lo[0], k.cell_inv, k.cdims[0]);
+        const int cy = cell_coord(q.y, k.cell_lo[1], k.cell_inv, k.cdims[1]);
+        const int cz = cell_coord(q.z, k.cell_lo[2], k.cell_inv, k.cdims[2]);
+        for_each_row<L>(k, bcstart, q, cy, cz, max(cx - 1, 0), min(cx + 1, k.cdims[0] - 1),
+                        [&](float, float, int b, int e) {
+            for (int j = b + sub; j < e; j += 2 * L) {
+                const double4 p0 = bpos[j], p1 = bpos[min(j + L, e - 1)];
+                visit(j, p0);
+                if (j + L < e) visit(j + L, p1);
+            }
+        });
+    }
 }
-
 
 // Virtual part of the update from global memory: the node box around x_i,
 // exact FP64 membership, brick map lookups.
@@ -174,17 +190,18 @@ __global__ void __launch_bounds__(256) k_gradient(
 }
 
 // ---- LDS-staged 3D gradient ---------------------------------------------
-// Work unit: a span of up to span_cells consecutive cells of one cell row
-// (the particles of a span are contiguous in the sorted order).  The block
-// stages q = V p of the node box that holds every particle's candidates
-// (nodes f-3 .. f+4 per axis around f = floor((x - origin) / s): the nodes
-// within H = 4s of x), zero off the virtual set and off the lattice, then
-// each thread sums its particle's 8 x 8 x 8 candidates from LDS.  Nodes at
-// or beyond H get S = 0 from the spline itself; the kernel gradient is
-// continuous and zero at H, so the FP32 distance decides membership (a
-// node within rounding of H contributes nothing measurable).  A span whose
-// box exceeds the stage (particles far outside their cells) takes the
-// global per-particle path.
+// Work unit: a block of cells (UnitArgs).  The workgroup stages q = V p of
+// the node box that holds every particle's candidates (nodes f-3 .. f+4 per
+// axis around f = floor((x - origin) / s): the nodes within H = 4s of x),
+// zero off the virtual set and off the lattice, then L lanes sum a
+// particle's 8 x 8 x 8 candidates from LDS.  Nodes at or beyond H get S = 0
+// from the spline itself; the kernel gradient is continuous and zero at H,
+// so the FP32 distance decides membership (a node within rounding of H
+// contributes nothing measurable).  A unit whose box exceeds the stage
+// (particles far outside their cells) takes the global per-particle path.
+// Bound by the candidates' arithmetic where the machine is full (of 164 us at
+// 1,012,500 particles about 80; staging 45, the boundary 30), by one
+// particle's chain of 350 candidates and 27 boundary cells below.
 constexpr int kGradThreads = 256;
 constexpr int kGradCap = 7168;   // staged nodes (28 KB: five blocks per CU)
 constexpr int kGradBoxBricks = 128;   // bricks a staged box may touch
@@ -195,38 +212,44 @@ __device__ __forceinline__ int node_floor(double x, double o, double inv) {
     return (int)f;
 }
 
-// Spans whose box exceeds the stage, from the overflow list that
+// Units whose box exceeds the stage, from the overflow list that
 // k_gradient3s fills: the global-memory path, one thread per particle.
 __global__ void __launch_bounds__(kGradThreads) k_gradient_overflow(
-    KConst k, const int4* chunks, const int32_t* over, const int32_t* nover,
+    KConst k, UnitArgs ua, const int32_t* over, const int32_t* nover,
     const double4* rpos, float4* rvel, const int32_t* slot_of_brick, const float* vq,
     const double4* bpos, const float4* bvel, const float4* bnrm, const int32_t* bcstart,
     SolveGuard guard) {
     if (!solve_accepted(guard)) return;
     const int no = *nover;
     for (int o = blockIdx.x; o < no; o += gridDim.x) {
-        const int4 ch = chunks[over[o]];
-        for (int p = ch.x + threadIdx.x; p < ch.y; p += kGradThreads) {
-            const double4 q = rpos[p];
-            const float4 vi = rvel[p];
-            float fx = 0.f, fy = 0.f, fz = 0.f;
-            virtual_term_global<3>(k, q, slot_of_brick, vq, fx, fy, fz);
-            boundary_term<3>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz);
-            float4 v = vi;
-            v.x += fx;
-            v.y += fy;
-            v.z += fz;
-            rvel[p] = v;
+        const UnitCells uc(k, ua, over[o]);
+        for (int r = 0; r < uc.rows(); r++) {
+            const int64_t row = uc.row(k, r);
+            const int end = ua.cstart[row + uc.m[0]];
+            for (int p = ua.cstart[row] + threadIdx.x; p < end; p += kGradThreads) {
+                const double4 q = rpos[p];
+                const float4 vi = rvel[p];
+                float fx = 0.f, fy = 0.f, fz = 0.f;
+                virtual_term_global<3>(k, q, slot_of_brick, vq, fx, fy, fz);
+                boundary_term<3>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz);
+                float4 v = vi;
+                v.x += fx;
+                v.y += fy;
+                v.z += fz;
+                rvel[p] = v;
+            }
         }
     }
 }
 
+// L lanes share a particle: lane `sub` takes x candidates P and 7 - P of every
+// row for the pairs P = sub, sub + L, ... of 4 (with 8 lanes: candidate sub).
 // CNT (test support): vq holds V_J instead of q_J, and only the number of
 // virtual particles whose term enters the sum (V_J > 0, r < H in the FP32
-// spline) goes into members[p]; spans beyond the stage are left out.
-template <bool CNT = false>
+// spline) goes into members[p]; units beyond the stage are left out.
+template <int L, bool CNT = false>
 __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
-    KConst k, const int4* chunks, int nchunks, const double4* rpos, float4* rvel,
+    KConst k, UnitArgs ua, int nunits, const double4* rpos, float4* rvel,
     const int32_t* slot_of_brick, const float* vq, const double4* bpos,
     const float4* bvel, const float4* bnrm, const int32_t* bcstart, int32_t* over,
     int32_t* nover, SolveGuard guard, int32_t* members = nullptr) {
@@ -234,36 +257,60 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
     __shared__ float s_q[kGradCap];
     __shared__ int s_bslot[kGradBoxBricks];   // slots of the box's bricks
     __shared__ int s_box[6];
-    __shared__ int s_walls;   // boundary particles in the cells around the span
-    const int chunk = xcd_remap(blockIdx.x, nchunks);
-    const int4 ch = chunks[chunk];
+    __shared__ int s_walls;   // boundary particles in the cells around the unit
+    __shared__ int s_first[kUnitRows];     // first particle of a row - those before
+    __shared__ int s_off[kUnitRows + 1];   // particles before row r (rows beyond: all)
+    const int unit = ua.units[xcd_remap(blockIdx.x, nunits)];
+    const UnitCells uc(k, ua, unit);
     const int t = threadIdx.x;
-    if (t < 3) {
-        s_box[t] = 0x7fffffff;
-        s_box[t + 3] = -0x7fffffff;
-    }
-    if (t == 3) s_walls = 0;
-    __syncthreads();
-    if (t < 9) {
-        // the boundary cells that the particles' walks would visit: the
-        // span's cells +-1 along x in the 3 x 3 neighbour rows
-        const int cdx = k.cdims[0], cdy = k.cdims[1], cdz = k.cdims[2];
-        const int row = ch.z / cdx;
-        const int cy = row % cdy, cz = row / cdy;
-        const int x0 = ch.z - row * cdx, x1 = ch.w - 1 - row * cdx;
-        const int yy = cy + t % 3 - 1, zz = cz + t / 3 - 1;
-        if (yy >= 0 && zz >= 0 && yy < cdy && zz < cdz) {
-            const int64_t rb = ((int64_t)zz * cdy + yy) * cdx;
-            const int lo = x0 > 0 ? x0 - 1 : 0, hi = x1 + 1 < cdx ? x1 + 1 : cdx - 1;
-            if (bcstart[rb + hi + 1] > bcstart[rb + lo]) s_walls = 1;
+    if (t < 64) {
+        int b = 0, len = 0;
+        if (t < uc.rows()) {
+            const int64_t row = uc.row(k, t);
+            b = ua.cstart[row];
+            len = ua.cstart[row + uc.m[0]] - b;
         }
-    }
+        int end = len;
+#pragma unroll
+        for (int o = 1; o < kUnitRows; o <<= 1) {
+            const int a = __shfl_up(end, o, 64);
+            if (t >= o) end += a;
+        }
+        if (t < kUnitRows) {
+            s_first[t] = b - (end - len);
+            s_off[t + 1] = end;
+        }
+        if (t == 0) s_off[0] = 0;
+        // the boundary cells that the particles' walks would visit: the
+        // unit's cells and those around them, a row per thread
+        const int w1 = uc.m[1] + 2, rows = w1 * (uc.m[2] + 2);
+        bool walls = false;
+        for (int r = t; r < rows; r += 64) {
+            const int y = uc.c[1] - 1 + r % w1, z = uc.c[2] - 1 + r / w1;
+            if (y < 0 || z < 0 || y >= k.cdims[1] || z >= k.cdims[2]) continue;
+            const int64_t row = ((int64_t)z * k.cdims[1] + y) * k.cdims[0];
+            const int lo = max(uc.c[0] - 1, 0), hi = min(uc.c[0] + uc.m[0], k.cdims[0] - 1);
+            walls |= bcstart[row + hi + 1] > bcstart[row + lo];
+        }
+        const bool any = __any(walls);
+        if (t == 0) s_walls = any;
+    } else if (t < 70)
+        s_box[t - 64] = t < 67 ? 0x7fffffff : -0x7fffffff;
+    __syncthreads();
+    const int count = s_off[kUnitRows];
+    // particle of task i: the last row with s_off <= i
+    auto particle = [&](int i) {
+        int r = 0;
+#pragma unroll
+        for (int o = kUnitRows / 2; o > 0; o >>= 1) r += s_off[r + o] <= i ? o : 0;
+        return s_first[r] + i;
+    };
     const double inv = 1.0 / k.spacing;
     {
         int mn[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff};
         int mx[3] = {-0x7fffffff, -0x7fffffff, -0x7fffffff};
-        for (int p = ch.x + t; p < ch.y; p += kGradThreads) {
-            const double4 q = rpos[p];
+        for (int i = t; i < count; i += kGradThreads) {
+            const double4 q = rpos[particle(i)];
             const double qc[3] = {q.x, q.y, q.z};
 #pragma unroll
             for (int a = 0; a < 3; a++) {
@@ -292,7 +339,7 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
     const int64_t e2 = (int64_t)s_box[5] - s_box[2] + 8;
     if (e0 * e1 * e2 > kGradCap) {
         // particles far outside their cells: left to k_gradient_overflow
-        if (!CNT && t == 0) over[atomicAdd(nover, 1)] = chunk;
+        if (!CNT && t == 0) over[atomicAdd(nover, 1)] = unit;
         return;
     }
     // the bricks the box touches (floor division by 8, also below zero)
@@ -300,8 +347,8 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
     const int nbx = ((lo0 + (int)e0 - 1) >> 3) - bx0 + 1;
     const int nby = ((lo1 + (int)e1 - 1) >> 3) - by0 + 1;
     const int nbz = ((lo2 + (int)e2 - 1) >> 3) - bz0 + 1;
-    if (nbx * nby * nbz > kGradBoxBricks) {   // (a box of at most 108 bricks fits)
-        if (!CNT && t == 0) over[atomicAdd(nover, 1)] = chunk;
+    if (nbx * nby * nbz > kGradBoxBricks) {
+        if (!CNT && t == 0) over[atomicAdd(nover, 1)] = unit;
         return;
     }
     // their slots (-1 off the virtual set or off the lattice) in one round
@@ -314,42 +361,39 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
         s_bslot[i] = sl;
     }
     __syncthreads();
+    const int n0 = (int)e0, n1 = (int)e1;
     {
-        // one wave per box row (iy, iz), lanes along x; four rows per pass,
-        // their loads issued together (no branch between them: an invalid
-        // node reads q[0] and keeps 0)
-        constexpr int kW = kGradThreads / 64;
-        const int n0 = (int)e0, n1 = (int)e1, nrow = (int)(e1 * e2);
-        const int lane = t & 63;
-        for (int rw0 = t >> 6; rw0 < nrow; rw0 += 4 * kW) {
-            for (int ix = lane; ix < n0; ix += 64) {
-                const int gx = lo0 + ix;
-                const bool x_in = gx >= 0 && gx < k.ndims[0];
-                const int bxi = (gx >> 3) - bx0;
-                float v[4];
+        // the box's nodes in turn, four loads of a thread issued together (no
+        // branch between them: an invalid node reads q[0] and keeps 0); a
+        // node's place from its number by two multiplications (m = 2^32 / d
+        // rounded up is exact for numbers below 2^16 by divisors below 2^16)
+        const int total = n0 * n1 * (int)e2;
+        const uint32_t m0 = 0xffffffffu / (uint32_t)n0 + 1u;
+        const uint32_t m1 = 0xffffffffu / (uint32_t)n1 + 1u;
+        for (int i0 = t; i0 < total; i0 += 4 * kGradThreads) {
+            float v[4];
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const int rw = rw0 + u * kW;
-                    const int iy = rw % n1, iz = rw / n1;
-                    const int gy = lo1 + iy, gz = lo2 + iz;
-                    const bool in = x_in && rw < nrow && gy >= 0 && gz >= 0 &&
-                                    gy < k.ndims[1] && gz < k.ndims[2];
-                    const int bi = in ? (((gz >> 3) - bz0) * nby + ((gy >> 3) - by0)) * nbx + bxi
-                                      : 0;
-                    const int sl = s_bslot[bi];
-                    const bool ok = in && sl >= 0;
-                    const int64_t g = ok ? (int64_t)sl * 512 + ((gz & 7) << 6) +
-                                               ((gy & 7) << 3) + (gx & 7)
-                                         : 0;
-                    const float q = vq[g];
-                    v[u] = ok ? q : 0.f;
-                }
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const int rw = rw0 + u * kW;
-                    if (rw < nrow) s_q[rw * n0 + ix] = v[u];
-                }
+            for (int u = 0; u < 4; u++) {
+                const uint32_t i = i0 + u * kGradThreads;
+                const uint32_t rw = __umulhi(i, m0), iz = __umulhi(rw, m1);
+                const int gx = lo0 + (int)(i - rw * n0), gy = lo1 + (int)(rw - iz * n1),
+                          gz = lo2 + (int)iz;
+                const bool in = (int)i < total && gx >= 0 && gy >= 0 && gz >= 0 &&
+                                gx < k.ndims[0] && gy < k.ndims[1] && gz < k.ndims[2];
+                const int bi = in ? (((gz >> 3) - bz0) * nby + ((gy >> 3) - by0)) * nbx +
+                                        ((gx >> 3) - bx0)
+                                  : 0;
+                const int sl = s_bslot[bi];
+                const bool ok = in && sl >= 0;
+                const int64_t g = ok ? (int64_t)sl * 512 + ((gz & 7) << 6) + ((gy & 7) << 3) +
+                                           (gx & 7)
+                                     : 0;
+                const float q = vq[g];
+                v[u] = ok ? q : 0.f;
             }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (i0 + u * kGradThreads < total) s_q[i0 + u * kGradThreads] = v[u];
         }
     }
     __syncthreads();
@@ -363,9 +407,10 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
     // The clamps fold into the fmas; c1 is applied once per particle.
     const float c1 = k.c1H;
     const double iHd = 1.0 / k.H;
-    for (int p0 = ch.x; p0 < ch.y; p0 += kGradThreads) {
-        const int p = p0 + t;
-        if (p >= ch.y) break;
+    constexpr int kC = 8 / L;   // x candidates of a lane
+    const int sub = L > 1 ? t % L : 0;
+    for (int i = t / L; i < count; i += kGradThreads / L) {   // uniform over the lanes of a particle
+        const int p = particle(i);
         const double4 q = rpos[p];
         const float4 vi = rvel[p];
         float fx = 0.f, fy = 0.f, fz = 0.f;
@@ -374,10 +419,17 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
             const int f0 = node_floor(q.x, k.origin[0], inv);
             const int f1 = node_floor(q.y, k.origin[1], inv);
             const int f2 = node_floor(q.z, k.origin[2], inv);
-            float dxf[8], dx2[8];   // x offsets of the 8 candidates, in units of H
+            // x candidate of this lane's c-th: the pairs (P, 7 - P) in turn
+            auto cand = [&](int c) {
+                if constexpr (L == 8) return sub;
+                const int P = sub + (c >> 1) * L;
+                return (c & 1) ? 7 - P : P;
+            };
+            float dxf[kC], dx2[kC];   // x offsets of the lane's candidates, in units of H
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                dxf[c] = (float)(dsub(node_coord(k.origin[0], f0 - 3 + c, k.spacing), q.x) * iHd);
+            for (int c = 0; c < kC; c++) {
+                dxf[c] = (float)(dsub(node_coord(k.origin[0], f0 - 3 + cand(c), k.spacing), q.x) *
+                                 iHd);
                 // + 1e-30: rsq stays finite at a coincident node (whose
                 // direction factors are all zero)
                 dx2[c] = dxf[c] * dxf[c] + 1e-30f;
@@ -386,14 +438,14 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
             const float dy0 = (float)(dsub(node_coord(k.origin[1], f1 - 3, k.spacing), q.y) * iHd);
             const float dz0 = (float)(dsub(node_coord(k.origin[2], f2 - 3, k.spacing), q.z) * iHd);
             const float sf = (float)(k.spacing * iHd);
-            const int n0 = (int)e0, n1 = (int)e1;
             const float* base = s_q + ((f2 - 3 - lo2) * n1 + (f1 - 3 - lo1)) * n0 + (f0 - 3 - lo0);
             // Candidate c of row (cy, cz) is node f - 3 + c: its offset from x
             // lies in (c - 4, c - 3] s.  With d(c) = the smallest |offset| of
             // index c (3, 2, 1, 0, 0, 1, 2, 3) a row holds members only if
             // d(cy)^2 + d(cz)^2 < 16, and only at |c - 3.5| < sqrt(R2) + 0.5,
             // R2 = 16 - d(cy)^2 - d(cz)^2: all 8 for R2 >= 11, c = 1..6 for
-            // R2 = 6..8, c = 2..5 for R2 = 3 (the uniform bounds below).  The
+            // R2 = 6..8, c = 2..5 for R2 = 3 (the uniform bounds below; the
+            // first pairs of a lane go when no lane's candidate is in).  The
             // whole 8 x 8 row nest is unrolled: the bounds are constants, and
             // the LDS reads are scheduled ahead of the candidates that use them.
 #pragma unroll
@@ -413,16 +465,18 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
                     const float* row = plane + cy * n0;
                     float sx = 0.f, ss = 0.f;
 #pragma unroll
-                    for (int c = 0; c < 8; c++) {
-                        if (c < cut || c > 7 - cut) continue;   // uniform
+                    for (int c = 0; c < kC; c++) {
+                        // the largest pair any lane has here: (c / 2) L + L - 1
+                        if (L < 8 && (c >> 1) * L + L - 1 < cut) continue;   // uniform
+                        const float qv = row[cand(c)];
                         const float w = dx2[c] + dyz;
                         const float u = __builtin_amdgcn_rsqf(w);
                         const float a = __builtin_amdgcn_fmed3f(fmaf(-w, u, 1.f), 0.f, 1.f);
                         const float b = __builtin_amdgcn_fmed3f(fmaf(a, 2.f, -1.f), 0.f, 1.f);
-                        const float sc = row[c] * u * fmaf(a, a, -(b * b));
+                        const float sc = qv * u * fmaf(a, a, -(b * b));
                         sx = fmaf(sc, dxf[c], sx);
                         ss += sc;
-                        if constexpr (CNT) nterms += (a > 0.f) & (row[c] > 0.f);
+                        if constexpr (CNT) nterms += (a > 0.f) & (qv > 0.f);
                     }
                     fx -= sx;
                     fy -= ss * dyc;
@@ -437,7 +491,14 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
             members[p] = nterms;
             continue;
         }
-        if (s_walls) boundary_term<3>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz);
+        if (s_walls) boundary_term<3, L>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz, sub);
+#pragma unroll
+        for (int o = 1; o < L; o <<= 1) {
+            fx += __shfl_xor(fx, o, 64);
+            fy += __shfl_xor(fy, o, 64);
+            fz += __shfl_xor(fz, o, 64);
+        }
+        if (sub != 0) continue;
         float4 v = vi;
         v.x += fx;
         v.y += fy;
@@ -519,46 +580,78 @@ __global__ void __launch_bounds__(128) k_query(
 
 }  // namespace
 
+// Lanes per particle and cells of a work unit by the number of particles: the
+// fewest lanes and the largest unit (least staged per particle: 77, 22 and 10
+// nodes) that fill the machine.  us of one launch that updates, 2x2x2 cells
+// with 8 lanes, 4x2x2 with 4, 4x4x4 with 1 (before: spans of 25 cells of one
+// row, 36 nodes staged per particle, one lane each):
+//   500 particles 19, 24, 42 (45)     32,000 23, 24, 41 (44)
+//   64,000        34, 29, 43 (50)    100,000 41, 34, 48 (61)
+// and by the launches of a run that update and those that do not, 4x2x2 and 4x4x4:
+//   212,503 24, 27 (33)    300,000 23, 23 (31)    1,012,500 122, 102 (146)
+struct UnitRule {
+    int lanes, u[3];
+};
+static UnitRule unit_rule(int64_t n) {
+    if (n <= 32000) return {8, {2, 2, 2}};
+    if (n <= 250000) return {4, {4, 2, 2}};
+    return {1, {4, 4, 4}};
+}
+
+// The rule's unit, shrunk until its node box fits the stage; false if not even
+// one cell's does.
+static bool unit_shape(const KConst& k, int64_t n, int u[3]) {
+    const UnitRule rule = unit_rule(n);
+    for (int a = 0; a < 3; a++) u[a] = rule.u[a];
+    const double ratio = k.cell_size / k.spacing;
+    auto nodes = [&](int m) { return (int64_t)std::floor(m * ratio) + 9; };
+    while (nodes(u[0]) * nodes(u[1]) * nodes(u[2]) > kGradCap) {
+        int* largest = std::max_element(u, u + 3);
+        if (--*largest < 1) return false;
+    }
+    return true;
+}
+
 int gradient_setup(vps_context* c) {
-    c->grad_span_cells = 0;
+    c->grad_staged = false;
     if (c->dim != 3) return VPS_OK;
     const KConst& k = c->k;
     // candidates f-3 .. f+4 per axis assume H = 4 s
     if (!(std::fabs(k.H - 4.0 * k.spacing) <= 1e-12 * k.H)) return VPS_OK;
-    const double ratio = k.cell_size / k.spacing;
-    const int64_t eyz = (int64_t)std::floor(ratio) + 9;   // box extent along y, z
-    const double room = (double)kGradCap / (double)(eyz * eyz) - 9.0;
-    int span = (int)std::floor(room / ratio);
-    if (span < 1) return VPS_OK;
-    if (span > k.cdims[0]) span = k.cdims[0];
-    c->grad_span_cells = span;
-    c->grad_nspan = (k.cdims[0] + span - 1) / span;
-    const int64_t nrows = (int64_t)k.cdims[1] * k.cdims[2];
-    VPS_TRY(dalloc(c, c->grad_chunks, (size_t)(nrows * c->grad_nspan)));
-    VPS_TRY(dalloc(c, c->grad_over, (size_t)(nrows * c->grad_nspan)));
+    int u[3];
+    if (!unit_shape(k, 0, u)) return VPS_OK;
+    int64_t total = 1;   // of the smallest units
+    for (int a = 0; a < 3; a++) total *= (k.cdims[a] + u[a] - 1) / u[a];
+    VPS_TRY(dalloc(c, c->grad_units, (size_t)total));
+    VPS_TRY(dalloc(c, c->grad_over, (size_t)total));
+    c->grad_staged = true;
     return VPS_OK;
 }
 
-SpanArgs gradient_span_args(vps_context* c, bool append) {
-    SpanArgs a{};
-    if (!append || c->grad_span_cells <= 0) return a;
-    a.total = (int64_t)c->k.cdims[1] * c->k.cdims[2] * c->grad_nspan;
-    a.span_cells = c->grad_span_cells;
-    a.nspan = c->grad_nspan;
+UnitArgs gradient_units(vps_context* c, bool append) {
+    if (!append || !c->grad_staged) return UnitArgs{};
+    UnitArgs a{};
+    (void)unit_shape(c->k, c->n, a.u);
+    a.total = 1;
+    for (int d = 0; d < 3; d++) {
+        a.nu[d] = (c->k.cdims[d] + a.u[d] - 1) / a.u[d];
+        a.total *= a.nu[d];
+    }
     a.cstart = c->cell_start.p;
-    a.chunks = c->grad_chunks.p;
+    a.units = c->grad_units.p;
     a.count = (int32_t*)(c->counters.p + 2);
+    c->grad_shape = a;
     return a;
 }
 
 // Terms of the staged gradient's virtual walk per real particle (test
-// support, sorted order; -1 stays where a span exceeds the stage).
+// support, sorted order; -1 stays where a unit exceeds the stage).
 int gradient_member_counts(vps_context* c, int32_t* members) {
-    if (c->dim != 3 || c->grad_span_cells <= 0 || c->nslots == 0) return VPS_ERR_INVALID_ARG;
-    if (c->grad_nchunks > 0)
-        hipLaunchKernelGGL(k_gradient3s<true>, dim3((unsigned)c->grad_nchunks),
-                           dim3(kGradThreads), 0, c->stream, c->k, c->grad_chunks.p,
-                           (int)c->grad_nchunks, c->rpos[c->cur].p, c->rvel[c->cur].p,
+    if (c->dim != 3 || !c->grad_staged || c->nslots == 0) return VPS_ERR_INVALID_ARG;
+    if (c->grad_nunits > 0)
+        hipLaunchKernelGGL((k_gradient3s<1, true>), dim3((unsigned)c->grad_nunits),
+                           dim3(kGradThreads), 0, c->stream, c->k, c->grad_shape,
+                           (int)c->grad_nunits, c->rpos[c->cur].p, c->rvel[c->cur].p,
                            c->brick_slot[c->which].p, c->vvol.p, c->bpos.p, c->bvel.p,
                            c->bnrm.p, c->bcell_start.p, (int32_t*)nullptr,
                            (int32_t*)nullptr, SolveGuard{}, members);
@@ -570,17 +663,23 @@ int pressure_gradient(vps_context* c, SolveGuard g) {
     const int64_t n = c->n;
     const int s = c->cur;
     const int w = c->which;
-    if (c->dim == 3 && c->grad_span_cells > 0) {
-        if (c->grad_nchunks > 0) {
-            int32_t* nover = (int32_t*)(c->counters.p + 3);   // zeroed with the spans
+    if (c->dim == 3 && c->grad_staged) {
+        if (c->grad_nunits > 0) {
+            int32_t* nover = (int32_t*)(c->counters.p + 3);   // zeroed with the units
             int32_t* over = c->grad_over.p;
-            hipLaunchKernelGGL(k_gradient3s<false>, dim3((unsigned)c->grad_nchunks),
-                               dim3(kGradThreads), 0, c->stream, c->k,
-                               c->grad_chunks.p, (int)c->grad_nchunks, c->rpos[s].p,
-                               c->rvel[s].p, c->brick_slot[w].p, c->vq.p, c->bpos.p,
-                               c->bvel.p, c->bnrm.p, c->bcell_start.p, over, nover, g);
+            auto run = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3((unsigned)c->grad_nunits), dim3(kGradThreads), 0,
+                                   c->stream, c->k, c->grad_shape, (int)c->grad_nunits,
+                                   c->rpos[s].p, c->rvel[s].p, c->brick_slot[w].p, c->vq.p,
+                                   c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, over,
+                                   nover, g, (int32_t*)nullptr);
+            };
+            const int lanes = unit_rule(n).lanes;
+            if (lanes == 8) run(k_gradient3s<8>);
+            else if (lanes == 4) run(k_gradient3s<4>);
+            else run(k_gradient3s<1>);
             hipLaunchKernelGGL(k_gradient_overflow, dim3(64), dim3(kGradThreads), 0,
-                               c->stream, c->k, c->grad_chunks.p, over, nover,
+                               c->stream, c->k, c->grad_shape, over, nover,
                                c->rpos[s].p, c->rvel[s].p, c->brick_slot[w].p, c->vq.p,
                                c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, g);
         }

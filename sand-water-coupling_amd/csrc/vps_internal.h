@@ -330,24 +330,46 @@ inline int walk_lanes(int64_t n) {
     return n <= 32000 ? 8 : (n <= 400000 ? 4 : (n <= 900000 ? 2 : 1));
 }
 
-// Work units of the 3D gradient: spans of up to span_cells consecutive cells
-// of one cell row.  Thread i appends span i when it holds particles.
-struct SpanArgs {
+// Work units of the 3D gradient: blocks of u[0] x u[1] x u[2] cells (at most
+// kUnitRows rows of cells, each a contiguous range of the sorted particles).
+// Thread i appends unit i when it holds particles.
+constexpr int kUnitRows = 16;
+struct UnitArgs {
     int64_t total = 0;
-    int span_cells = 0, nspan = 0;
+    int u[3] = {1, 1, 1}, nu[3] = {0, 0, 0};   // cells of a unit, units per axis
     const int32_t* cstart = nullptr;
-    int4* chunks = nullptr;   // particle range, cell range
+    int32_t* units = nullptr;   // numbers of the units with particles
     int32_t* count = nullptr;
 };
-__device__ __forceinline__ void span_append(const KConst& k, const SpanArgs& a, int64_t i) {
+// The cells of a unit: first cell and number per axis (the last units of an
+// axis may be cut off).
+struct UnitCells {
+    int c[3], m[3];
+    __device__ __forceinline__ UnitCells(const KConst& k, const UnitArgs& a, int64_t i) {
+        const int64_t q = i / a.nu[0];
+        const int at[3] = {(int)(i - q * a.nu[0]), (int)(q % a.nu[1]), (int)(q / a.nu[1])};
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            c[d] = at[d] * a.u[d];
+            m[d] = min(a.u[d], k.cdims[d] - c[d]);
+        }
+    }
+    __device__ __forceinline__ int rows() const { return m[1] * m[2]; }
+    // first cell of row r
+    __device__ __forceinline__ int64_t row(const KConst& k, int r) const {
+        return ((int64_t)(c[2] + r / m[1]) * k.cdims[1] + c[1] + r % m[1]) * k.cdims[0] + c[0];
+    }
+};
+__device__ __forceinline__ void unit_append(const KConst& k, const UnitArgs& a, int64_t i) {
     if (i >= a.total) return;
-    const int64_t row = i / a.nspan;
-    const int sp = (int)(i - row * a.nspan);
-    const int64_t c0 = row * k.cdims[0] + (int64_t)sp * a.span_cells;
-    const int e = (sp + 1) * a.span_cells < k.cdims[0] ? (sp + 1) * a.span_cells : k.cdims[0];
-    const int64_t c1 = row * k.cdims[0] + e;
-    const int b = a.cstart[c0], f = a.cstart[c1];
-    if (f > b) a.chunks[atomicAdd(a.count, 1)] = make_int4(b, f, (int)c0, (int)c1);
+    const UnitCells uc(k, a, i);
+    int any = 0;
+#pragma unroll
+    for (int r = 0; r < kUnitRows; r++) {   // all loads in flight together
+        const int64_t g = uc.row(k, min(r, uc.rows() - 1));
+        any |= a.cstart[g + uc.m[0]] - a.cstart[g];
+    }
+    if (any) a.units[atomicAdd(a.count, 1)] = (int32_t)i;
 }
 
 // ---- reductions ----------------------------------------------------------
@@ -513,11 +535,11 @@ struct vps_context {
     // cell-sorted boundary, 3D: FP32 offset from the cell corner, w = +-1/rho_b
     // (negative: clamped into a border cell, exact test only)
     vps::DBuf<float4> bofs;
-    vps::DBuf<int4> grad_chunks;        // 3D gradient: particle and cell ranges of spans
-    vps::DBuf<int32_t> grad_over;       // spans left to the global-memory path
-    int grad_span_cells = 0;            // cells per span (0: global-memory gradient)
-    int grad_nspan = 0;                 // spans per cell row
-    int64_t grad_nchunks = 0;           // non-empty spans of the last generation
+    vps::DBuf<int32_t> grad_units;      // 3D gradient: units that hold particles
+    vps::DBuf<int32_t> grad_over;       // units left to the global-memory path
+    bool grad_staged = false;           // false: global-memory gradient
+    vps::UnitArgs grad_shape;           // units of the last generation
+    int64_t grad_nunits = 0;            // and how many of them hold particles
     vps::DBuf<float4> vel_next;         // velocities after a Jacobi pass (DEM, viscosity)
     vps::DBuf<double> couple_stage;     // grain coupling: boundary x, n, v
     int64_t couple_walls = -1;          // walls already staged there (-1: none)
@@ -645,10 +667,10 @@ void dfree(DBuf<T>& b) {
 }
 
 // launchers (defined in the .hip files)
-// 3D gradient set-up at creation: span length and the span list buffer
+// 3D gradient set-up at creation: whether it is staged, and the list buffers
 int gradient_setup(vps_context* c);
-// the spans of the current sort for span_append (total 0: none to append)
-SpanArgs gradient_span_args(vps_context* c, bool append);
+// the units of the current sort for unit_append (total 0: none to append)
+UnitArgs gradient_units(vps_context* c, bool append);
 // exclusive scan of in into out (out may alias in); clear_in (== in, not
 // aliased with out) zeroes the input once read
 int scan_exclusive_i32(vps_context* c, const int32_t* in, int32_t* out,

@@ -36,12 +36,12 @@ template <int D>
 __global__ void __launch_bounds__(256) k_mark_bricks(const double4* pos,
                                                      int64_t n, KConst k,
                                                      uint32_t* flag, uint32_t* bits,
-                                                     int64_t nwords, int32_t* span_count) {
+                                                     int64_t nwords, int32_t* unit_count) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     for (int64_t w = i; w < nwords; w += (int64_t)gridDim.x * 256) bits[w] = 0u;
-    if (i == 0) {   // the gradient's span and overflow lists are rebuilt next
-        span_count[0] = 0;
-        span_count[2] = 0;
+    if (i == 0) {   // the gradient's unit and overflow lists are rebuilt next
+        unit_count[0] = 0;
+        unit_count[2] = 0;
     }
     if (i >= n) return;
     const double4 p = pos[i];
@@ -715,15 +715,15 @@ struct StoreColumn {
 // Tables over the slots of one generation, in one launch: the slots of the
 // 3^D neighbour bricks of every slot (zero brick if absent), and in 3D the
 // column order, order[off[column] + active bricks below] = slot (by the thread
-// of the middle neighbour), and the gradient's spans (by the first threads;
-// see span_append).
+// of the middle neighbour), and the gradient's units (by the first threads;
+// see unit_append).
 template <int D>
 __global__ void __launch_bounds__(256) k_slot_tables(
     KConst k, const int32_t* brick_of_slot, const int32_t* slot_of_brick, const int32_t* nslots_p,
-    int64_t grid, int32_t zero, int32_t* nbr, const int32_t* off, int32_t* order, SpanArgs sp) {
+    int64_t grid, int32_t zero, int32_t* nbr, const int32_t* off, int32_t* order, UnitArgs ua) {
     constexpr int NN = D == 3 ? 27 : 9;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if constexpr (D == 3) span_append(k, sp, i);
+    if constexpr (D == 3) unit_append(k, ua, i);
     const int32_t nsl = *nslots_p;
     // the grid may exceed the slot count; a count beyond the grid leaves the
     // tables to the rerun on the exact grid
@@ -848,7 +848,7 @@ __global__ void __launch_bounds__(256) k_after_solve(int64_t nnode,
 
 // Slot-indexed passes of one generation on a grid of `grid` blocks (slots);
 // blocks at or beyond the device-side slot count return at once.  first: not a
-// rerun on the exact grid (the gradient's spans are appended once).
+// rerun on the exact grid (the gradient's units are appended once).
 static int generate_slots(vps_context* c, int w, int64_t grid, bool first) {
     const int D = c->dim;
     const int rs = c->cur;
@@ -883,14 +883,14 @@ static int generate_slots(vps_context* c, int w, int64_t grid, bool first) {
         // (one column per thread: each is a loop of its own)
         VPS_TRY(scan_launch_as<1>(c, LoadColumn{plane, c->k.bdims[2], sob},
                                   StoreColumn{c->col_off.p}, plane, nullptr));
-        const SpanArgs sp = gradient_span_args(c, first);
-        hipLaunchKernelGGL(k_slot_tables<3>, dim3(blocks(std::max(grid * 27, sp.total), 256)),
+        const UnitArgs ua = gradient_units(c, first);
+        hipLaunchKernelGGL(k_slot_tables<3>, dim3(blocks(std::max(grid * 27, ua.total), 256)),
                            dim3(256), 0, c->stream, c->k, bos, sob, nsl, grid,
-                           (int32_t)c->nbricks, c->nbr_slot.p, c->col_off.p, c->col_order.p, sp);
+                           (int32_t)c->nbricks, c->nbr_slot.p, c->col_off.p, c->col_order.p, ua);
     } else
         hipLaunchKernelGGL(k_slot_tables<2>, dim3(blocks(grid * 9, 256)), dim3(256), 0, c->stream,
                            c->k, bos, sob, nsl, grid, (int32_t)c->nbricks, c->nbr_slot.p,
-                           (const int32_t*)nullptr, (int32_t*)nullptr, SpanArgs{});
+                           (const int32_t*)nullptr, (int32_t*)nullptr, UnitArgs{});
     VPS_TRY(scan_launch(c, LoadPopc{c->bits.p}, StorePrefix{(int32_t*)c->word_prefix.p}, c->nwords,
                         (int32_t*)(dcnt + 1)));
     if (D == 3)
@@ -904,7 +904,7 @@ static int generate_slots(vps_context* c, int w, int64_t grid, bool first) {
                            nsl, c->vvol.p, c->bits.p,
                            (const int32_t*)c->word_prefix.p, c->vrank.p);
     VPS_HIP(c, hipGetLastError());
-    // slot, virtual and gradient-span counts in one read-back
+    // slot, virtual and gradient-unit counts in one read-back
     VPS_HIP(c, hipMemcpyAsync(c->host_counters, dcnt, 24, hipMemcpyDeviceToHost,
                               c->stream));
     VPS_HIP(c, hipStreamSynchronize(c->stream));
@@ -957,7 +957,7 @@ int virtual_generate(vps_context* c) {
     c->nslots = nslots;
     c->which = w;
     c->nvirt = nslots ? *(int32_t*)(c->host_counters + 1) : 0;
-    c->grad_nchunks = *(int32_t*)(c->host_counters + 2);
+    c->grad_nunits = *(int32_t*)(c->host_counters + 2);
     return VPS_OK;
 }
 
