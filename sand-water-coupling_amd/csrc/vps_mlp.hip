@@ -70,6 +70,14 @@ enum {
 };
 constexpr int kTrainBlocks = 256;               // one block of 4 waves per CU
 constexpr int kTrainWaves = 4 * kTrainBlocks;
+// Tiles of 16 samples per training wave, and the blocks that have any (the
+// partials of the others need neither writing nor adding).
+struct TrainShape {
+    int tiles, blocks;
+    explicit TrainShape(int64_t n)
+        : tiles((int)((n + 16 * kTrainWaves - 1) / (16 * kTrainWaves))),
+          blocks((int)((n + 64 * (int64_t)tiles - 1) / (64 * (int64_t)tiles))) {}
+};
 // largest batch of vps_mlp_loss_and_grad(_device): 4,096 tiles of 16 samples
 // per training wave
 constexpr int64_t kMaxLossBatch = (int64_t)16 * kTrainWaves * 4096;
@@ -128,11 +136,13 @@ __device__ __forceinline__ void load_weights(const float* P, Wregs& W) {
     for (int mt = 0; mt < 4; mt++) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int k = 4 * q + j;
-            W.w1[mt][j] = k < kIn ? f2bf(P[OFF_W1 + (mt * 16 + r) * kIn + k]) : (short)0;
+            // (selects on the values, not branches around the loads)
+            const short w1 = f2bf(P[OFF_W1 + (mt * 16 + r) * kIn + 4 * (q & 1) + j]);
+            const short w3 = f2bf(P[OFF_W3 + mt * 16 + 4 * q + j]);
+            W.w1[mt][j] = q < 2 ? w1 : (short)0;
             W.b1[mt][j] = P[OFF_B1 + mt * 16 + 4 * q + j];
             W.b2[mt][j] = P[OFF_B2 + mt * 16 + 4 * q + j];
-            W.w3[mt][j] = r == 0 ? f2bf(P[OFF_W3 + mt * 16 + 4 * q + j]) : (short)0;
+            W.w3[mt][j] = r == 0 ? w3 : (short)0;
         }
         if constexpr (W2REG) {
 #pragma unroll
@@ -152,13 +162,26 @@ struct Fwd {
     float out;   // lanes 0..15: output of node l
 };
 
+// Row strides (in bf16) of the LDS copies: 8-byte reads by 16 rows x 4 groups
+// of 4 columns fall on distinct banks (strides of 34 and 10 banks; with the
+// plain 64 and 16 columns the 16 rows share 2 and 8 of the 64 banks).
+constexpr int kWS = kHid + 4;   // W2, W2^T: hidden columns
+constexpr int kNS = 16 + 4;     // staged activations: node columns
+
 // W2 A tile (m-tile mo, k-tile kt) read from an LDS copy W2[out][in] (bf16)
 __device__ __forceinline__ bf16x4 w2_tile(const uint16_t* sW, int mo, int kt) {
     const int l = threadIdx.x & 63, r = l & 15, q = l >> 4;
-    const uint16_t* p = sW + (mo * 16 + r) * kHid + kt * 16 + 4 * q;
-    bf16x4 v;
-#pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = (short)p[j];
+    return *reinterpret_cast<const bf16x4*>(sW + (mo * 16 + r) * kWS + kt * 16 + 4 * q);
+}
+// sum over the 16 lanes of a row of the wave, in every lane
+__device__ __forceinline__ float row_sum(float v) {
+#define VPS_DPP_ADD(ctrl) \
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ctrl, 0xf, 0xf, false))
+    VPS_DPP_ADD(0xb1);    // quad_perm [1, 0, 3, 2]
+    VPS_DPP_ADD(0x4e);    // quad_perm [2, 3, 0, 1]
+    VPS_DPP_ADD(0x141);   // row_half_mirror
+    VPS_DPP_ADD(0x140);   // row_mirror
+#undef VPS_DPP_ADD
     return v;
 }
 
@@ -536,41 +559,88 @@ __device__ __forceinline__ uint64_t mix64(uint64_t x) {
 // Per wave: tiles_per_wave tiles of 16 samples.  The 4 waves of a block sum
 // their gradients through LDS (fixed order); the block writes one row of
 // kNParams floats and its loss partial.  Loss = sum (out - t)^2 / nsamples.
+// One block per CU (the accumulators and activations take the registers of
+// one wave per SIMD), so what counts is one wave's chain: the parameters come
+// in once, coalesced, and become register tiles from LDS; W2, W2^T and the
+// staged activations are read 8 bytes at a time from rows padded off the same
+// banks; the next tile's samples load while one is computed; a wave waits for
+// itself only; lane sums go by DPP.  65,536 samples: 19.6 us (before 39.9), 24
+// samples: 9.9 (before 24.9), 1,000,000: 142 (before 334; about 920 instructions a tile).
 template <bool DIRECT>
 __global__ void __launch_bounds__(256) k_mlp_train(
     const float* P, FeatSrc fs, const float* vx, const int32_t* slot_of_rank,
     int64_t nv, const float* fdirect, const float* tdirect, int64_t nsamples,
     int tiles_per_wave, uint64_t seed, float* grad_part, double* loss_part) {
-    // per-wave bf16 staging tiles; reused as the FP32 gradient exchange of
-    // the block reduction (2 x kNParams floats) after the sample loop
-    constexpr int kTileBytes = 4 * (3 * kHid * 16 + 16 * 16) * 2;
-    constexpr int kRedBytes = 2 * kNParams * 4;
+    // the parameters at first; then per-wave bf16 staging tiles; after the
+    // sample loop the FP32 gradients of the four waves (kNParams floats each)
+    constexpr int kWaveStage = (3 * kHid + 16) * kNS;   // bf16 of one wave
+    constexpr int kTileBytes = 4 * kWaveStage * 2;
+    constexpr int kRedBytes = 4 * kNParams * 4;
     constexpr int kStageBytes = kTileBytes > kRedBytes ? kTileBytes : kRedBytes;
     __shared__ __align__(16) uint8_t s_stage[kStageBytes];
     __shared__ double s_loss[4];
-    auto s_dz2 = reinterpret_cast<uint16_t(*)[kHid * 16]>(s_stage);
-    auto s_h1 = reinterpret_cast<uint16_t(*)[kHid * 16]>(s_stage + 4 * kHid * 16 * 2);
-    auto s_dz1 = reinterpret_cast<uint16_t(*)[kHid * 16]>(s_stage + 8 * kHid * 16 * 2);
-    auto s_x = reinterpret_cast<uint16_t(*)[16 * 16]>(s_stage + 12 * kHid * 16 * 2);
     float* s_red = reinterpret_cast<float*>(s_stage);
-    __shared__ uint16_t sW2[kHid * kHid];    // W2[out][in]
-    __shared__ uint16_t sW2T[kHid * kHid];   // W2^T[in][out]
+    __shared__ __align__(16) uint16_t sW2[kHid * kWS];    // W2[out][in]
+    __shared__ __align__(16) uint16_t sW2T[kHid * kWS];   // W2^T[in][out]
     const int lane = threadIdx.x & 63, r = lane & 15, q = lane >> 4;
     const int wl = threadIdx.x >> 6;
+    uint16_t* s_dz2 = reinterpret_cast<uint16_t*>(s_stage) + wl * kWaveStage;
+    uint16_t* s_h1 = s_dz2 + kHid * kNS;
+    uint16_t* s_dz1 = s_h1 + kHid * kNS;
+    uint16_t* s_x = s_dz1 + kHid * kNS;
     const int64_t wave = (int64_t)blockIdx.x * 4 + wl;
-    for (int e = threadIdx.x; e < kHid * kHid; e += 256) {
-        const uint16_t b = (uint16_t)f2bf(P[OFF_W2 + e]);
-        sW2[e] = b;
-        sW2T[(e % kHid) * kHid + e / kHid] = b;
+    // One tile's samples: the features of this lane's node and its target.
+    struct Sample {
+        float f[4];
+        float target;
+        bool ok;
+    };
+    auto load_sample = [&](int it, Sample& S) {
+        const int64_t k = (wave * tiles_per_wave + it) * 16 + r;   // sample id
+        S.ok = it < tiles_per_wave && k < nsamples;
+        int64_t node = k;
+        S.target = 0.f;
+        if constexpr (DIRECT) {
+            if (S.ok) S.target = tdirect[k];
+        } else {
+            // uniform over the virtual particles of this solve
+            node = S.ok ? slot_of_rank[mix64(seed ^ (uint64_t)k) % (uint64_t)nv] : 0;
+            const int h = fs.hh[node];
+            S.ok = S.ok && h >= 1;
+            if (S.ok)
+                S.target = (vx[node] - fs.p1[node] - prior(h, fs.dp1[node], fs.dp2[node])) *
+                           fs.scale[SC_INV_TAU];
+        }
+        (void)tile_features<DIRECT>(fs, fdirect, nsamples, node, S.ok, S.f);
+    };
+    Sample next;
+    load_sample(0, next);
+    {
+        constexpr int kLoads = (kNParams + 255) / 256;
+        float pv[kLoads];
+#pragma unroll
+        for (int u = 0; u < kLoads; u++) pv[u] = P[min((int)threadIdx.x + 256 * u, kNParams - 1)];
+#pragma unroll
+        for (int u = 0; u < kLoads; u++) {
+            const int i = threadIdx.x + 256 * u, e = i - OFF_W2;
+            if (i < kNParams) s_red[i] = pv[u];
+            if (e >= 0 && e < kHid * kHid) {
+                const uint16_t b = (uint16_t)f2bf(pv[u]);
+                sW2[(e / kHid) * kWS + e % kHid] = b;
+                sW2T[(e % kHid) * kWS + e / kHid] = b;
+            }
+        }
     }
+    __syncthreads();
     Wregs W;
-    load_weights<false>(P, W);
+    load_weights<false>(s_red, W);
     // W3 in C layout
     f32x4 w3c[4];
 #pragma unroll
     for (int mi = 0; mi < 4; mi++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) w3c[mi][i] = bf2f(f2bf(P[OFF_W3 + mi * 16 + 4 * q + i]));
+        for (int i = 0; i < 4; i++)
+            w3c[mi][i] = bf2f(f2bf(s_red[OFF_W3 + mi * 16 + 4 * q + i]));
     __syncthreads();
     f32x4 gW2[4][4], gW1[4], gb1[4], gb2[4], gW3[4];
 #pragma unroll
@@ -585,25 +655,20 @@ __global__ void __launch_bounds__(256) k_mlp_train(
     float gb3 = 0.f;
     double loss = 0;
     const float inv_n = 1.f / (float)nsamples;
+    // LDS writes and reads of one wave stay in order (the hardware keeps the
+    // order, the fence the compiler's)
+    auto wave_order = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
     for (int it = 0; it < tiles_per_wave; it++) {
-        const int64_t k = (wave * tiles_per_wave + it) * 16 + r;   // sample id
-        bool ok = k < nsamples;
-        int64_t node = k;
-        float target = 0.f;
-        if constexpr (DIRECT) {
-            if (ok) target = tdirect[k];
-        } else {
-            // uniform over the virtual particles of this solve
-            node = ok ? slot_of_rank[mix64(seed ^ (uint64_t)k) % (uint64_t)nv] : 0;
-            const int h = fs.hh[node];
-            ok = ok && h >= 1;
-            if (ok)
-                target = (vx[node] - fs.p1[node] -
-                          prior(h, fs.dp1[node], fs.dp2[node])) *
-                         fs.scale[SC_INV_TAU];
-        }
-        float fo[4];
-        const bf16x4 xb = tile_features<DIRECT>(fs, fdirect, nsamples, node, ok, fo);
+        const Sample S = next;
+        load_sample(it + 1, next);
+        const bool ok = S.ok;
+        const float target = S.target;
+        bf16x4 xb;
+#pragma unroll
+        for (int j = 0; j < 4; j++) xb[j] = f2bf(S.f[j]);
         Fwd F;
         forward<true>(W, sW2, xb, F);
         // dL/dout for the 16 nodes (lanes 0..15), broadcast to the columns
@@ -646,27 +711,26 @@ __global__ void __launch_bounds__(256) k_mlp_train(
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = t * 16 + 4 * q + i;
-                s_dz2[wl][row * 16 + r] = (uint16_t)dz2b[t][i];
-                s_h1[wl][row * 16 + r] = (uint16_t)F.h1[t][i];
-                s_dz1[wl][row * 16 + r] = (uint16_t)f2bf(dz1[t][i]);
+                s_dz2[row * kNS + r] = (uint16_t)dz2b[t][i];
+                s_h1[row * kNS + r] = (uint16_t)F.h1[t][i];
+                s_dz1[row * kNS + r] = (uint16_t)f2bf(dz1[t][i]);
             }
 #pragma unroll
-        for (int j = 0; j < 4; j++) s_x[wl][(4 * q + j) * 16 + r] = (uint16_t)xb[j];
-        __syncthreads();
+        for (int j = 0; j < 4; j++) s_x[(4 * q + j) * kNS + r] = (uint16_t)xb[j];
+        wave_order();
         // node-contracted products: A(hidden x node), B(node x hidden/feature)
         bf16x4 a_dz2[4], b_h1[4], a_dz1[4];
+        auto tile = [&](const uint16_t* st, int t) {
+            return *reinterpret_cast<const bf16x4*>(st + (t * 16 + r) * kNS + 4 * q);
+        };
 #pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                a_dz2[t][j] = (short)s_dz2[wl][(t * 16 + r) * 16 + 4 * q + j];
-                b_h1[t][j] = (short)s_h1[wl][(t * 16 + r) * 16 + 4 * q + j];
-                a_dz1[t][j] = (short)s_dz1[wl][(t * 16 + r) * 16 + 4 * q + j];
-            }
-        bf16x4 b_x;
-#pragma unroll
-        for (int j = 0; j < 4; j++) b_x[j] = (short)s_x[wl][r * 16 + 4 * q + j];
-        __syncthreads();
+        for (int t = 0; t < 4; t++) {
+            a_dz2[t] = tile(s_dz2, t);
+            b_h1[t] = tile(s_h1, t);
+            a_dz1[t] = tile(s_dz1, t);
+        }
+        const bf16x4 b_x = tile(s_x, 0);
+        wave_order();
 #pragma unroll
         for (int mo = 0; mo < 4; mo++)
 #pragma unroll
@@ -679,76 +743,62 @@ __global__ void __launch_bounds__(256) k_mlp_train(
 #pragma unroll
     for (int t = 0; t < 4; t++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                gb1[t][i] += __shfl_xor(gb1[t][i], o, 64);
-                gb2[t][i] += __shfl_xor(gb2[t][i], o, 64);
-                gW3[t][i] += __shfl_xor(gW3[t][i], o, 64);
-            }
+        for (int i = 0; i < 4; i++) {
+            gb1[t][i] = row_sum(gb1[t][i]);
+            gb2[t][i] = row_sum(gb2[t][i]);
+            gW3[t][i] = row_sum(gW3[t][i]);
+        }
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         gb3 += __shfl_xor(gb3, o, 64);
         loss += __shfl_xor(loss, o, 64);
     }
-    // Every gradient entry this lane holds, with its parameter index (each
-    // index is held by exactly one lane of the wave); f returns the new value.
-    auto each = [&](auto&& f) {
+    __syncthreads();                      // staging tiles no longer read
+    // every wave writes its entries (each parameter is held by one lane), then
+    // the block adds the four, coalesced and in a fixed order: (w0 + w2) + (w1 + w3)
+    {
+        float* G = s_red + wl * kNParams;
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int row = t * 16 + 4 * q + i;
-                if (r < kIn) gW1[t][i] = f(OFF_W1 + row * kIn + r, gW1[t][i]);
+                if (r < kIn) G[OFF_W1 + row * kIn + r] = gW1[t][i];
                 if (r == 0) {
-                    gb1[t][i] = f(OFF_B1 + row, gb1[t][i]);
-                    gb2[t][i] = f(OFF_B2 + row, gb2[t][i]);
-                    gW3[t][i] = f(OFF_W3 + row, gW3[t][i]);
+                    G[OFF_B1 + row] = gb1[t][i];
+                    G[OFF_B2 + row] = gb2[t][i];
+                    G[OFF_W3 + row] = gW3[t][i];
                 }
 #pragma unroll
                 for (int mi = 0; mi < 4; mi++)
-                    gW2[t][mi][i] = f(OFF_W2 + row * kHid + mi * 16 + r, gW2[t][mi][i]);
+                    G[OFF_W2 + row * kHid + mi * 16 + r] = gW2[t][mi][i];
             }
-        if (lane == 0) gb3 = f(OFF_B3, gb3);
-    };
-    // block sum in a fixed order: (w0 + w2) + (w1 + w3)
-    if (lane == 0) s_loss[wl] = loss;
-    __syncthreads();                      // staging tiles no longer read
-    if (wl >= 2)
-        each([&](int idx, float v) {
-            s_red[(wl - 2) * kNParams + idx] = v;
-            return v;
-        });
-    __syncthreads();
-    if (wl < 2) each([&](int idx, float v) { return v + s_red[wl * kNParams + idx]; });
-    __syncthreads();
-    if (wl == 1)
-        each([&](int idx, float v) {
-            s_red[idx] = v;
-            return v;
-        });
-    __syncthreads();
-    if (wl == 0) {
-        float* G = grad_part + (int64_t)blockIdx.x * kNParams;
-        each([&](int idx, float v) {
-            G[idx] = v + s_red[idx];
-            return v;
-        });
-        if (lane == 0)
-            loss_part[blockIdx.x] = ((s_loss[0] + s_loss[2]) + (s_loss[1] + s_loss[3])) *
-                                    (double)inv_n;
+        if (lane == 0) {
+            G[OFF_B3] = gb3;
+            s_loss[wl] = loss;
+        }
     }
+    __syncthreads();
+    float* G = grad_part + (int64_t)blockIdx.x * kNParams;
+#pragma unroll 10
+    for (int p = threadIdx.x; p < kNParams; p += 256)
+        G[p] = (s_red[p] + s_red[p + 2 * kNParams]) +
+               (s_red[p + kNParams] + s_red[p + 3 * kNParams]);
+    if (threadIdx.x == 0)
+        loss_part[blockIdx.x] =
+            ((s_loss[0] + s_loss[2]) + (s_loss[1] + s_loss[3])) * (double)inv_n;
 }
 
-// Sum of the per-block partials (fixed order).  Block = 64 parameters x 4
-// row groups; each thread sums rows g, g + 4, ... of its parameter, the 4
-// groups are added in order.
+// Sum of the per-block partials (fixed order).  Block = 16 parameters x 16
+// row groups; a thread sums rows g, g + 16, ... of its parameter (16 of 256,
+// all loads in flight), the groups are added pairwise.
+constexpr int kRedParams = 16;
 __global__ void __launch_bounds__(256) k_mlp_reduce(
     const float* grad_part, int nrows, const double* loss_part, float* grad,
     double* loss) {
-    __shared__ float s_g[4][64];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int p = blockIdx.x * 64 + tx;
+    __shared__ float s_g[16][kRedParams];
+    const int tx = threadIdx.x % kRedParams, ty = threadIdx.x / kRedParams;
+    const int p = blockIdx.x * kRedParams + tx;
     if (blockIdx.x == 0 && threadIdx.x < 64) {
         double s = 0;
         for (int w = threadIdx.x; w < nrows; w += 64) s += loss_part[w];
@@ -757,13 +807,16 @@ __global__ void __launch_bounds__(256) k_mlp_reduce(
     }
     float g = 0.f;
     if (p < kNParams) {
-#pragma unroll 8
-        for (int w = ty; w < nrows; w += 4) g += grad_part[(int64_t)w * kNParams + p];
+#pragma unroll 16
+        for (int w = ty; w < nrows; w += 16) g += grad_part[(int64_t)w * kNParams + p];
     }
     s_g[ty][tx] = g;
-    __syncthreads();
-    if (ty != 0 || p >= kNParams) return;
-    grad[p] = (s_g[0][tx] + s_g[1][tx]) + (s_g[2][tx] + s_g[3][tx]);
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) {
+        __syncthreads();
+        if (ty < o) s_g[ty][tx] += s_g[ty + o][tx];
+    }
+    if (ty == 0 && p < kNParams) grad[p] = s_g[0][tx];
 }
 
 // One Adam step (beta 0.9 / 0.999, eps 1e-8) on the reduced gradient, in one
@@ -957,9 +1010,9 @@ static void init_params(std::vector<float>& p, uint64_t seed) {
 // ---- scratch of vps_mlp_loss_and_grad_device (allocates nothing) ---------
 // One call's per-block partial losses (kTrainBlocks doubles) and partial
 // gradients (kTrainBlocks x kNParams floats): 4.92 MB on every device the
-// library runs on, held until the process ends.  Every call overwrites all
-// of it (each training block writes its whole row and its loss), so nothing
-// needs clearing; calls that overlap on one device race on it.
+// library runs on, held until the process ends.  Every call overwrites what it
+// reads (each of its training blocks writes its whole row and its loss), so
+// nothing needs clearing; calls that overlap on one device race on it.
 constexpr size_t kScratchLossBytes = (size_t)kTrainBlocks * sizeof(double);
 constexpr size_t kScratchBytes =
     kScratchLossBytes + (size_t)kTrainBlocks * kNParams * sizeof(float);
@@ -1172,18 +1225,18 @@ int mlp_after_solve(vps_context* c, const vps_stats* st) {
     // earlier solves with history
     if (m->training && m->hist_solves >= 2 && c->nvirt > 0) {
         const int64_t ns = m->batch;
-        const int tpw = (int)((ns + 16 * kTrainWaves - 1) / (16 * kTrainWaves));
+        const TrainShape ts(ns);
         for (int it = 0; it < m->steps_per_solve; it++) {
             m->adam_t++;
             const float b1t = (float)std::pow(0.9, (double)m->adam_t);
             const float b2t = (float)std::pow(0.999, (double)m->adam_t);
-            hipLaunchKernelGGL(k_mlp_train<false>, dim3(kTrainBlocks), dim3(256),
+            hipLaunchKernelGGL(k_mlp_train<false>, dim3(ts.blocks), dim3(256),
                                0, c->stream, m->P.p, feat_src(c, m->step_scale), c->vx[w].p,
                                m->slot_of_rank.p, c->nvirt, nullptr, nullptr, ns,
-                               tpw, m->seed ^ (uint64_t)m->adam_t * 0x100000001ull,
+                               ts.tiles, m->seed ^ (uint64_t)m->adam_t * 0x100000001ull,
                                m->grad_part.p, m->loss_part.p);
-            hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(kNParams, 64)), dim3(256),
-                               0, c->stream, m->grad_part.p, kTrainBlocks,
+            hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(kNParams, kRedParams)), dim3(256),
+                               0, c->stream, m->grad_part.p, ts.blocks,
                                m->loss_part.p, m->grad.p, m->loss.p);
             hipLaunchKernelGGL(k_mlp_adam, dim3(1), dim3(1024), 0, c->stream, m->grad.p,
                                m->loss.p, m->P.p, m->m.p, m->v.p, (float)m->lr, b1t, b2t,
@@ -1344,15 +1397,15 @@ int vps_mlp_loss_and_grad(vps_context* c, int64_t n, const float* features,
     VPS_TRY(dalloc(c, dt, (size_t)n));
     VPS_HIP(c, hipMemcpy(df.p, features, (size_t)n * kIn * 4, hipMemcpyHostToDevice));
     VPS_HIP(c, hipMemcpy(dt.p, targets, (size_t)n * 4, hipMemcpyHostToDevice));
-    const int tpw = (int)((n + 16 * kTrainWaves - 1) / (16 * kTrainWaves));
+    const TrainShape ts(n);
     FeatSrc none{};
     DBuf<double> dl;
     VPS_TRY(dalloc(c, dl, 1));
-    hipLaunchKernelGGL(k_mlp_train<true>, dim3(kTrainBlocks), dim3(256), 0,
+    hipLaunchKernelGGL(k_mlp_train<true>, dim3(ts.blocks), dim3(256), 0,
                        c->stream, m->P.p, none, nullptr, nullptr, n, df.p, dt.p, n,
-                       tpw, 0ull, m->grad_part.p, m->loss_part.p);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(kNParams, 64)), dim3(256), 0,
-                       c->stream, m->grad_part.p, kTrainBlocks, m->loss_part.p,
+                       ts.tiles, 0ull, m->grad_part.p, m->loss_part.p);
+    hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(kNParams, kRedParams)), dim3(256), 0,
+                       c->stream, m->grad_part.p, ts.blocks, m->loss_part.p,
                        m->grad.p, dl.p);
     VPS_HIP(c, hipGetLastError());
     if (grad)
@@ -1390,13 +1443,13 @@ int vps_mlp_loss_and_grad_device(vps_context* c, int64_t n, const float* d_featu
     MlpState* m = S(c);
     double* loss_part = (double*)base;
     float* grad_part = (float*)(base + kScratchLossBytes);
-    const int tpw = (int)((n + 16 * kTrainWaves - 1) / (16 * kTrainWaves));
+    const TrainShape ts(n);
     FeatSrc none{};
-    hipLaunchKernelGGL(k_mlp_train<true>, dim3(kTrainBlocks), dim3(256), 0, c->stream,
-                       m->P.p, none, nullptr, nullptr, n, d_features, d_targets, n, tpw,
+    hipLaunchKernelGGL(k_mlp_train<true>, dim3(ts.blocks), dim3(256), 0, c->stream,
+                       m->P.p, none, nullptr, nullptr, n, d_features, d_targets, n, ts.tiles,
                        0ull, grad_part, loss_part);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(kNParams, 64)), dim3(256), 0, c->stream,
-                       grad_part, kTrainBlocks, loss_part, d_grad, d_loss);
+    hipLaunchKernelGGL(k_mlp_reduce, dim3(blocks(kNParams, kRedParams)), dim3(256), 0, c->stream,
+                       grad_part, ts.blocks, loss_part, d_grad, d_loss);
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;
 }
