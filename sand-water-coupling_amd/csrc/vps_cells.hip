@@ -102,25 +102,29 @@ __global__ void __launch_bounds__(256) k_cell_place(
 
 // rho_i = m * sum_j W_h(|x_i - x_j|) over j with FP64 |x_j - x_i|^2 < h^2
 // (SmoothedParticles.cpp:25-31 via getNeighborWeight, .cpp:48-54).
-template <int D>
-__global__ void __launch_bounds__(256) k_density(const double4* pos,
-                                                 const int32_t* cstart,
-                                                 int64_t n, KConst k,
-                                                 float* rho, float4* vel,
-                                                 int set_volume) {
-    const int nb = (int)((n + 255) / 256);
-    const int64_t i = (int64_t)xcd_remap(blockIdx.x, nb) * 256 + threadIdx.x;
-    if (i >= n) return;
+// 2D; L lanes share a particle (see walk_lanes2).
+template <int L>
+__global__ void __launch_bounds__(256) k_density2(const double4* pos,
+                                                  const int32_t* cstart,
+                                                  int64_t n, KConst k,
+                                                  float* rho, float4* vel,
+                                                  int set_volume) {
+    const int64_t tid = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    const int64_t i = tid / L;
+    const int sub = L > 1 ? (int)(tid % L) : 0;
+    if (i >= n) return;   // uniform over the lanes of a particle
     const double4 q = pos[i];
     float sum = 0.f;
-    for_each_candidate<D>(k, cstart, pos, q.x, q.y, q.z, [&](int j, const double4& pj) {
-        const double d2 = D == 3 ? sq_dist3(pj.x, pj.y, pj.z, q.x, q.y, q.z)
-                                 : sq_dist2(pj.x, pj.y, q.x, q.y);
+    for_each_candidate2<L>(k, cstart, pos, q.x, q.y, sub, [&](int, double px, double py) {
+        const double d2 = sq_dist2(px, py, q.x, q.y);
         if (d2 < k.h2) {
             const KW w = kernel_f32(d2, k.h2, k.hf, k.inv_h, k.c0h, k.c1h);
             sum += w.w;
         }
     });
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    if (sub != 0) return;
     const float r = k.mass * sum;
     rho[i] = r;
     if (set_volume) vel[i].w = k.mass / r;
@@ -365,10 +369,15 @@ int real_density(vps_context* c, bool set_volume) {
         else if (lanes == 2) run(k_density3f<false, uint32_t, 2>, 2);
         else if (n * 16 <= (int64_t)UINT32_MAX) run(k_density3f<false, uint32_t, 1>, 1);
         else run(k_density3f<false, uint64_t, 1>, 1);
-    } else
-        hipLaunchKernelGGL(k_density<2>, dim3(blocks(n, 256)), dim3(256), 0,
-                           c->stream, c->rpos[s].p, c->cell_start.p, n, c->k,
-                           c->rrho.p, c->rvel[s].p, set_volume ? 1 : 0);
+    } else {
+        auto run = [&](auto kern, int lanes) {
+            hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
+                               c->rpos[s].p, c->cell_start.p, n, c->k, c->rrho.p, c->rvel[s].p,
+                               set_volume ? 1 : 0);
+        };
+        if (walk_lanes2(n) == 4) run(k_density2<4>, 4);
+        else run(k_density2<1>, 1);
+    }
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;
 }

@@ -60,6 +60,10 @@ __device__ __forceinline__ void boundary_term(const KConst& k, const double4& q,
     };
     if constexpr (L == 1) {
         for_each_candidate<D>(k, bcstart, bpos, q.x, q.y, q.z, visit);
+    } else if constexpr (D == 2) {
+        for_each_candidate2<L>(k, bcstart, bpos, q.x, q.y, sub, [&](int j, double px, double py) {
+            visit(j, make_double4(px, py, 0.0, 0.0));
+        });
     } else {
         const int cx = cell_coord(q.x, k.cell_lo[0], k.cell_inv, k.cdims[0]);
         const int cy = cell_coord(q.y, k.cell_lo[1], k.cell_inv, k.cdims[1]);
@@ -76,12 +80,13 @@ __device__ __forceinline__ void boundary_term(const KConst& k, const double4& q,
 }
 
 // Virtual part of the update from global memory: the node box around x_i,
-// exact FP64 membership, brick map lookups.
-template <int D>
+// exact FP64 membership, brick map lookups.  L lanes share a particle, each
+// taking every L-th row.
+template <int D, int L = 1>
 __device__ __forceinline__ void virtual_term_global(const KConst& k, const double4& q,
                                                     const int32_t* slot_of_brick,
                                                     const float* vq, float& fx,
-                                                    float& fy, float& fz) {
+                                                    float& fy, float& fz, int sub = 0) {
     const double qc[3] = {q.x, q.y, q.z};
     const double inv = 1.0 / k.spacing;
     int lo[3] = {0, 0, 0}, cnt[3] = {1, 1, 1};
@@ -119,7 +124,7 @@ __device__ __forceinline__ void virtual_term_global(const KConst& k, const doubl
                 dz2 = dsq(dz);
                 if (!(dz2 < k.H2)) continue;   // no node of this plane within H
             }
-            for (int iy = 0; iy < cnt[1]; iy++) {
+            for (int iy = sub; iy < cnt[1]; iy += L) {
                 const int cy = lo[1] + iy;
                 const double dy = dsub(node_coord(k.origin[1], cy, k.spacing), q.y);
                 const double dy2 = dsq(dy);
@@ -170,19 +175,27 @@ __device__ __forceinline__ void virtual_term_global(const KConst& k, const doubl
     }
 }
 
-template <int D>
+template <int D, int L>
 __global__ void __launch_bounds__(256) k_gradient(
     KConst k, int64_t n, const double4* rpos, float4* rvel,
     const int32_t* slot_of_brick, const float* vq, const double4* bpos,
     const float4* bvel, const float4* bnrm, const int32_t* bcstart, SolveGuard guard) {
-    const int nblk = (int)((n + 255) / 256);
-    const int64_t i = (int64_t)xcd_remap(blockIdx.x, nblk) * 256 + threadIdx.x;
-    if (i >= n || !solve_accepted(guard)) return;
+    const int64_t tid = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    const int64_t i = tid / L;
+    const int sub = L > 1 ? (int)(tid % L) : 0;
+    if (i >= n || !solve_accepted(guard)) return;   // uniform over the lanes of a particle
     const double4 q = rpos[i];
     float4 vi = rvel[i];
     float fx = 0.f, fy = 0.f, fz = 0.f;
-    virtual_term_global<D>(k, q, slot_of_brick, vq, fx, fy, fz);
-    boundary_term<D>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz);
+    virtual_term_global<D, L>(k, q, slot_of_brick, vq, fx, fy, fz, sub);
+    boundary_term<D, L>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz, sub);
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) {
+        fx += __shfl_xor(fx, o, 64);
+        fy += __shfl_xor(fy, o, 64);
+        if (D == 3) fz += __shfl_xor(fz, o, 64);
+    }
+    if (sub != 0) return;
     vi.x += fx;
     vi.y += fy;
     if (D == 3) vi.z += fz;
@@ -683,16 +696,16 @@ int pressure_gradient(vps_context* c, SolveGuard g) {
                                c->rpos[s].p, c->rvel[s].p, c->brick_slot[w].p, c->vq.p,
                                c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, g);
         }
-    } else if (c->dim == 3)
-        hipLaunchKernelGGL(k_gradient<3>, dim3(blocks(n, 256)), dim3(256), 0,
-                           c->stream, c->k, n, c->rpos[s].p, c->rvel[s].p,
-                           c->brick_slot[w].p, c->vq.p, c->bpos.p, c->bvel.p,
-                           c->bnrm.p, c->bcell_start.p, g);
-    else
-        hipLaunchKernelGGL(k_gradient<2>, dim3(blocks(n, 256)), dim3(256), 0,
-                           c->stream, c->k, n, c->rpos[s].p, c->rvel[s].p,
-                           c->brick_slot[w].p, c->vq.p, c->bpos.p, c->bvel.p,
-                           c->bnrm.p, c->bcell_start.p, g);
+    } else {
+        auto run = [&](auto kern, int lanes) {
+            hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream, c->k,
+                               n, c->rpos[s].p, c->rvel[s].p, c->brick_slot[w].p, c->vq.p,
+                               c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, g);
+        };
+        if (c->dim == 3) run(k_gradient<3, 1>, 1);
+        else if (walk_lanes2(n) == 4) run(k_gradient<2, 4>, 4);
+        else run(k_gradient<2, 1>, 1);
+    }
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;
 }

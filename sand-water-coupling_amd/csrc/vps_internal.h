@@ -280,6 +280,49 @@ __device__ __forceinline__ void for_each_candidate(const KConst& k,
         }
 }
 
+// 2D candidates of a point by L lanes that share it, each taking every L-th of
+// a row: the bounds of the three rows are loaded at once, then the first U
+// positions of all rows.
+template <int L, typename F>
+__device__ __forceinline__ void for_each_candidate2(const KConst& k, const int32_t* cstart,
+                                                    const double4* pos, double qx, double qy,
+                                                    int sub, F&& f) {
+    if constexpr (L == 1) {
+        for_each_candidate<2>(k, cstart, pos, qx, qy, 0.0,
+                              [&](int j, const double4& p) { f(j, p.x, p.y); });
+    } else {
+        constexpr int U = 4;   // (12 candidates a row are the rule)
+        const int cx = cell_coord(qx, k.cell_lo[0], k.cell_inv, k.cdims[0]);
+        const int cy = cell_coord(qy, k.cell_lo[1], k.cell_inv, k.cdims[1]);
+        const int x0 = max(cx - 1, 0), x1 = min(cx + 1, k.cdims[0] - 1);
+        int b[3], e[3];
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            const int y = cy + r - 1;
+            const int row = min(max(y, 0), k.cdims[1] - 1) * k.cdims[0];
+            b[r] = cstart[row + x0] + sub;
+            e[r] = cstart[row + x1 + 1];
+            if (y < 0 || y >= k.cdims[1]) e[r] = 0;
+        }
+        double2 p[3][U];
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (b[r] + u * L < e[r]) p[r][u] = *(const double2*)(pos + b[r] + u * L);
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (b[r] + u * L < e[r]) f(b[r] + u * L, p[r][u].x, p[r][u].y);
+            for (int j = b[r] + U * L; j < e[r]; j += L) {
+                const double2 pj = *(const double2*)(pos + j);
+                f(j, pj.x, pj.y);
+            }
+        }
+    }
+}
+
 // The 3 x 3 x-rows of cells around cell (., cy, cz), each one candidate range
 // of the cells x0 .. x1: f(ty, tz, begin, end) with ty, tz = q - C of the row's
 // cells, rounded once from FP64.  With several lanes per particle
@@ -329,6 +372,14 @@ __device__ __forceinline__ void for_each_row(const KConst& k, const int32_t* cst
 inline int walk_lanes(int64_t n) {
     return n <= 32000 ? 8 : (n <= 400000 ? 4 : (n <= 900000 ? 2 : 1));
 }
+
+// The same of the 2D walks (36 candidates).  us with 1, 4, 8 lanes:
+//   particles   density         viscosity       virtual sums   gradient
+//   400         10, 5.7, 4.9    12, 6.1, 6.7    26, 13, 10     14, 7.2, 6.1
+//   40,000      11, 6.5, 6.5    14, 8.4, 7.7    27, 17, 20     11, 7.6, 8.7
+//   97,000      12, 9.0, 10     18, 11, 13      32, 26, 33     9.2, 8.2, 10
+//   250,000     15, 17, 21      20, 21, 24      48, 62, 77     13, 15, 19
+inline int walk_lanes2(int64_t n) { return n <= 130000 ? 4 : 1; }
 
 // Work units of the 3D gradient: blocks of u[0] x u[1] x u[2] cells (at most
 // kUnitRows rows of cells, each a contiguous range of the sorted particles).

@@ -177,21 +177,29 @@ __global__ void __launch_bounds__(256) k_viscosity3f(const double4* pos, const f
     vout[i] = v;
 }
 
+template <int L>
 __global__ void __launch_bounds__(256) k_viscosity2(const double4* pos, const int32_t* cstart,
                                                     const float4* vel, const float* rho,
                                                     int64_t n, KConst k, float scale,
                                                     float4* vout) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
+    const int64_t tid = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t i = tid / L;
+    const int sub = L > 1 ? (int)(tid % L) : 0;
+    if (i >= n) return;   // uniform over the lanes of a particle
     const double4 q = pos[i];
     const float4 vi = vel[i];
     ViscAcc acc;
-    for_each_candidate<2>(k, cstart, pos, q.x, q.y, q.z, [&](int j, const double4& pj) {
-        const double d2 = sq_dist2(pj.x, pj.y, q.x, q.y);
+    for_each_candidate2<L>(k, cstart, pos, q.x, q.y, sub, [&](int j, double px, double py) {
+        const double d2 = sq_dist2(px, py, q.x, q.y);
         if (!(d2 > 0) || !(d2 < k.h2)) return;
-        acc.add(k, (float)d2, (float)(pj.x - q.x), (float)(pj.y - q.y), 0.f, vi, vel[j],
-                rho[j]);
+        acc.add(k, (float)d2, (float)(px - q.x), (float)(py - q.y), 0.f, vi, vel[j], rho[j]);
     });
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) {
+        acc.lx += __shfl_xor(acc.lx, o, 64);
+        acc.ly += __shfl_xor(acc.ly, o, 64);
+    }
+    if (sub != 0) return;
     float4 v = vi;
     v.x += scale * acc.lx;
     v.y += scale * acc.ly;
@@ -276,10 +284,15 @@ int apply_viscosity(vps_context* c, double dt, double nu) {
         else if (lanes == 4) run(k_viscosity3f<4>, 4);
         else if (lanes == 2) run(k_viscosity3f<2>, 2);
         else run(k_viscosity3f<1>, 1);
-    } else
-        hipLaunchKernelGGL(k_viscosity2, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
-                           c->rpos[s].p, c->cell_start.p, c->rvel[s].p, c->rrho.p, n, c->k,
-                           scale, c->vel_next.p);
+    } else {
+        auto run = [&](auto kern, int lanes) {
+            hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
+                               c->rpos[s].p, c->cell_start.p, c->rvel[s].p, c->rrho.p, n, c->k,
+                               scale, c->vel_next.p);
+        };
+        if (walk_lanes2(n) == 4) run(k_viscosity2<4>, 4);
+        else run(k_viscosity2<1>, 1);
+    }
     VPS_HIP(c, hipGetLastError());
     std::swap(c->rvel[s], c->vel_next);   // every particle's velocity was written
     return VPS_OK;

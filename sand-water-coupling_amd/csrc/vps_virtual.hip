@@ -209,17 +209,15 @@ struct BAcc {
 // Everything after the real walk: the exact threshold decision, the boundary
 // walk, v_I, D_I and the outputs.
 // Boundary walk of one node from the global cell table (FP64 throughout).
-template <int D>
-struct BoundaryWalkGlobal {
+struct BoundaryWalkGlobal3 {
     const int32_t* bcstart;
     const double4* bpos;
     __device__ __forceinline__ void operator()(const KConst& k, double qx, double qy,
                                                double qz, const float4* bvel,
                                                const float4* bnrm, BAcc& b) const {
-        for_each_candidate<D>(k, bcstart, bpos, qx, qy, qz, [&](int j, const double4& pj) {
-            const double d2 = D == 3 ? sq_dist3(pj.x, pj.y, pj.z, qx, qy, qz)
-                                     : sq_dist2(pj.x, pj.y, qx, qy);
-            if (d2 < k.h2) b.add_exact<D>(k, qx, qy, qz, pj, d2, bvel[j], bnrm[j].w);
+        for_each_candidate<3>(k, bcstart, bpos, qx, qy, qz, [&](int j, const double4& pj) {
+            const double d2 = sq_dist3(pj.x, pj.y, pj.z, qx, qy, qz);
+            if (d2 < k.h2) b.add_exact<3>(k, qx, qy, qz, pj, d2, bvel[j], bnrm[j].w);
         });
     }
 };
@@ -277,28 +275,27 @@ __device__ __forceinline__ void finish_node(
     atomicOr(&bits[lin >> 5], 1u << (lin & 31));
 }
 
-// The real walk straight from global memory (2D, and 3D bricks whose
-// neighbourhood does not fit the LDS stage).
-template <int D>
-__device__ __forceinline__ void real_walk_global(const KConst& k,
+// The real walk straight from global memory (bricks whose neighbourhood does
+// not fit the LDS stage).
+__device__ __forceinline__ void real_walk_global3(const KConst& k,
                                                  const int32_t* rcstart,
                                                  const double4* rpos,
                                                  const float4* rvel,
                                                  const float* rrho, double qx,
                                                  double qy, double qz,
                                                  RealAcc& a) {
-    for_each_candidate<D>(k, rcstart, rpos, qx, qy, qz, [&](int j, const double4& pj) {
-        const double d2 = D == 3 ? sq_dist3(pj.x, pj.y, pj.z, qx, qy, qz)
-                                 : sq_dist2(pj.x, pj.y, qx, qy);
+    for_each_candidate<3>(k, rcstart, rpos, qx, qy, qz, [&](int j, const double4& pj) {
+        const double d2 = sq_dist3(pj.x, pj.y, pj.z, qx, qy, qz);
         if (d2 < k.h2)
-            a.add<D>(k, d2, (float)(qx - pj.x), (float)(qy - pj.y),
-                     D == 3 ? (float)(qz - pj.z) : 0.f, rvel[j], 1.f / rrho[j]);
+            a.add<3>(k, d2, (float)(qx - pj.x), (float)(qy - pj.y), (float)(qz - pj.z), rvel[j],
+                     1.f / rrho[j]);
     });
 }
 
-// Fused per-node pass.  One workgroup = one brick; thread = node.
-template <int D, int NB>
-__global__ void __launch_bounds__(NB) k_virtual_sums(
+// Fused per-node pass in 2D.  One workgroup = one brick, S lanes per node (see
+// walk_lanes2), straight from global memory: 36 candidates a node.
+template <int S>
+__global__ void __launch_bounds__(64 * S) k_virtual_sums2(
     KConst k, const int32_t* brick_of_slot, const int32_t* nslots_p,
     const double4* rpos, const float4* rvel, const float* rrho,
     const int32_t* rcstart, const double4* bpos, const float4* bvel,
@@ -308,28 +305,37 @@ __global__ void __launch_bounds__(NB) k_virtual_sums(
     if ((int)blockIdx.x >= nslots) return;
     const int slot = xcd_remap(blockIdx.x, nslots);
     const int brick = brick_of_slot[slot];
-    const int t = threadIdx.x;
-    const int lx = t & 7, ly = (t >> 3) & 7, lz = D == 3 ? t >> 6 : 0;
-    const int bx = brick % k.bdims[0];
-    const int by = (brick / k.bdims[0]) % k.bdims[1];
-    const int bz = D == 3 ? brick / k.bdims[0] / k.bdims[1] : 0;
-    const int cx = bx * kBrick + lx, cy = by * kBrick + ly,
-              cz = bz * kBrick + lz;
-    const int64_t out = (int64_t)slot * NB + t;
-    if (cx >= k.ndims[0] || cy >= k.ndims[1] || (D == 3 && cz >= k.ndims[2])) {
-        vrho[out] = 0.f;
-        vvol[out] = 0.f;
-        vb[out] = 0.f;
-        return;
+    const int node = threadIdx.x / S, sub = S > 1 ? threadIdx.x % S : 0;
+    const int cx = brick % k.bdims[0] * kBrick + (node & 7),
+              cy = brick / k.bdims[0] * kBrick + (node >> 3);
+    const int64_t out = (int64_t)slot * 64 + node;
+    if (cx >= k.ndims[0] || cy >= k.ndims[1]) {
+        if (sub == 0) vrho[out] = vvol[out] = vb[out] = 0.f;
+        return;   // uniform over the lanes of a node
     }
     const double qx = node_coord(k.origin[0], cx, k.spacing);
     const double qy = node_coord(k.origin[1], cy, k.spacing);
-    const double qz = D == 3 ? node_coord(k.origin[2], cz, k.spacing) : 0.0;
     RealAcc a;
-    real_walk_global<D>(k, rcstart, rpos, rvel, rrho, qx, qy, qz, a);
-    finish_node<D>(k, a, qx, qy, qz, cx, cy, cz, out, rpos, rcstart,
-                   BoundaryWalkGlobal<D>{bcstart, bpos}, bvel, bnrm, vrho, vvol,
-                   vb, bits);
+    for_each_candidate2<S>(k, rcstart, rpos, qx, qy, sub, [&](int j, double px, double py) {
+        const double d2 = sq_dist2(px, py, qx, qy);
+        if (d2 < k.h2)
+            a.add<2>(k, d2, (float)(qx - px), (float)(qy - py), 0.f, rvel[j], 1.f / rrho[j]);
+    });
+    if constexpr (S > 1) {
+#pragma unroll
+        for (int o = 1; o < S; o <<= 1) a.add_lanes(o);
+    }
+    auto boundary = [&](const KConst& k, double qx, double qy, double, const float4* bvel,
+                        const float4* bnrm, BAcc& b) {
+        for_each_candidate2<S>(k, bcstart, bpos, qx, qy, sub, [&](int j, double px, double py) {
+            const double d2 = sq_dist2(px, py, qx, qy);
+            if (d2 < k.h2)
+                b.add_exact<2>(k, qx, qy, 0.0, make_double4(px, py, 0.0, 0.0), d2, bvel[j],
+                               bnrm[j].w);
+        });
+    };
+    finish_node<2, S>(k, a, qx, qy, 0.0, cx, cy, 0, out, rpos, rcstart, boundary, bvel, bnrm,
+                      vrho, vvol, vb, bits);
 }
 
 // 3D with the brick's neighbourhood staged in LDS: one workgroup of 512
@@ -600,9 +606,9 @@ __global__ void __launch_bounds__(512, 4) k_virtual_sums3s(
     RealAcc a;
     if (!staged) {
         if (sub != 0) return;
-        real_walk_global<3>(k, rcstart, rpos, rvel, rrho, qx, qy, qz, a);
+        real_walk_global3(k, rcstart, rpos, rvel, rrho, qx, qy, qz, a);
         finish_node<3>(k, a, qx, qy, qz, cx, cy, cz, out, rpos, rcstart,
-                       BoundaryWalkGlobal<3>{bcstart, bpos}, bvel, bnrm, vrho,
+                       BoundaryWalkGlobal3{bcstart, bpos}, bvel, bnrm, vrho,
                        vvol, vb, bits);
         return;
     }
@@ -652,7 +658,7 @@ __global__ void __launch_bounds__(512, 4) k_virtual_sums3s(
     auto boundary = [&](const KConst& k, double qx, double qy, double qz, const float4* bvel,
                         const float4* bnrm, BAcc& b) {
         if (!pooled) {
-            if (sub == 0) BoundaryWalkGlobal<3>{bcstart, bpos}(k, qx, qy, qz, bvel, bnrm, b);
+            if (sub == 0) BoundaryWalkGlobal3{bcstart, bpos}(k, qx, qy, qz, bvel, bnrm, b);
             return;
         }
         if (nboundary == 0) return;
@@ -867,13 +873,16 @@ static int generate_slots(vps_context* c, int w, int64_t grid, bool first) {
         else if (lanes == 4) run(k_virtual_sums3s<4>, 4);
         else if (lanes == 2) run(k_virtual_sums3s<2>, 2);
         else run(k_virtual_sums3s<1>, 1);
-    } else
-        hipLaunchKernelGGL((k_virtual_sums<2, 64>), dim3((unsigned)grid),
-                           dim3(64), 0, c->stream, c->k, c->slot_brick[w].p,
-                           nsl, c->rpos[rs].p, c->rvel[rs].p, c->rrho.p,
-                           c->cell_start.p, c->bpos.p, c->bvel.p, c->bnrm.p,
-                           c->bcell_start.p, c->vrho.p, c->vvol.p, c->vb.p,
-                           c->bits.p);
+    } else {
+        auto run = [&](auto kern, int s) {
+            hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * s), 0, c->stream, c->k,
+                               c->slot_brick[w].p, nsl, c->rpos[rs].p, c->rvel[rs].p, c->rrho.p,
+                               c->cell_start.p, c->bpos.p, c->bvel.p, c->bnrm.p,
+                               c->bcell_start.p, c->vrho.p, c->vvol.p, c->vb.p, c->bits.p);
+        };
+        if (walk_lanes2(c->n) == 4) run(k_virtual_sums2<4>, 4);
+        else run(k_virtual_sums2<1>, 1);
+    }
     // the column order and the tables, on the grid (before the read-back
     // below, so that they run while the host waits)
     const int32_t* bos = c->slot_brick[w].p;
