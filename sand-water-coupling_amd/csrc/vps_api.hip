@@ -216,7 +216,6 @@ void free_all(vps_context* c) {
     dfree(c->bofs);
     dfree(c->vel_next);
     dfree(c->grad_units);
-    dfree(c->grad_over);
     dfree(c->couple_stage);
     dfree(c->io_stage);
     dfree(c->cell_of);

@@ -225,36 +225,6 @@ __device__ __forceinline__ int node_floor(double x, double o, double inv) {
     return (int)f;
 }
 
-// Units whose box exceeds the stage, from the overflow list that
-// k_gradient3s fills: the global-memory path, one thread per particle.
-__global__ void __launch_bounds__(kGradThreads) k_gradient_overflow(
-    KConst k, UnitArgs ua, const int32_t* over, const int32_t* nover,
-    const double4* rpos, float4* rvel, const int32_t* slot_of_brick, const float* vq,
-    const double4* bpos, const float4* bvel, const float4* bnrm, const int32_t* bcstart,
-    SolveGuard guard) {
-    if (!solve_accepted(guard)) return;
-    const int no = *nover;
-    for (int o = blockIdx.x; o < no; o += gridDim.x) {
-        const UnitCells uc(k, ua, over[o]);
-        for (int r = 0; r < uc.rows(); r++) {
-            const int64_t row = uc.row(k, r);
-            const int end = ua.cstart[row + uc.m[0]];
-            for (int p = ua.cstart[row] + threadIdx.x; p < end; p += kGradThreads) {
-                const double4 q = rpos[p];
-                const float4 vi = rvel[p];
-                float fx = 0.f, fy = 0.f, fz = 0.f;
-                virtual_term_global<3>(k, q, slot_of_brick, vq, fx, fy, fz);
-                boundary_term<3>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz);
-                float4 v = vi;
-                v.x += fx;
-                v.y += fy;
-                v.z += fz;
-                rvel[p] = v;
-            }
-        }
-    }
-}
-
 // L lanes share a particle: lane `sub` takes x candidates P and 7 - P of every
 // row for the pairs P = sub, sub + L, ... of 4 (with 8 lanes: candidate sub).
 // CNT (test support): vq holds V_J instead of q_J, and only the number of
@@ -264,8 +234,8 @@ template <int L, bool CNT = false>
 __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
     KConst k, UnitArgs ua, int nunits, const double4* rpos, float4* rvel,
     const int32_t* slot_of_brick, const float* vq, const double4* bpos,
-    const float4* bvel, const float4* bnrm, const int32_t* bcstart, int32_t* over,
-    int32_t* nover, SolveGuard guard, int32_t* members = nullptr) {
+    const float4* bvel, const float4* bnrm, const int32_t* bcstart, SolveGuard guard,
+    int32_t* members = nullptr) {
     if (!solve_accepted(guard)) return;   // uniform over the block
     __shared__ float s_q[kGradCap];
     __shared__ int s_bslot[kGradBoxBricks];   // slots of the box's bricks
@@ -350,18 +320,30 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
     const int64_t e0 = (int64_t)s_box[3] - s_box[0] + 8;
     const int64_t e1 = (int64_t)s_box[4] - s_box[1] + 8;
     const int64_t e2 = (int64_t)s_box[5] - s_box[2] + 8;
-    if (e0 * e1 * e2 > kGradCap) {
-        // particles far outside their cells: left to k_gradient_overflow
-        if (!CNT && t == 0) over[atomicAdd(nover, 1)] = unit;
-        return;
-    }
+    // particles far outside their cells: straight from global memory
+    auto beyond_stage = [&] {
+        if constexpr (CNT) return;
+        for (int i = t; i < count; i += kGradThreads) {
+            const int p = particle(i);
+            const double4 q = rpos[p];
+            float4 v = rvel[p];
+            float fx = 0.f, fy = 0.f, fz = 0.f;
+            virtual_term_global<3>(k, q, slot_of_brick, vq, fx, fy, fz);
+            boundary_term<3>(k, q, v, bpos, bvel, bnrm, bcstart, fx, fy, fz);
+            v.x += fx;
+            v.y += fy;
+            v.z += fz;
+            rvel[p] = v;
+        }
+    };
+    const bool over_nodes = e0 * e1 * e2 > kGradCap;
     // the bricks the box touches (floor division by 8, also below zero)
     const int bx0 = lo0 >> 3, by0 = lo1 >> 3, bz0 = lo2 >> 3;
     const int nbx = ((lo0 + (int)e0 - 1) >> 3) - bx0 + 1;
     const int nby = ((lo1 + (int)e1 - 1) >> 3) - by0 + 1;
     const int nbz = ((lo2 + (int)e2 - 1) >> 3) - bz0 + 1;
-    if (nbx * nby * nbz > kGradBoxBricks) {
-        if (!CNT && t == 0) over[atomicAdd(nover, 1)] = unit;
+    if (over_nodes || nbx * nby * nbz > kGradBoxBricks) {
+        beyond_stage();
         return;
     }
     // their slots (-1 off the virtual set or off the lattice) in one round
@@ -636,7 +618,6 @@ int gradient_setup(vps_context* c) {
     int64_t total = 1;   // of the smallest units
     for (int a = 0; a < 3; a++) total *= (k.cdims[a] + u[a] - 1) / u[a];
     VPS_TRY(dalloc(c, c->grad_units, (size_t)total));
-    VPS_TRY(dalloc(c, c->grad_over, (size_t)total));
     c->grad_staged = true;
     return VPS_OK;
 }
@@ -666,8 +647,7 @@ int gradient_member_counts(vps_context* c, int32_t* members) {
                            dim3(kGradThreads), 0, c->stream, c->k, c->grad_shape,
                            (int)c->grad_nunits, c->rpos[c->cur].p, c->rvel[c->cur].p,
                            c->brick_slot[c->which].p, c->vvol.p, c->bpos.p, c->bvel.p,
-                           c->bnrm.p, c->bcell_start.p, (int32_t*)nullptr,
-                           (int32_t*)nullptr, SolveGuard{}, members);
+                           c->bnrm.p, c->bcell_start.p, SolveGuard{}, members);
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;
 }
@@ -678,23 +658,17 @@ int pressure_gradient(vps_context* c, SolveGuard g) {
     const int w = c->which;
     if (c->dim == 3 && c->grad_staged) {
         if (c->grad_nunits > 0) {
-            int32_t* nover = (int32_t*)(c->counters.p + 3);   // zeroed with the units
-            int32_t* over = c->grad_over.p;
             auto run = [&](auto kern) {
                 hipLaunchKernelGGL(kern, dim3((unsigned)c->grad_nunits), dim3(kGradThreads), 0,
                                    c->stream, c->k, c->grad_shape, (int)c->grad_nunits,
                                    c->rpos[s].p, c->rvel[s].p, c->brick_slot[w].p, c->vq.p,
-                                   c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, over,
-                                   nover, g, (int32_t*)nullptr);
+                                   c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, g,
+                                   (int32_t*)nullptr);
             };
             const int lanes = unit_rule(n).lanes;
             if (lanes == 8) run(k_gradient3s<8>);
             else if (lanes == 4) run(k_gradient3s<4>);
             else run(k_gradient3s<1>);
-            hipLaunchKernelGGL(k_gradient_overflow, dim3(64), dim3(kGradThreads), 0,
-                               c->stream, c->k, c->grad_shape, over, nover,
-                               c->rpos[s].p, c->rvel[s].p, c->brick_slot[w].p, c->vq.p,
-                               c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, g);
         }
     } else {
         auto run = [&](auto kern, int lanes) {

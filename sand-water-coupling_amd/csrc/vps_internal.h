@@ -587,7 +587,6 @@ struct vps_context {
     // (negative: clamped into a border cell, exact test only)
     vps::DBuf<float4> bofs;
     vps::DBuf<int32_t> grad_units;      // 3D gradient: units that hold particles
-    vps::DBuf<int32_t> grad_over;       // units left to the global-memory path
     bool grad_staged = false;           // false: global-memory gradient
     vps::UnitArgs grad_shape;           // units of the last generation
     int64_t grad_nunits = 0;            // and how many of them hold particles

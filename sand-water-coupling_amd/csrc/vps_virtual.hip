@@ -39,10 +39,7 @@ __global__ void __launch_bounds__(256) k_mark_bricks(const double4* pos,
                                                      int64_t nwords, int32_t* unit_count) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     for (int64_t w = i; w < nwords; w += (int64_t)gridDim.x * 256) bits[w] = 0u;
-    if (i == 0) {   // the gradient's unit and overflow lists are rebuilt next
-        unit_count[0] = 0;
-        unit_count[2] = 0;
-    }
+    if (i == 0) unit_count[0] = 0;   // the gradient's unit list is rebuilt next
     if (i >= n) return;
     const double4 p = pos[i];
     const double pc[3] = {p.x, p.y, p.z};
