@@ -429,17 +429,14 @@ int boundary_density(vps_context* c) {
     {
         // the density walk as for the real particles, on the sort's offsets,
         // then the offsets with w = +-1 / rho_b for the virtual sums
-        auto run = [&](auto kern, int lanes) {
-            hipLaunchKernelGGL(kern, dim3(blocks(nb * lanes, 256)), dim3(256), 0, c->stream,
-                               c->bpos.p, c->bofs.p, c->bcell_start.p, nb, c->k, (float*)nullptr,
-                               (float*)nullptr, c->bnrm.p, c->bvel.p, 0, (int32_t*)nullptr);
-        };
-        const int lanes = walk_lanes(nb);
-        if (lanes == 8) run(k_density3f<true, uint32_t, 8>, 8);
-        else if (lanes == 4) run(k_density3f<true, uint32_t, 4>, 4);
-        else if (lanes == 2) run(k_density3f<true, uint32_t, 2>, 2);
-        else if (nb * 16 <= (int64_t)UINT32_MAX) run(k_density3f<true, uint32_t, 1>, 1);
-        else run(k_density3f<true, uint64_t, 1>, 1);
+        if (nb * 16 <= (int64_t)UINT32_MAX)
+            hipLaunchKernelGGL((k_density3f<true, uint32_t, 1>), dim3(blocks(nb, 256)), dim3(256),
+                               0, c->stream, c->bpos.p, c->bofs.p, c->bcell_start.p, nb, c->k,
+                               (float*)nullptr, (float*)nullptr, c->bnrm.p, c->bvel.p, 0);
+        else
+            hipLaunchKernelGGL((k_density3f<true, uint64_t, 1>), dim3(blocks(nb, 256)), dim3(256),
+                               0, c->stream, c->bpos.p, c->bofs.p, c->bcell_start.p, nb, c->k,
+                               (float*)nullptr, (float*)nullptr, c->bnrm.p, c->bvel.p, 0);
         hipLaunchKernelGGL(k_boundary_offsets3, dim3(blocks(nb, 256)), dim3(256), 0,
                            c->stream, c->bpos.p, c->bnrm.p, nb, c->k, c->bofs.p);
     }

@@ -369,8 +369,6 @@ __device__ __forceinline__ void for_each_row(const KConst& k, const int32_t* cst
 //   212,503       45, 35, 35, 41                            (77, 46, 33, 38)
 //   300,000       53, 53, 52, 59     600,000  96, 84, 90, 107
 //   1,012,500    131, 131, 142, 172
-// (of wall sheets: 5,760 boundary particles 36, 20, 13, 9; 116,856: 35, 23, 19,
-// 24; 696,816: 78, 63, 70, 94)
 inline int walk_lanes(int64_t n) {
     return n <= 32000 ? 8 : (n <= 400000 ? 4 : (n <= 900000 ? 2 : 1));
 }
