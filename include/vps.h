@@ -149,7 +149,7 @@ typedef struct vps_stats {
     double ms_gradient;        /* pressure gradient + velocity update */
     double ms_total;
     double ms_spmv_avg;        /* average duration of one CG SpMV launch */
-    double ms_update_avg;      /* average duration of one CG update launch */
+    double ms_update_avg;      /* 0: the update is part of the iteration launch */
     int64_t spmv_launches;
     int64_t reserved[4];       /* [0] residual replacements of the last solve,
                                   [1] host microseconds spent launching its CG
@@ -462,7 +462,7 @@ int vps_debug_apply_operator(vps_context* ctx, const double* p, double* out);
  * density walk (boundary particles within h of each boundary particle),
  * 2: the pressure gradient's walk over the virtual particles within H of
  * each real particle (VirtualParticle.cpp:118-124; -1 for a particle whose
- * span is beyond the staged path), 3: the viscosity walk (real particles
+ * unit is beyond the staged path), 3: the viscosity walk (real particles
  * within h of each real particle, itself excluded).  The walks decide
  * membership on FP32
  * distances: only a pair within rounding of the cutoff, whose term is zero

@@ -479,7 +479,7 @@ __global__ void __launch_bounds__(512, 4) k_virtual_sums3s(
     const float4* bofs, const float4* bvel, const float4* bnrm, const int32_t* bcstart,
     float* vrho, float* vvol, float* vb, uint32_t* bits) {
     constexpr int kPlanes = kBrick / S;
-    constexpr int kRowsAtOnce = 5;   // rows a wave loads at once (36 rows of a brick in one go)
+    constexpr int kRowsAtOnce = 5;   // rows a wave loads at once (a brick has about 49; with 7: 268 for 263 us at 1M)
     __shared__ Stage<S> st;
     const int nslots = *nslots_p;   // the grid may exceed the slot count
     if ((int)blockIdx.x >= nslots * S) return;
@@ -928,7 +928,7 @@ int virtual_generate(vps_context* c) {
     const int w = c->last_solve_buf >= 0 ? 1 - c->last_solve_buf : 0;
     const int D = c->dim;
     const int s = c->cur;
-    // brick flags are zero on entry (cleared by k_assign_slots)
+    // brick flags are zero on entry (cleared by AssignSlot)
     const unsigned mb = blocks(c->n, 256) > 0 ? blocks(c->n, 256) : 1;
     if (D == 3)
         hipLaunchKernelGGL(k_mark_bricks<3>, dim3(mb), dim3(256),
