@@ -65,7 +65,7 @@ constexpr int kT2 = kT * kT;
 constexpr int kHaloIters2 = (kT2 + 63) / 64;   // 4
 constexpr int kUpdBlocks = 256;                // grid of the vector passes
 constexpr int kUpdThreads = 1024;
-constexpr int kIterBlocks = 1024;              // most blocks of an iteration launch
+constexpr int kIterBlocks = 768;               // most blocks of an iteration launch
 
 // 2D tile element e -> (neighbour brick 0..8) << 9 | local node; elements
 // past the tile map to the zero brick slot 9.  (3D decodes arithmetically.)
@@ -463,13 +463,18 @@ __device__ __forceinline__ void block_sums4(const double v[4], double* scratch, 
     __syncthreads();
 }
 
-// What a block of an iteration launch needs of the previous one.  Every lane
-// loads (indices past the partials read the last one): loads under a
-// condition make the compiler's waits for them cover every later load.
-template <int NT>
+// What a block of an iteration launch needs of the previous one.  Wave q < 4
+// forms sum q of the partials by itself: lane l loads the partials l, l + 64,
+// ... (U of them cover the largest launch that takes this U), sums them
+// pairwise and one DPP tree adds the lanes; every thread then forms the
+// scalars from the four sums: one barrier in all.  Measured against partials
+// spread over the whole block, summed through LDS scratch, with the scalars
+// formed by one thread (three barriers), us per launch:
+//   2D 400 4.58, now 3.63    10,605 nodes 5.20, 4.42    97,353 particles 5.25, 4.90
+//   3D 12 bricks 7.5, 7.1    270 7.65, 7.42    600 9.72, 9.55    2,411 19.2, 18.9
+template <int U>
 struct IterHead {
-    static constexpr int U = (kIterBlocks + NT - 1) / NT;
-    double v[4][U];
+    double v[U];
     double thr_rec;
     float alpha, beta;
     int stop;
@@ -480,89 +485,83 @@ struct IterHead {
         thr_rec = st->thr_rec;
         alpha = st->alpha;
         beta = st->beta;
+        const int l = threadIdx.x & 63;
+        const int q = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        if (q < 4) {
+            const double* p = q == 0 ? it.prev[0]
+                                     : (q == 1 ? it.prev[1] : (q == 2 ? it.prev[2] : it.prev[3]));
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int i = min((int)threadIdx.x + NT * u, it.nprev - 1);
-#pragma unroll
-            for (int q = 0; q < 4; q++) v[q][u] = it.prev[q][i];
+            for (int u = 0; u < U; u++) v[u] = p[min(l + 64 * u, it.nprev - 1)];
         }
     }
 };
 
-// alpha_(kk-1) and beta_kk of an iteration launch into s_ab, and s_mode: 0 go
-// on, 1 the solve ended (apply the last x update only), 2 non-finite alpha
-// (no update).  Block 0 records the state.  The caller synchronises.
-template <int NT>
-__device__ __forceinline__ void iter_scalars(const StencilArgs& a, const IterArgs& it,
-                                             const IterHead<NT>& hd, double* scratch,
-                                             double* sred, float* s_ab, int* s_mode) {
+// alpha_(kk-1) and beta_kk of an iteration launch, and the mode: 0 go on, 1
+// the solve ended (apply the last x update only), 2 non-finite alpha (no
+// update).  Block 0 records the state.  Holds one barrier.
+struct IterScalars {
+    float al, be;
+    int mode;
+};
+template <int U>
+__device__ __forceinline__ IterScalars iter_scalars(const StencilArgs& a, const IterArgs& it,
+                                                    const IterHead<U>& hd, double* sred) {
     const int t = threadIdx.x, kk = a.kk;
     if (it.resume) {
-        if (t == 0) {
-            *s_mode = 0;
-            s_ab[0] = hd.alpha;
-            s_ab[1] = hd.beta;
-        }
-        return;
+        __syncthreads();
+        return {hd.alpha, hd.beta, 0};
     }
-    double sv[4];
+    if (t < 256) {
+        const int l = t & 63;
+        double w[U];
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-        sv[q] = 0;
+        for (int u = 0; u < U; u++) w[u] = l + 64 * u < it.nprev ? hd.v[u] : 0.0;
 #pragma unroll
-        for (int u = 0; u < IterHead<NT>::U; u += 2) {
-            const double w0 = t + NT * u < it.nprev ? hd.v[q][u] : 0.0;
-            const double w1 = u + 1 < IterHead<NT>::U && t + NT * (u + 1) < it.nprev
-                                  ? hd.v[q][u + 1 < IterHead<NT>::U ? u + 1 : u] : 0.0;
-            sv[q] += w0 + w1;
-        }
+        for (int h = 1; h < U; h <<= 1)
+#pragma unroll
+            for (int u = 0; u + h < U; u += 2 * h) w[u] += w[u + h];
+        const double sum = wave_sum_all(w[0]);
+        if (l == 0) sred[t >> 6] = sum;
     }
-    // the four sums through LDS: wave w reduces sum w with one DPP tree
-    // instead of every wave reducing all four
-    block_sums4<NT>(sv, scratch, sred);
-    if (t == 0) {
+    __syncthreads();
+    const double pt = sred[0], rt = sred[1], tt = sred[2], rr = sred[3];
+    const int k = a.iter_base + kk - 1;   // Eigen's index of the reduced SpMV
+    const double ald = rr / pt;
+    const float al = (float)ald;
+    const double a64 = (double)al;   // the alpha the vectors are updated with
+    const double rn = (rr - 2.0 * a64 * rt) + a64 * a64 * tt;
+    int done = 0, iter = 0;
+    float be = 0.f;
+    if (!isfinite(ald) || !isfinite(rn)) {
+        done = 3;
+        iter = k;
+    } else if (rn < hd.thr_rec) {
+        done = 1;
+        iter = k;
+    } else if (k + 1 >= a.max_iter) {
+        done = 2;
+        iter = k + 1;
+    } else {
+        be = (float)(rn / rr);
+    }
+    if (t == 0 && blockIdx.x == 0) {
         CgState* st = a.st;
-        const double pt = sred[0], rt = sred[1], tt = sred[2], rr = sred[3];
-        const int k = a.iter_base + kk - 1;   // Eigen's index of the reduced SpMV
-        const double ald = rr / pt;
-        const float al = (float)ald;
-        const double a64 = (double)al;   // the alpha the vectors are updated with
-        const double rn = (rr - 2.0 * a64 * rt) + a64 * a64 * tt;
-        int done = 0, iter = 0;
-        float be = 0.f;
-        if (!isfinite(ald) || !isfinite(rn)) {
-            done = 3;
-            iter = k;
-        } else if (rn < hd.thr_rec) {
-            done = 1;
-            iter = k;
-        } else if (k + 1 >= a.max_iter) {
-            done = 2;
-            iter = k + 1;
+        st->alpha = al;
+        st->pt = pt;
+        st->rr_prev = rr;
+        st->rr = rn;
+        if (done) {
+            st->iter = iter;
+            st->done = done;
+            __hip_atomic_store(&st->stop, kk + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
-            be = (float)(rn / rr);
-        }
-        *s_mode = done == 0 ? 0 : (done == 3 ? 2 : 1);
-        s_ab[0] = al;
-        s_ab[1] = be;
-        if (blockIdx.x == 0) {
-            st->alpha = al;
-            st->pt = pt;
-            st->rr_prev = rr;
-            st->rr = rn;
-            if (done) {
-                st->iter = iter;
-                st->done = done;
-                __hip_atomic_store(&st->stop, kk + 1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                st->beta = be;
-            }
+            st->beta = be;
         }
     }
+    return {al, be, done == 0 ? 0 : (done == 3 ? 2 : 1)};
 }
 
-template <int OP, int NT>
+template <int OP, int NT, int U>
 __global__ void __launch_bounds__(NT) k_cg_iter3(StencilArgs a, CoefF cc, IterArgs it,
                                                           const int32_t* __restrict__ order) {
     constexpr int UI = (kUnits + NT - 1) / NT;   // 16-byte loads per thread and array
@@ -576,14 +575,12 @@ __global__ void __launch_bounds__(NT) k_cg_iter3(StencilArgs a, CoefF cc, IterAr
     __shared__ __align__(16) float own[kOwnX];
     __shared__ __align__(16) float own_r[kOwnX];
     __shared__ uint32_t sbase[2][27];
-    __shared__ double sred[4][4];
-    __shared__ float s_ab[2];
-    __shared__ int s_mode;
+    __shared__ double sred[2][4];
     const int kk = a.kk;
     const int t = threadIdx.x;
     // everything the prologue reads goes out at once, this block's first
     // slots included
-    IterHead<NT> hd;
+    IterHead<U> hd;
     hd.load(a, it);
     const int l = t & 63, wv = t >> 6;
     const int x = l & 7, y = l >> 3;
@@ -641,10 +638,9 @@ __global__ void __launch_bounds__(NT) k_cg_iter3(StencilArgs a, CoefF cc, IterAr
             }
         }
     };
-    iter_scalars<NT>(a, it, hd, reinterpret_cast<double*>(tile), sred[0], s_ab, &s_mode);
-    __syncthreads();
-    const int mode = s_mode;
-    const float al = s_ab[0], be = s_ab[1];
+    const IterScalars sc = iter_scalars(a, it, hd, sred[0]);
+    const int mode = sc.mode;
+    const float al = sc.al, be = sc.be;
     if (mode == 2) return;   // non-finite alpha: no update
     if (mode == 1) {
         // the solve ended: the last x update only (own nodes of every brick)
@@ -865,19 +861,17 @@ __global__ void __launch_bounds__(64) k_stencil2(StencilArgs a, C cc) {
 // 2D CG iteration: one launch per iteration as in 3D.  A 2D system has few
 // nodes, so an iteration is bound by launches and dependent loads, not by
 // bandwidth: an SpMV and an update launch (6.7 + 4.1 us and two gaps at
-// 10,605 nodes) became one of 5.0 us.  One wave per 8x8 brick
+// 10,605 nodes) became one of 4.4 us.  One wave per 8x8 brick
 // (four bricks to a block, further bricks grid-strided).  The 14x14 halo is
 // 14 rows of four 16-byte half rows, 56 units: one unit of p, r and t per
 // lane, all issued before the previous launch's sums are formed.  Each wave
 // keeps its tile to itself, so no barrier is needed between its stages.
-template <int OP>
+template <int OP, int U>
 __global__ void __launch_bounds__(256) k_cg_iter2(StencilArgs a, CoefF cc, IterArgs it) {
     __shared__ __align__(16) float tile[4][kT * kRS];
     __shared__ double scratch[4 * 256];
     __shared__ double sred[2][4];
-    __shared__ float s_ab[2];
-    __shared__ int s_mode;
-    IterHead<256> hd;
+    IterHead<U> hd;
     hd.load(a, it);
     const int l = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int nsl = (int)a.nslots, G = (int)gridDim.x;
@@ -908,10 +902,9 @@ __global__ void __launch_bounds__(256) k_cg_iter2(StencilArgs a, CoefF cc, IterA
         Tt = a.in3[o];
     };
     issue(min(b0, nsl - 1), nbs);
-    iter_scalars<256>(a, it, hd, scratch, sred[0], s_ab, &s_mode);
-    __syncthreads();
-    const int mode = s_mode;
-    const float al = s_ab[0], be = s_ab[1];
+    const IterScalars sc = iter_scalars(a, it, hd, sred[0]);
+    const int mode = sc.mode;
+    const float al = sc.al, be = sc.be;
     if (mode == 2) return;   // non-finite alpha: no update
     double rsum[4] = {0, 0, 0, 0};
     float* tl = tile[wv];
@@ -1302,20 +1295,34 @@ static IterLaunch iter_launch(const vps_context* c, int nslots) {
     const bool row = c->p.op_mode == VPS_OP_ROW;
     IterLaunch L;
     int work, per_cu;
+    bool wide = false;
     if (c->dim == 2) {
-        L.kern2 = row ? k_cg_iter2<VPS_OP_ROW> : k_cg_iter2<VPS_OP_TRANSPOSE>;
         work = (nslots + 3) / 4;
         per_cu = 3;
     } else {
-        const bool wide = nslots <= 12 * cus;
-        if (wide) L.kern3 = row ? k_cg_iter3<VPS_OP_ROW, 512> : k_cg_iter3<VPS_OP_TRANSPOSE, 512>;
-        else L.kern3 = row ? k_cg_iter3<VPS_OP_ROW, 256> : k_cg_iter3<VPS_OP_TRANSPOSE, 256>;
+        wide = nslots <= 12 * cus;
         L.threads = wide ? 512 : 256;
         work = nslots;
         per_cu = !wide ? 3 : (4 * nslots <= 5 * cus ? 1 : 2);
     }
-    const int most = std::min(kIterBlocks, per_cu * cus);
+    const int most = std::min(wide ? 512 : kIterBlocks, per_cu * cus);
     L.blocks = work >= 8 ? std::max(8, std::min(work, most) & ~7) : work;
+    // loads per lane of the previous launch's partials (64 lanes a sum)
+    auto pick = [&](auto t, auto r) { return row ? r : t; };
+    if (c->dim == 2)
+        L.kern2 = L.blocks <= 64
+                      ? pick(k_cg_iter2<VPS_OP_TRANSPOSE, 1>, k_cg_iter2<VPS_OP_ROW, 1>)
+                      : (L.blocks <= 512
+                             ? pick(k_cg_iter2<VPS_OP_TRANSPOSE, 8>, k_cg_iter2<VPS_OP_ROW, 8>)
+                             : pick(k_cg_iter2<VPS_OP_TRANSPOSE, 12>, k_cg_iter2<VPS_OP_ROW, 12>));
+    else if (!wide)
+        L.kern3 = pick(k_cg_iter3<VPS_OP_TRANSPOSE, 256, 12>, k_cg_iter3<VPS_OP_ROW, 256, 12>);
+    else if (L.blocks <= 64)
+        L.kern3 = pick(k_cg_iter3<VPS_OP_TRANSPOSE, 512, 1>, k_cg_iter3<VPS_OP_ROW, 512, 1>);
+    else if (L.blocks <= 256)
+        L.kern3 = pick(k_cg_iter3<VPS_OP_TRANSPOSE, 512, 4>, k_cg_iter3<VPS_OP_ROW, 512, 4>);
+    else
+        L.kern3 = pick(k_cg_iter3<VPS_OP_TRANSPOSE, 512, 8>, k_cg_iter3<VPS_OP_ROW, 512, 8>);
     return L;
 }
 
