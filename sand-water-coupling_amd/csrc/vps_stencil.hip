@@ -425,8 +425,8 @@ __global__ void __launch_bounds__(kS3Threads) k_stencil3(StencilArgs a, C cc) {
 // reaches the same alpha_(kk-1) = r.r / p.t, the r.r after the update
 // (expanded as r.r - 2 alpha r.t + alpha^2 t.t, anchored every iteration on
 // the direct r.r of the stored r), Eigen's test on it and beta_kk
-// without a reduction launch in between (about 1K partials per set, one
-// round of loads).  Then per brick: x += alpha p_old, r = r_old - alpha t_old,
+// without a reduction launch in between (at most kIterBlocks partials a
+// set, one round of loads).  Then per brick: x += alpha p_old, r = r_old - alpha t_old,
 // p = r + beta p_old, t = M p with k_stencil3's tile and plane sums, and one partial
 // per block of p.t, r.t, t.t and r.r.  A brick that sits on the block's
 // previous brick shares 6 of its 14 halo planes with it: their plane sums
@@ -445,6 +445,8 @@ struct IterArgs {
 // values go through LDS scratch (32 NT bytes), wave w < 4 adds the values of
 // lanes l, l + 64, ... of sum w pairwise and reduces them with one DPP tree;
 // out[w] (LDS) holds sum w for the whole block afterwards.
+// (Every wave reducing all four by DPP, with one barrier less: 3.72 against
+// 3.63 us a launch in 2D at 400 particles, 9.85 against 9.55 at 600 bricks.)
 template <int NT>
 __device__ __forceinline__ void block_sums4(const double v[4], double* scratch, double* out) {
     const int t = threadIdx.x, l = t & 63, wv = t >> 6;
@@ -1271,6 +1273,7 @@ struct IterLaunch {
 // The 3D rule, from launches timed at 12, 270, 600, 2,411 and 18,720 bricks
 // (us per launch, 256 threads and three blocks per CU against 512 threads):
 //   8.96 / 7.8   9.5 / 7.75   10.2 / 9.9   20.7 / 20.2   118 / 137
+// (with the head of one barrier 7.1, 7.4, 9.55, 18.9 and 112).
 // Up to a few bricks per block the launch is one chain of loads, sums and
 // barriers, which 512 threads per brick shorten (two rounds of loads and
 // plane sums instead of four); with a dozen bricks per CU and more the
