@@ -89,11 +89,6 @@ __device__ __forceinline__ double sq_dist2(double ax, double ay, double bx,
     const double dx = ax - bx, dy = ay - by;
     return dx * dx + dy * dy;
 }
-template <int D>
-__device__ __forceinline__ double sq_dist(const double* a, const double* b) {
-    if constexpr (D == 2) return sq_dist2(a[0], a[1], b[0], b[1]);
-    else return sq_dist3(a[0], a[1], a[2], b[0], b[1], b[2]);
-}
 __device__ __forceinline__ double dsub(double a, double b) {
 #pragma clang fp contract(off)
     return a - b;
@@ -145,19 +140,13 @@ __device__ __forceinline__ KW kernel_f32(double d2, double kr2, float kr,
     return o;
 }
 
-// FP32 cubic spline from x = r / kr (valid for 0 <= x): W and
+// FP32 cubic spline from x = r / kr (valid for 0 <= x):
 // S = -W'(r) / r, the factor of gradK(d) = S d, without divisions
 // (SmoothedParticles.h:60-72: W' = c1 x (3x - 2) below x = 1/2, so
 // -W'/r = c1 (2 - 3x) / kr there; -c1 (1 - x)^2 above, so -W'/r =
 // c1 (1 - x)^2 / r).  rinv = 1 / r is only used for x >= 1/2.
 // Both pieces are evaluated and selected (no branch: the lanes of a wave
 // mix both sides); max(1 - x, 0) makes the outer piece vanish for x >= 1.
-__device__ __forceinline__ float spline_w(float x, float c0) {
-    const float in = c0 * (6.f * x * x * (x - 1.f) + 1.f);
-    const float omx = fmaxf(1.f - x, 0.f);
-    const float out = 2.f * c0 * omx * omx * omx;
-    return x < 0.5f ? in : out;
-}
 __device__ __forceinline__ float spline_s(float x, float rinv, float c1,
                                           float inv_kr) {
     const float in = c1 * inv_kr * (2.f - 3.f * x);
@@ -185,20 +174,6 @@ __device__ __forceinline__ float spline_w_ab(SplineAB s, float c0) {
 }
 __device__ __forceinline__ float spline_s_ab(SplineAB s, float rinv, float c1) {
     return c1 * rinv * fmaf(s.a, s.a, -(s.b * s.b));
-}
-
-// Candidate masks of an FP32 pre-test on cell-relative offsets (w < 0 marks
-// a particle clamped into a border cell): `fast` inside h by the FP32 band,
-// `exact` where the FP64 test decides (the band around h^2, r = 0, clamped
-// particles); neither: outside h.
-struct Pretest {
-    bool fast, exact;
-};
-__device__ __forceinline__ Pretest pretest(const KConst& k, float d2f, float w) {
-    const bool ok = w >= 0.f;
-    const bool fast = ok & (d2f > 0.f) & (d2f < k.h2f_lo);
-    const bool exact = !fast & (!ok | (d2f < k.h2f_hi));
-    return Pretest{fast, exact};
 }
 
 // ---- launch geometry ----------------------------------------------------

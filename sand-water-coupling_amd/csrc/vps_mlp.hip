@@ -791,7 +791,8 @@ __global__ void __launch_bounds__(256) k_mlp_train(
 
 // Sum of the per-block partials (fixed order).  Block = 16 parameters x 16
 // row groups; a thread sums rows g, g + 16, ... of its parameter (16 of 256,
-// all loads in flight), the groups are added pairwise.
+// all loads in flight), the groups are added pairwise.  4.5 us for 256 rows
+// (5.1 with 64 parameters x 4 groups a block).
 constexpr int kRedParams = 16;
 __global__ void __launch_bounds__(256) k_mlp_reduce(
     const float* grad_part, int nrows, const double* loss_part, float* grad,

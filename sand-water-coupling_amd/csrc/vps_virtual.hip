@@ -466,8 +466,8 @@ inline int sums_lanes(int64_t n) {
     return n <= 16000 ? 8 : (n <= 32000 ? 4 : (n <= 250000 ? 2 : 1));
 }
 
-// Bound by instructions and the latency of the walk (of 280 us at 1M: staging
-// 45, candidate tests 105, sums 85, boundary 45).  Before (one lane per node
+// Bound by instructions and the latency of the walk (of 264 us at 1M:
+// staging about 40, candidate tests 100, sums 80, boundary 45).  Before (one lane per node
 // for all sizes, the boundary walked in global memory, two masks per test,
 // rows staged through a binary search): 70 us at 576 particles, 77 at 64,800,
 // 120 at 212,503, 297 at 1,012,500.
