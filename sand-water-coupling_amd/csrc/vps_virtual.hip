@@ -435,7 +435,8 @@ struct StagedRows {
         const bool cut_l = xlo < xhi && xlo > 0, cut_r = xhi > xlo && xhi < k.cdims[0] - 1;
         const float gl = gap((float)(qx - cell_corner(k, 0, xlo)));
         const float gr = gap((float)(qx - cell_corner(k, 0, xhi)));
-        const float dl2 = cut_l ? gl * gl : 1e30f, dr2 = cut_r ? gr * gr : 1e30f;
+        // (0: the cell stays; rem below is positive)
+        const float dl2 = cut_l ? gl * gl : 0.f, dr2 = cut_r ? gr * gr : 0.f;
         for (int z = zlo; z <= zhi; z++) {
             const float tz = (float)(qz - cell_corner(k, 2, z));
             const float gz = z > 0 && z < k.cdims[2] - 1 ? gap(tz) : 0.f;
