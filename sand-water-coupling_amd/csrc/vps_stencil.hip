@@ -1582,6 +1582,15 @@ int cg_solve(vps_context* c, vps_stats* stats) {
                      std::to_string(kMaxReplacements) + " residual replacements";
             return finish(VPS_ERR_NO_CONVERGENCE);
         }
+        if (!three && hs.iter > iter_base && hs.iter + 1 >= max_iter) {
+            // going on from here would be an iteration beyond the limit (in
+            // 3D, where one may bring the solve home, it is still taken)
+            hs.iter++;
+            hs.rr = hs.true_rr;
+            hs.true_rr = -1.0;
+            hs.done = 2;
+            break;
+        }
         replacements++;
         // the correction so far goes into the FP64 base; the iteration goes
         // on with a fresh FP32 correction from the true residual
