@@ -463,8 +463,12 @@ struct StagedRows {
 //   32,000        54, 35, 33, 47     64,800  59, 45, 55, 71
 //   212,503       94, 90, 112, 153   300,000 112, 116, 147, 219
 //   1,012,500    264, 274, 382, 558
-inline int sums_lanes(int64_t n) {
-    return n <= 16000 ? 8 : (n <= 32000 ? 4 : (n <= 250000 ? 2 : 1));
+// A launch holds less than 2^32 threads, and the first generation's grid covers
+// every brick: the largest lattices take fewer lanes.
+inline int sums_lanes(int64_t n, int64_t nbricks) {
+    int lanes = n <= 16000 ? 8 : (n <= 32000 ? 4 : (n <= 250000 ? 2 : 1));
+    while (nbricks * 512 * lanes > (int64_t)UINT32_MAX) lanes /= 2;
+    return lanes;
 }
 
 // Bound by instructions and the latency of the walk (of 264 us at 1M:
@@ -866,7 +870,7 @@ static int generate_slots(vps_context* c, int w, int64_t grid, bool first) {
                                c->bvel.p, c->bnrm.p, c->bcell_start.p, c->vrho.p, c->vvol.p,
                                c->vb.p, c->bits.p);
         };
-        const int lanes = sums_lanes(c->n);
+        const int lanes = sums_lanes(c->n, c->nbricks);
         if (lanes == 8) run(k_virtual_sums3s<8>, 8);
         else if (lanes == 4) run(k_virtual_sums3s<4>, 4);
         else if (lanes == 2) run(k_virtual_sums3s<2>, 2);
