@@ -22,6 +22,7 @@
 //      and a popcount scan, so every node knows its index in the reference's
 //      virtual list without the list ever being materialised.
 #include <algorithm>
+#include <cmath>
 
 #include "vps_scan.h"
 
@@ -950,13 +951,13 @@ int virtual_generate(vps_context* c) {
                         AssignSlot{c->brick_flag.p, c->brick_slot[w].p, c->slot_brick[w].p},
                         c->nbricks, (int32_t*)dcnt));
     // The slot count stays on the device: the slot passes run on a grid
-    // sized from the last generation's count (all bricks the first time),
-    // and again on the exact grid in the rare step where it grew past that.
-    int64_t grid = c->nbricks;
-    if (c->nslots > 0) {
-        grid = c->nslots + c->nslots / 8 + 64;
-        if (grid > c->nbricks) grid = c->nbricks;
-    }
+    // sized from the last generation's count (the first time by the bricks
+    // that the particles can mark at most, see k_mark_bricks), and again on
+    // the exact grid in the rare step where it grew past that.
+    double most = (double)c->n;
+    for (int a = 0; a < D; a++) most *= std::floor((2 * c->k.h / c->k.spacing + 2) / kBrick) + 2;
+    if (c->nslots > 0) most = (double)(c->nslots + c->nslots / 8 + 64);
+    const int64_t grid = (int64_t)std::min(most, (double)c->nbricks);
     VPS_TRY(generate_slots(c, w, grid, true));
     int64_t nslots = *(int32_t*)c->host_counters;
     if (nslots > grid) {
