@@ -336,12 +336,14 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
             rvel[p] = v;
         }
     };
-    const bool over_nodes = e0 * e1 * e2 > kGradCap;
+    // (extents one by one first: the product of three may not fit 64 bits)
+    const bool over_nodes =
+        e0 > kGradCap || e1 > kGradCap || e2 > kGradCap || e0 * e1 * e2 > kGradCap;
     // the bricks the box touches (floor division by 8, also below zero)
     const int bx0 = lo0 >> 3, by0 = lo1 >> 3, bz0 = lo2 >> 3;
-    const int nbx = ((lo0 + (int)e0 - 1) >> 3) - bx0 + 1;
-    const int nby = ((lo1 + (int)e1 - 1) >> 3) - by0 + 1;
-    const int nbz = ((lo2 + (int)e2 - 1) >> 3) - bz0 + 1;
+    const int nbx = (int)((lo0 + e0 - 1) >> 3) - bx0 + 1;
+    const int nby = (int)((lo1 + e1 - 1) >> 3) - by0 + 1;
+    const int nbz = (int)((lo2 + e2 - 1) >> 3) - bz0 + 1;
     if (over_nodes || nbx * nby * nbz > kGradBoxBricks) {
         beyond_stage();
         return;
