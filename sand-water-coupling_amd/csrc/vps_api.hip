@@ -495,6 +495,8 @@ int vps_create(const vps_params* params, vps_context** out) {
             hipMemset(c->counters.p, 0, 64 * sizeof(int64_t)) != hipSuccess ||
             // counting arrays start at zero; their consumers clear them again
             hipMemset(c->cell_count.p, 0, (size_t)(c->ncells + 1) * 4) != hipSuccess ||
+            // (no particles in any cell before the first sort)
+            hipMemset(c->cell_start.p, 0, (size_t)(c->ncells + 1) * 4) != hipSuccess ||
             hipMemset(c->brick_flag.p, 0, (size_t)c->nbricks * 4) != hipSuccess ||
             hipMemset(c->vq.p, 0, cap * 4) != hipSuccess ||
             hipMemset(c->vrho.p, 0, cap * 4) != hipSuccess ||
@@ -1057,7 +1059,8 @@ int vps_debug_apply_operator(vps_context* c, const double* p, double* out) {
 int vps_debug_member_counts(vps_context* c, int32_t which, int32_t* counts) {
     if (!c || !counts || which < 0 || which > 3) return VPS_ERR_INVALID_ARG;
     if (c->dim != 3) return fail(c, VPS_ERR_INVALID_ARG, "member counts are 3D only");
-    if (which == 2 && (c->nslots == 0 || !c->grad_staged))
+    // (a new particle set leaves the last one's units behind)
+    if (which == 2 && (!c->initialized || c->nslots == 0 || !c->grad_staged))
         return fail(c, VPS_ERR_STATE, "no virtual set or no staged gradient");
     const int64_t n = which == 1 ? c->nb : c->n;
     if (n == 0) return VPS_OK;
