@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(256) k_density2(const double4* pos,
 // Off: the type of the candidates' byte offsets (uint32_t when the set's
 // offsets fit, so the loads take a scalar base and a 32-bit lane offset).
 // CNT (test support): only the number of terms that enter the sum (a > 0: r < h,
-// where the spline is nonzero) into members[i].
+// where the spline is nonzero) into members[i], with the lanes of a run.
 // L: lanes of a wave that share a particle, each taking every L-th candidate
 // of a row; their sums meet in a butterfly.  One lane per particle is the
 // least work; with few particles the machine is not full, and the time is that
@@ -209,7 +209,9 @@ __global__ void __launch_bounds__(256) k_density3f(const double4* pos, const flo
             }
     });
     if constexpr (CNT) {
-        members[i] = nterms;
+#pragma unroll
+        for (int o = 1; o < L; o <<= 1) nterms += __shfl_xor(nterms, o, 64);
+        if (sub == 0) members[i] = nterms;
         return;
     }
 #pragma unroll
@@ -352,23 +354,31 @@ int cells_sort_boundary(vps_context* c) {
     return VPS_OK;
 }
 
+// 3D density of the real particles; CNT: its terms instead, into members.
+template <bool CNT>
+static void real_density3(vps_context* c, bool set_volume, int32_t* members) {
+    const int64_t n = c->n;
+    const int s = c->cur;
+    auto run = [&](auto kern, int lanes) {
+        hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
+                           c->rpos[s].p, c->rofs.p, c->cell_start.p, n, c->k, c->rrho.p,
+                           c->rrinv.p, (float4*)nullptr, c->rvel[s].p, set_volume ? 1 : 0,
+                           members);
+    };
+    const int lanes = walk_lanes(n);
+    if (lanes == 8) run(k_density3f<false, uint32_t, 8, CNT>, 8);
+    else if (lanes == 4) run(k_density3f<false, uint32_t, 4, CNT>, 4);
+    else if (lanes == 2) run(k_density3f<false, uint32_t, 2, CNT>, 2);
+    else if (n * 16 <= (int64_t)UINT32_MAX) run(k_density3f<false, uint32_t, 1, CNT>, 1);
+    else run(k_density3f<false, uint64_t, 1, CNT>, 1);
+}
+
 // Densities of the real particles, after their sort (3D: with its offsets).
 int real_density(vps_context* c, bool set_volume) {
     const int64_t n = c->n;
     const int s = c->cur;
     if (c->dim == 3) {
-        auto run = [&](auto kern, int lanes) {
-            hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
-                               c->rpos[s].p, c->rofs.p, c->cell_start.p, n, c->k, c->rrho.p,
-                               c->rrinv.p, (float4*)nullptr, c->rvel[s].p, set_volume ? 1 : 0,
-                               (int32_t*)nullptr);
-        };
-        const int lanes = walk_lanes(n);
-        if (lanes == 8) run(k_density3f<false, uint32_t, 8>, 8);
-        else if (lanes == 4) run(k_density3f<false, uint32_t, 4>, 4);
-        else if (lanes == 2) run(k_density3f<false, uint32_t, 2>, 2);
-        else if (n * 16 <= (int64_t)UINT32_MAX) run(k_density3f<false, uint32_t, 1>, 1);
-        else run(k_density3f<false, uint64_t, 1>, 1);
+        real_density3<false>(c, set_volume, nullptr);
     } else {
         auto run = [&](auto kern, int lanes) {
             hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
@@ -399,13 +409,8 @@ int density_member_counts(vps_context* c, int which, int32_t* members) {
     const int64_t n = which == 0 ? c->n : c->nb;
     if (n == 0) return VPS_OK;
     if (which == 0) {
-        const int s = c->cur;
-        hipLaunchKernelGGL(k_cell_offsets3, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
-                           c->rpos[s].p, n, c->k, c->rofs.p);
-        hipLaunchKernelGGL((k_density3f<false, uint64_t, 1, true>), dim3(blocks(n, 256)),
-                           dim3(256), 0, c->stream, c->rpos[s].p, c->rofs.p, c->cell_start.p,
-                           n, c->k, (float*)nullptr, (float*)nullptr, (float4*)nullptr,
-                           (float4*)nullptr, 0, members);
+        VPS_TRY(real_offsets(c));
+        real_density3<true>(c, false, members);
     } else {
         DBuf<float4> ofs;
         VPS_TRY(dalloc(c, ofs, (size_t)n));

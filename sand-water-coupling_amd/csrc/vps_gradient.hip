@@ -485,7 +485,9 @@ __global__ void __launch_bounds__(kGradThreads, 4) k_gradient3s(
             fz *= c1;
         }
         if constexpr (CNT) {
-            members[p] = nterms;
+#pragma unroll
+            for (int o = 1; o < L; o <<= 1) nterms += __shfl_xor(nterms, o, 64);
+            if (sub == 0) members[p] = nterms;
             continue;
         }
         if (s_walls) boundary_term<3, L>(k, q, vi, bpos, bvel, bnrm, bcstart, fx, fy, fz, sub);
@@ -640,16 +642,28 @@ UnitArgs gradient_units(vps_context* c, bool append) {
     return a;
 }
 
+// The staged gradient on the units of the last generation; CNT: its terms
+// instead (q the volumes), into members.
+template <bool CNT>
+static void gradient3s(vps_context* c, const float* q, SolveGuard g, int32_t* members) {
+    if (c->grad_nunits == 0) return;
+    auto run = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)c->grad_nunits), dim3(kGradThreads), 0, c->stream,
+                           c->k, c->grad_shape, (int)c->grad_nunits, c->rpos[c->cur].p,
+                           c->rvel[c->cur].p, c->brick_slot[c->which].p, q, c->bpos.p, c->bvel.p,
+                           c->bnrm.p, c->bcell_start.p, g, members);
+    };
+    const int lanes = unit_rule(c->n).lanes;
+    if (lanes == 8) run(k_gradient3s<8, CNT>);
+    else if (lanes == 4) run(k_gradient3s<4, CNT>);
+    else run(k_gradient3s<1, CNT>);
+}
+
 // Terms of the staged gradient's virtual walk per real particle (test
 // support, sorted order; -1 stays where a unit exceeds the stage).
 int gradient_member_counts(vps_context* c, int32_t* members) {
     if (c->dim != 3 || !c->grad_staged || c->nslots == 0) return VPS_ERR_INVALID_ARG;
-    if (c->grad_nunits > 0)
-        hipLaunchKernelGGL((k_gradient3s<1, true>), dim3((unsigned)c->grad_nunits),
-                           dim3(kGradThreads), 0, c->stream, c->k, c->grad_shape,
-                           (int)c->grad_nunits, c->rpos[c->cur].p, c->rvel[c->cur].p,
-                           c->brick_slot[c->which].p, c->vvol.p, c->bpos.p, c->bvel.p,
-                           c->bnrm.p, c->bcell_start.p, SolveGuard{}, members);
+    gradient3s<true>(c, c->vvol.p, SolveGuard{}, members);
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;
 }
@@ -659,19 +673,7 @@ int pressure_gradient(vps_context* c, SolveGuard g) {
     const int s = c->cur;
     const int w = c->which;
     if (c->dim == 3 && c->grad_staged) {
-        if (c->grad_nunits > 0) {
-            auto run = [&](auto kern) {
-                hipLaunchKernelGGL(kern, dim3((unsigned)c->grad_nunits), dim3(kGradThreads), 0,
-                                   c->stream, c->k, c->grad_shape, (int)c->grad_nunits,
-                                   c->rpos[s].p, c->rvel[s].p, c->brick_slot[w].p, c->vq.p,
-                                   c->bpos.p, c->bvel.p, c->bnrm.p, c->bcell_start.p, g,
-                                   (int32_t*)nullptr);
-            };
-            const int lanes = unit_rule(n).lanes;
-            if (lanes == 8) run(k_gradient3s<8>);
-            else if (lanes == 4) run(k_gradient3s<4>);
-            else run(k_gradient3s<1>);
-        }
+        gradient3s<false>(c, c->vq.p, g, nullptr);
     } else {
         auto run = [&](auto kern, int lanes) {
             hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream, c->k,

@@ -160,7 +160,9 @@ __global__ void __launch_bounds__(256) k_viscosity3f(const double4* pos, const f
         }
     });
     if constexpr (CNT) {
-        members[i] = nterms;
+#pragma unroll
+        for (int o = 1; o < L; o <<= 1) nterms += __shfl_xor(nterms, o, 64);
+        if (sub == 0) members[i] = nterms;
         return;
     }
 #pragma unroll
@@ -248,6 +250,23 @@ int apply_gravity(vps_context* c, double dt, double g) {
     return VPS_OK;
 }
 
+// 3D viscosity into vel_next; CNT: its terms instead, into members.
+template <bool CNT>
+static void viscosity3(vps_context* c, float scale, int32_t* members) {
+    const int64_t n = c->n;
+    const int s = c->cur;
+    auto run = [&](auto kern, int lanes) {
+        hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
+                           c->rpos[s].p, c->rofs.p, c->cell_start.p, c->rvel[s].p, c->rrho.p, n,
+                           c->k, scale, c->vel_next.p, members);
+    };
+    const int lanes = walk_lanes(n);
+    if (lanes == 8) run(k_viscosity3f<8, CNT>, 8);
+    else if (lanes == 4) run(k_viscosity3f<4, CNT>, 4);
+    else if (lanes == 2) run(k_viscosity3f<2, CNT>, 2);
+    else run(k_viscosity3f<1, CNT>, 1);
+}
+
 // Terms of the 3D viscosity walk per real particle (test support, sorted
 // order), on offsets recomputed from the current positions.
 int viscosity_member_counts(vps_context* c, int32_t* members) {
@@ -255,10 +274,7 @@ int viscosity_member_counts(vps_context* c, int32_t* members) {
     if (c->dim != 3) return VPS_ERR_INVALID_ARG;
     if (n == 0) return VPS_OK;
     VPS_TRY(real_offsets(c));
-    const int s = c->cur;
-    hipLaunchKernelGGL((k_viscosity3f<1, true>), dim3(blocks(n, 256)), dim3(256), 0, c->stream,
-                       c->rpos[s].p, c->rofs.p, c->cell_start.p, c->rvel[s].p, c->rrho.p, n,
-                       c->k, 0.f, (float4*)nullptr, members);
+    viscosity3<true>(c, 0.f, members);
     VPS_HIP(c, hipGetLastError());
     return VPS_OK;
 }
@@ -274,16 +290,7 @@ int apply_viscosity(vps_context* c, double dt, double nu) {
     // v += nu lapl dt with lapl = 2 (Dim + 2) m sum(...)
     const float scale = (float)(nu * (2.0 * (c->dim + 2.0) * c->p.mass) * dt);
     if (c->dim == 3) {
-        auto run = [&](auto kern, int lanes) {
-            hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
-                               c->rpos[s].p, c->rofs.p, c->cell_start.p, c->rvel[s].p, c->rrho.p,
-                               n, c->k, scale, c->vel_next.p, (int32_t*)nullptr);
-        };
-        const int lanes = walk_lanes(n);
-        if (lanes == 8) run(k_viscosity3f<8>, 8);
-        else if (lanes == 4) run(k_viscosity3f<4>, 4);
-        else if (lanes == 2) run(k_viscosity3f<2>, 2);
-        else run(k_viscosity3f<1>, 1);
+        viscosity3<false>(c, scale, nullptr);
     } else {
         auto run = [&](auto kern, int lanes) {
             hipLaunchKernelGGL(kern, dim3(blocks(n * lanes, 256)), dim3(256), 0, c->stream,
