@@ -36,13 +36,16 @@ __global__ void __launch_bounds__(256) k_check_finite(int64_t n, const double* a
     if (bad) *flag = 1;
 }
 
-// Caller-order FP64 arrays (either may be null) from the cell-sorted state.
-__global__ void __launch_bounds__(256) k_download(int64_t n, int dim, const int32_t* id,
-                                                  const double4* pos, const float4* vel,
-                                                  double* x, double* v) {
+// Caller-order FP64 arrays (either may be null) from the cell-sorted state:
+// the particles of ids first .. first + m - 1.
+__global__ void __launch_bounds__(256) k_download(int64_t n, int64_t first, int64_t m, int dim,
+                                                  const int32_t* id, const double4* pos,
+                                                  const float4* vel, double* x, double* v) {
     const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= n) return;
-    const int64_t i = (int64_t)id[k] * dim;
+    const int64_t j = id[k] - first;
+    if (j < 0 || j >= m) return;
+    const int64_t i = j * dim;
     if (x) {
         const double4 p = pos[k];
         x[i] = p.x;
@@ -57,26 +60,28 @@ __global__ void __launch_bounds__(256) k_download(int64_t n, int dim, const int3
     }
 }
 
-__global__ void k_upload(int64_t n, int dim, const double* x, const double* v,
+// The m particles from `first` on of a new set.
+__global__ void k_upload(int64_t first, int64_t m, int dim, const double* x, const double* v,
                          double4* pos, float4* vel, int32_t* id) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    pos[i] = make_double4(x[dim * i], x[dim * i + 1], dim == 3 ? x[dim * i + 2] : 0.0, 0.0);
-    vel[i] = v ? make_float4((float)v[dim * i], (float)v[dim * i + 1],
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, k = first + i;
+    if (i >= m) return;
+    pos[k] = make_double4(x[dim * i], x[dim * i + 1], dim == 3 ? x[dim * i + 2] : 0.0, 0.0);
+    vel[k] = v ? make_float4((float)v[dim * i], (float)v[dim * i + 1],
                              dim == 3 ? (float)v[dim * i + 2] : 0.f, 0.f)
                : make_float4(0.f, 0.f, 0.f, 0.f);
-    id[i] = (int32_t)i;
+    id[k] = (int32_t)k;
 }
 
 // Overwrites x and v of the resident (cell-sorted) state from caller-order
-// arrays, keeping the frozen volumes; nothing when the arrays held a
-// non-finite value.
-__global__ void k_upload_resident(int64_t n, int dim, const double* x,
-                                  const double* v, const int32_t* id,
-                                  double4* pos, float4* vel, const int32_t* bad) {
+// arrays of the ids first .. first + m - 1, keeping the frozen volumes; nothing
+// when the arrays held a non-finite value.
+__global__ void k_upload_resident(int64_t n, int64_t first, int64_t m, int dim, const double* x,
+                                  const double* v, const int32_t* id, double4* pos, float4* vel,
+                                  const int32_t* bad) {
     const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (k >= n || *bad) return;
-    const int64_t i = id[k];
+    const int64_t i = id[k] - first;
+    if (i < 0 || i >= m) return;
     pos[k] = make_double4(x[dim * i], x[dim * i + 1], dim == 3 ? x[dim * i + 2] : 0.0, 0.0);
     if (v) {
         float4 u = vel[k];
@@ -271,13 +276,19 @@ int ensure_particle_capacity(vps_context* c, int64_t n) {
     return VPS_OK;
 }
 
-// Staging of the host state: n * dim positions, then n * dim velocities, on
-// the device; two pinned pieces of at most kIoPiece bytes on the host (512 KB:
-// as fast as 2 MB, and a context's first read-back, which touches them first,
-// takes 0.5 ms longer instead of 1.3).
+// Staging of the host state: positions, then velocities of at most io_pass
+// particles, on the device; two pinned pieces of at most kIoPiece bytes on the
+// host (512 KB: as fast as 2 MB, and a context's first read-back, which touches
+// them first, takes 0.5 ms longer instead of 1.3).  Both stay with the context,
+// so the device part is bounded: beyond 512 MB (11 million particles in 3D) a
+// set goes in several passes, each a scan of the ids (about 0.1 ms).
 constexpr size_t kIoPiece = (size_t)512 << 10;
+constexpr size_t kIoStage = (size_t)512 << 20;
+int64_t io_pass(const vps_context* c, int64_t n) {
+    return std::min(n, (int64_t)(kIoStage / (2 * c->dim * sizeof(double))));
+}
 int ensure_io(vps_context* c, int64_t n) {
-    const size_t count = (size_t)n * 2 * c->dim;
+    const size_t count = (size_t)io_pass(c, n) * 2 * c->dim;
     VPS_TRY(dalloc(c, c->io_stage, count));
     const size_t piece = std::min(kIoPiece, count * sizeof(double));
     if (c->io_host_piece < piece) {
@@ -603,31 +614,48 @@ int vps_set_particles(vps_context* c, int64_t n, const double* x,
     if (n > ((int64_t)1 << 31) - 1)
         return fail(c, VPS_ERR_INVALID_ARG, "particles: too many");
     const int D = c->dim;
+    const int64_t pass = io_pass(c, n);
+    // one pass: checked on the device; several: before the first
+    if (pass < n && (!finite_all(x, n * D) || (v && !finite_all(v, n * D))))
+        return fail(c, VPS_ERR_NONFINITE, "particles: non-finite input");
     VPS_TRY(ensure_io(c, n));
     double* dx = c->io_stage.p;
-    double* dv = v ? dx + n * D : nullptr;
-    VPS_HIP(c, hipMemcpyAsync(dx, x, (size_t)n * D * 8, hipMemcpyHostToDevice, c->stream));
-    if (v)
-        VPS_HIP(c, hipMemcpyAsync(dv, v, (size_t)n * D * 8, hipMemcpyHostToDevice, c->stream));
+    double* dv = v ? dx + pass * D : nullptr;
+    auto stage = [&](int64_t first, int64_t m) -> int {
+        VPS_HIP(c, hipMemcpyAsync(dx, x + first * D, (size_t)m * D * 8, hipMemcpyHostToDevice,
+                                  c->stream));
+        if (v)
+            VPS_HIP(c, hipMemcpyAsync(dv, v + first * D, (size_t)m * D * 8,
+                                      hipMemcpyHostToDevice, c->stream));
+        return VPS_OK;
+    };
+    const bool resident = c->initialized && n == c->n;
     // the flag is zero between calls
     int32_t* bad = (int32_t*)(c->counters.p + 12);
-    const int64_t nd = n * D * (v ? 2 : 1);
-    hipLaunchKernelGGL(k_check_finite, dim3(std::min(blocks(nd, 256), 2048u)), dim3(256), 0,
-                       c->stream, nd, dx, bad);
-    const bool resident = c->initialized && n == c->n;
-    if (resident) {
-        // keep the frozen volumes: overwrite x, v in the resident order
+    auto upload = [&](int64_t first, int64_t m) {
         const int s = c->cur;
-        hipLaunchKernelGGL(k_upload_resident, dim3(blocks(n, 256)), dim3(256), 0,
-                           c->stream, n, D, dx, dv, c->rid[s].p, c->rpos[s].p, c->rvel[s].p,
-                           bad);
-    }
-    VPS_HIP(c, hipGetLastError());
-    VPS_HIP(c, hipMemcpyAsync(c->host_counters + 12, bad, 4, hipMemcpyDeviceToHost, c->stream));
-    VPS_HIP(c, hipStreamSynchronize(c->stream));
-    if (*(int32_t*)(c->host_counters + 12)) {
-        VPS_HIP(c, hipMemsetAsync(bad, 0, 4, c->stream));
-        return fail(c, VPS_ERR_NONFINITE, "particles: non-finite input");
+        if (resident)   // keep the frozen volumes: overwrite x, v in the resident order
+            hipLaunchKernelGGL(k_upload_resident, dim3(blocks(n, 256)), dim3(256), 0, c->stream,
+                               n, first, m, D, dx, dv, c->rid[s].p, c->rpos[s].p, c->rvel[s].p,
+                               bad);
+        else
+            hipLaunchKernelGGL(k_upload, dim3(blocks(m, 256)), dim3(256), 0, c->stream, first, m,
+                               D, dx, dv, c->rpos[s].p, c->rvel[s].p, c->rid[s].p);
+    };
+    if (pass == n) {
+        VPS_TRY(stage(0, n));
+        const int64_t nd = n * D * (v ? 2 : 1);
+        hipLaunchKernelGGL(k_check_finite, dim3(std::min(blocks(nd, 256), 2048u)), dim3(256), 0,
+                           c->stream, nd, dx, bad);
+        if (resident) upload(0, n);
+        VPS_HIP(c, hipGetLastError());
+        VPS_HIP(c, hipMemcpyAsync(c->host_counters + 12, bad, 4, hipMemcpyDeviceToHost,
+                                  c->stream));
+        VPS_HIP(c, hipStreamSynchronize(c->stream));
+        if (*(int32_t*)(c->host_counters + 12)) {
+            VPS_HIP(c, hipMemsetAsync(bad, 0, 4, c->stream));
+            return fail(c, VPS_ERR_NONFINITE, "particles: non-finite input");
+        }
     }
     if (!resident) {
         c->n = n;
@@ -635,10 +663,15 @@ int vps_set_particles(vps_context* c, int64_t n, const double* x,
         c->cg_drift = 1.0;   // a new particle set: no drift measured on it yet
         VPS_TRY(ensure_particle_capacity(c, n));
         c->cur = 0;
-        hipLaunchKernelGGL(k_upload, dim3(blocks(n, 256)), dim3(256), 0, c->stream, n, D, dx,
-                           dv, c->rpos[0].p, c->rvel[0].p, c->rid[0].p);
-        VPS_HIP(c, hipGetLastError());
+        if (pass == n) upload(0, n);
     }
+    for (int64_t first = 0; pass < n && first < n; first += pass) {
+        const int64_t m = std::min(pass, n - first);
+        VPS_TRY(stage(first, m));
+        upload(first, m);
+    }
+    VPS_HIP(c, hipGetLastError());
+    if (pass < n) VPS_HIP(c, hipStreamSynchronize(c->stream));
     c->generated = false;
     return VPS_OK;
 }
@@ -650,12 +683,18 @@ int vps_get_particles(vps_context* c, double* x, double* v) {
     const int D = c->dim;
     const int s = c->cur;
     VPS_TRY(ensure_io(c, n));
+    const int64_t pass = io_pass(c, n);
     double* dx = c->io_stage.p;
-    hipLaunchKernelGGL(k_download, dim3(blocks(n, 256)), dim3(256), 0, c->stream, n, D,
-                       c->rid[s].p, c->rpos[s].p, c->rvel[s].p, x ? dx : nullptr,
-                       v ? dx + n * D : nullptr);
-    VPS_HIP(c, hipGetLastError());
-    return copy_out(c, (const char*)dx, (char*)x, (char*)v, (size_t)n * D * 8);
+    for (int64_t first = 0; first < n; first += pass) {
+        const int64_t m = std::min(pass, n - first);
+        hipLaunchKernelGGL(k_download, dim3(blocks(n, 256)), dim3(256), 0, c->stream, n, first, m,
+                           D, c->rid[s].p, c->rpos[s].p, c->rvel[s].p, x ? dx : nullptr,
+                           v ? dx + m * D : nullptr);
+        VPS_HIP(c, hipGetLastError());
+        VPS_TRY(copy_out(c, (const char*)dx, (char*)(x ? x + first * D : nullptr),
+                         (char*)(v ? v + first * D : nullptr), (size_t)m * D * 8));
+    }
+    return VPS_OK;
 }
 
 int vps_initialize(vps_context* c, vps_stats* st) {
