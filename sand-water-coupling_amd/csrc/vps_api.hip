@@ -427,6 +427,13 @@ int vps_create(const vps_params* params, vps_context** out) {
         delete c;
         return fail(nullptr, VPS_ERR_HIP, "no HIP device or stream");
     }
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) ==
+            hipSuccess &&
+        cus > 0)
+        c->cus = cus;
+    else
+        (void)hipGetLastError();
     fill_kconst(c);
     const KConst& k = c->k;
     c->ncells = (int64_t)k.cdims[0] * k.cdims[1] * k.cdims[2];

@@ -545,6 +545,7 @@ struct vps_context {
     int brick_nodes = 512;
     hipStream_t stream = nullptr;
     int device = 0;
+    int cus = 256;   // compute units of the device
     std::string err;
 
     // real particles (double buffered for the reorder)

@@ -1282,19 +1282,7 @@ struct IterLaunch {
 // (270 bricks: 7.75 with 256 blocks, 8.5 with 264), two beyond (600 bricks:
 // 9.8 against 10.1).
 static IterLaunch iter_launch(const vps_context* c, int nslots) {
-    static int cus_of[64] = {};
-    const int dev = c->device >= 0 && c->device < 64 ? c->device : 0;
-    if (cus_of[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, c->device) !=
-                hipSuccess ||
-            n <= 0) {
-            (void)hipGetLastError();
-            n = 256;
-        }
-        cus_of[dev] = n;
-    }
-    const int cus = cus_of[dev];
+    const int cus = c->cus;
     const bool row = c->p.op_mode == VPS_OP_ROW;
     IterLaunch L;
     int work, per_cu;
