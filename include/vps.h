@@ -148,7 +148,8 @@ typedef struct vps_stats {
     double ms_cg;              /* warm start + CG */
     double ms_gradient;        /* pressure gradient + velocity update */
     double ms_total;
-    double ms_spmv_avg;        /* average duration of one CG SpMV launch */
+    double ms_spmv_avg;        /* average duration of one CG iteration launch
+                                  (sums, update and SpMV) */
     double ms_update_avg;      /* 0: the update is part of the iteration launch */
     int64_t spmv_launches;
     int64_t reserved[4];       /* [0] residual replacements of the last solve,
@@ -275,13 +276,17 @@ int vps_projection_step(vps_context* ctx, vps_stats* stats);
  * on the resident state.  Not part of the projection. */
 int vps_advect(vps_context* ctx, double dt, double gravity);
 
-/* Requests that the next vps_project also computes the FP64 true residual
- * ||b - M x||/||b|| into stats.cg_true_rel_residual. */
+/* On (the default), a solve ends only once the FP64 true residual
+ * ||b - M x||/||b|| meets the tolerance, and reports it in
+ * stats.cg_true_rel_residual.  Off, it ends on the recursive residual alone:
+ * r.r after an update, as the sums of the launch before predict it
+ * (r.r - 2 alpha r.t + alpha^2 t.t, exact but for the FP32 rounding of r). */
 int vps_set_check_true_residual(vps_context* ctx, int32_t enable);
 
-/* Stamps the start and end of every fused CG SpMV and CG update launch of
- * the next solves (events of hipExtLaunchKernelGGL: the kernels' own
- * execution), reported as stats.ms_spmv_avg / ms_update_avg. */
+/* Stamps the start and end of every CG iteration launch of the next solves
+ * (events of hipExtLaunchKernelGGL: the kernels' own execution), reported as
+ * stats.ms_spmv_avg.  A launch forms the previous one's sums, applies the
+ * update and multiplies, in 2D and 3D, so stats.ms_update_avg is 0. */
 int vps_set_kernel_timing(vps_context* ctx, int32_t enable);
 
 /* Asynchronous steps (no counterpart in the reference, whose steps run on
