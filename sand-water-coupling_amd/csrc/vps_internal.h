@@ -34,7 +34,6 @@ constexpr int kBrick = 8;                  // brick side in lattice nodes
 constexpr int kBrickNodes3 = 512;
 constexpr int kBrickNodes2 = 64;
 constexpr int kStencilR = 3;               // |offset| < 4 lattice spacings
-constexpr int kMaxReduceBlocks = 65536;
 
 // Constants every kernel needs, passed by value.
 struct KConst {
@@ -441,46 +440,6 @@ __device__ __forceinline__ T wave_max(T v) {
     return v;
 }
 
-// Deterministic grid-wide sum: every block writes its partial, the last block
-// to arrive sums the partials in index order.  Returns true in the block that
-// produced the total (written to *out by thread 0).
-template <int BS>
-__device__ bool grid_sum_last(double v, double* partials, unsigned* counter,
-                              double* out) {
-    __shared__ double sred[BS / 64];
-    __shared__ bool is_last;
-    v = wave_sum(v);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) sred[wv] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0;
-        for (int i = 0; i < BS / 64; i++) s += sred[i];
-        partials[blockIdx.x] = s;
-        __threadfence();
-        const unsigned t = atomicAdd(counter, 1u);
-        is_last = (t == gridDim.x - 1);
-    }
-    __syncthreads();
-    if (!is_last) return false;
-    __threadfence();
-    double s = 0;
-    for (int i = threadIdx.x; i < (int)gridDim.x; i += BS)
-        s += __hip_atomic_load(&partials[i], __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-    s = wave_sum(s);
-    __syncthreads();
-    if (lane == 0) sred[wv] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0;
-        for (int i = 0; i < BS / 64; i++) t += sred[i];
-        *out = t;
-        *counter = 0;
-    }
-    return true;
-}
-
 // ---- device buffers -------------------------------------------------------
 template <typename T>
 struct DBuf {
@@ -492,23 +451,18 @@ struct DBuf {
 struct CgState {
     double bb;        // b.b
     double thr;       // tol^2 b.b (or DBL_MIN)
-    double abs_new;   // r.r of the current residual
     double rr;        // latest r.r
     double pt;        // p.t
     double true_rr;   // ||b - M x||^2 from the FP64 check
-    double thr_scale; // tol^2
     double abs0;      // r.r at the (re)start of the iteration
     float alpha, beta;
     int iter;         // Eigen iteration counter
     int done;         // 0 running, 1 converged, 2 max iterations, 3 nonfinite,
                       // 4 b = 0, 5 guarded start rejected (r0.r0 not <= b.b)
-    int first;        // 1 before the first SpMV of a (re)start
-    int pad;
     unsigned counter[4];
-    double rr_prev;   // 3D iteration: r.r before the last update
-    double thr_rec;   // 3D iteration: threshold of the recursive r.r
-    int final_kk;     // 3D iteration: the launch that applies the last x update
-    // 3D iteration launches: 0 while running; kk + 1 of the launch that
+    double rr_prev;   // r.r before the last update
+    double thr_rec;   // threshold of the recursive r.r
+    // the iteration launches: 0 while running; kk + 1 of the launch that
     // ended the solve; kStopBefore when it ended before any launch (read by
     // the iteration launches only: one word, so a block never mixes a stop
     // declared in its own launch with one from an earlier launch)
@@ -606,7 +560,7 @@ struct vps_context {
     vps::DBuf<int32_t> col_off, col_order;
     // per-node fields, slot-major
     vps::DBuf<float> vrho, vvol, vb, vdiag, vx[2], vr, vp[2], vt, vq, vrowsum;
-    // 3D CG iteration: second r and t (ping-pong with vr, vt) and the
+    // CG iteration: second r and t (ping-pong with vr, vt) and the
     // FP64-checked true residual
     vps::DBuf<float> vr2, vt2, vrt;
     vps::DBuf<double> vdiag64;
@@ -624,9 +578,9 @@ struct vps_context {
     bool generated = false;
     bool check_true = true;
     int prev_iters = 0;
-    // 3D CG: ||b - M x||^2 / (recursive r.r) at the last solve's convergence;
-    // the FP32 recursion runs to tol^2 b.b divided by it (at most 4x) so the
-    // FP64 check usually passes without a replacement
+    // ||b - M x||^2 / (recursive r.r) at the last solve's convergence; the FP32
+    // recursion runs to tol^2 b.b divided by it (at most 4x; in 2D see cg_solve)
+    // so the FP64 check usually passes without a replacement
     double cg_drift = 1.0;
     int64_t start_fallbacks = 0;   // solves restarted from the plain start
     bool start_guard = false;      // cg_solve: the start may be rejected
@@ -646,7 +600,7 @@ struct vps_context {
 
     // timing
     hipEvent_t ev[16] = {};
-    std::vector<hipEvent_t> kev;        // per-launch events (SpMV/update)
+    std::vector<hipEvent_t> kev;        // start and end of timed iteration launches
     bool kernel_timing = false;
     bool async_steps = false;   // steps return without waiting for their end
 

@@ -979,7 +979,6 @@ __global__ void __launch_bounds__(1024) k_cg_start(const double* pbb,
     st->abs0 = rr;
     st->iter = 0;
     st->true_rr = -1.0;
-    st->final_kk = -1;
     // IterativeSolver.h:25 setTolerance(max(tol, eps / ||b||)); Eigen's
     // threshold max(tol^2 ||b||^2, DBL_MIN) (ConjugateGradient.h)
     const double eps_tol = DBL_EPSILON / sqrt(bb);
@@ -1052,7 +1051,6 @@ __global__ void __launch_bounds__(1024) k_resume(const double* part, CgState* st
         st->beta = (float)(a / st->rr_prev);
         st->rr = a;
         st->true_rr = -1.0;
-        st->final_kk = -1;
         st->done = 0;
         st->stop = 0;
     }
@@ -1089,7 +1087,6 @@ __global__ void __launch_bounds__(1024) k_restart(const double* part,
         st->rr = a;
         st->alpha = 0.f;
         st->beta = 0.f;
-        st->final_kk = -1;
         st->done = a < st->thr ? 1 : 0;
         st->stop = st->done ? kStopBefore : 0;
     }
@@ -1411,7 +1408,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     }
     bool start_checked = max_iter == 0;
     const bool prof = c->kernel_timing;
-    const int64_t max_timed = (int64_t)c->kev.size() / 4;
+    const int64_t max_timed = (int64_t)c->kev.size() / 2;
     int64_t timed = 0, spmv_launches = 0;
     int kk = 0;          // iteration since the (re)start
     int iter_base = 0;   // Eigen iterations before the (re)start
@@ -1446,7 +1443,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
                 s.max_iter = max_iter;
                 // (an update resumed from the state: not timed)
                 const bool do_time = prof && timed < max_timed && !resume_pending;
-                hipEvent_t* ev = do_time ? &c->kev[4 * timed] : nullptr;
+                hipEvent_t* ev = do_time ? &c->kev[2 * timed] : nullptr;
                 const int o = (kk + 1) & 1, nw = kk & 1;
                 s.in = kk == 0 ? rbuf[o] : pb[o];
                 s.in2 = rbuf[o];
@@ -1621,7 +1618,7 @@ int cg_solve(vps_context* c, vps_stats* stats) {
     int64_t counted = 0;
     for (int64_t j = 0; j < timed; j++) {
         if (timed_iter[(size_t)j] > hs.iter) break;   // no-op launches
-        spmv_ms += ms_between(c->kev[4 * j], c->kev[4 * j + 1]);
+        spmv_ms += ms_between(c->kev[2 * j], c->kev[2 * j + 1]);
         counted++;
     }
     if (stats) {

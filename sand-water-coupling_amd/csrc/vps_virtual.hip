@@ -204,8 +204,6 @@ struct BAcc {
     }
 };
 
-// Everything after the real walk: the exact threshold decision, the boundary
-// walk, v_I, D_I and the outputs.
 // Boundary walk of one node from the global cell table (FP64 throughout).
 struct BoundaryWalkGlobal3 {
     const int32_t* bcstart;
@@ -220,6 +218,8 @@ struct BoundaryWalkGlobal3 {
     }
 };
 
+// Everything after the real walk: the exact threshold decision, the boundary
+// walk, v_I, D_I and the outputs.
 // S lanes share a node: the real sums are the node's, the boundary walk is one
 // lane's part, and lane 0 writes.
 template <int D, int S = 1, typename BW>
