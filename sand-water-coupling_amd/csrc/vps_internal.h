@@ -353,6 +353,8 @@ inline int walk_lanes(int64_t n) {
 //   40,000      11, 6.5, 6.5    14, 8.4, 7.7    27, 17, 20     11, 7.6, 8.7
 //   97,000      12, 9.0, 10     18, 11, 13      32, 26, 33     9.2, 8.2, 10
 //   250,000     15, 17, 21      20, 21, 24      48, 62, 77     13, 15, 19
+// (Eight gain 1 to 3 us in three of the four at 400 particles and lose in the
+// sums at 40,000; one number serves all small sizes.)
 inline int walk_lanes2(int64_t n) { return n <= 130000 ? 4 : 1; }
 
 // Work units of the 3D gradient: blocks of u[0] x u[1] x u[2] cells (at most
